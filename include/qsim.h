@@ -106,13 +106,11 @@ int qs_sv_init(qs_ctx* ctx, void* vec, int n, int dtype, uint64_t index, void* s
 int qs_sv_apply_gate(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gate, void* stream);
 
 /* A gate sequence.  fuse=0: one pass per gate (same kernels as qs_sv_apply_gate).
-   fuse=1: the fusion planner groups gates into LDS/register-resident tiles and
-   runs each group in one read+write pass.  fuse=2: as 1, and the planner may
-   also move qubits onto the low index bits between passes (every qubit is back
-   on its own bit when the call returns) when that saves at least 8% of the
-   passes, for lists of more than 480 gates; faster on long state-vector
-   circuits, not on density matrices.  Plans without moves (fuse=1, and fuse=2
-   lists of up to 480 gates) are launched pass by pass while they are planned.
+   fuse=1, 2 (the same): the fusion planner groups gates into LDS/register-resident
+   tiles and runs each group in one read+write pass, launched while the next ones
+   are planned.  Passes may move qubits between index bits (every qubit is back on
+   its own bit when the call's work is done); lists with noise superoperators are
+   planned without moves.
    Replaces the per-gate loop of StateVectorSimulator.run
    (statevector_simulator.py:155-164, 202-315).
    *passes (may be NULL) receives the number of full-state passes executed. */
@@ -131,7 +129,7 @@ int qs_set_fusion(qs_ctx* ctx, int tile_log2, int low_bits);
 int qs_set_fusion_launch(qs_ctx* ctx, int prefetch, int wg_per_cu);
 
 /* Captured gate sequences (HIP graphs).  qs_graph_capture plans the sequence
-   once (the same fused passes as qs_sv_apply_gates with fuse=2), uploads the
+   once (the same fused passes as qs_sv_apply_gates with fuse=1), uploads the
    program into memory the graph owns and captures the passes on `vec` in a HIP
    graph; init_zero != 0 puts a |0...0> initialisation in front.  Every
    qs_graph_launch then replays them on `stream` with no host-side planning:

@@ -26,6 +26,11 @@ enum FKind : int32_t {
   F_XX2 = 8,     // two targets, entries only where row ^ col is 00 or 11 (noise superoperators,
                  // Rxx/Ryy/FSim): a_s' = d_s a_s + o_s a_(s^3), payload d_0..d_3, o_0..o_3;
                  // pure != 0: real payload.  Never controlled.
+  // programs planned in wires only:
+  F_PHASE = 9,   // amplitudes whose selected bits are all 1 (creg register bits, cthr thread bits,
+                 // cblk tile-number bits) times one number: pure 0 f, 1 real f, 2 the unit number
+                 // given as shears (t, s): re += t im, im += s re, re += t im, 3 minus that number
+  F_ROT = 10,    // real rotation of a register pair as shears (t, s): x0 += t x1, x1 += s x0, x0 += t x1
 };
 
 constexpr int FMAX_TB = 10;
@@ -51,10 +56,13 @@ struct FOp {
   uint32_t cregv;   // ... and the values those register bits must have
   uint32_t cthr;    // control mask in thread-index space ...
   uint32_t cthrv;   // ... and the values those thread bits must have
+  uint32_t cblk;    // control mask in tile-number space (bits outside the tile) ...
+  uint32_t cblkv;   // ... and the values those bits must have: other tiles skip the op
 };
 
-// Its device encoding: eight 32-bit words, read with one scalar load (every
-// field a whole dword, so no sub-dword vector loads are needed):
+// Its device encoding for k_fused: eight 32-bit words, read with one scalar load
+// (every field a whole dword, so no sub-dword vector loads are needed); k_wires
+// has its own (encode_wire_op):
 //   w0 = kind | pure << 8 | npos << 16 | ntt << 24
 //   w1 = pos[0] | pos[1] << 8 | pos[2] << 16 | pos[3] << 24
 //   w2 = tpos[0] | tpos[1] << 8,  w3 = coef,  w4..w7 = creg, cregv, cthr, cthrv
@@ -76,6 +84,24 @@ static FOpW encode_op(const FOp& o) {
   return e;
 }
 
+// Programs planned in wires: ops only the larger instance of their kernel has.
+static bool wire_heavy(const FOp& o) {
+  switch (o.kind) {
+    case F_DENSE2:
+    case F_XX2:
+    case F_SWAP2:
+    case F_DENSE3:
+    case F_DENSE4:
+      return true;
+    case F_DENSE1:
+      return o.creg != 0 || o.cthr != 0;
+    case F_PERM1:
+      return !o.pure || (o.creg != 0 && (o.cthr != 0 || __builtin_popcount(o.creg) != 1 || o.cregv != o.creg));
+    default:
+      return false;
+  }
+}
+
 // RELAYOUT payload in the aux table (uint32): the register position p of the
 // tile bit h that splits the exchange into two rounds; the RB register-slot and
 // TB thread-slot LDS offsets of the current layout; the flip term of the
@@ -84,14 +110,19 @@ static FOpW encode_op(const FOp& o) {
 // the byte offset the single tile bit its slot carries contributes under the
 // relayout's XOR-linear placement (0 for the slot of h), so an amplitude's LDS
 // address is the XOR of its slots' offsets.  The write side is carried per
-// relayout because relabelings change the layout between relayouts.
+// relayout because relabelings change the layout between relayouts.  With
+// pure != 0 a count and that many (tile-number bit, offset) pairs follow: flips
+// of the current layout that depend on the tile.
+constexpr int FMAX_SX = 8;
 struct PassHdr {
   int32_t nops;
   int32_t op0;
   int32_t coef0;
   int32_t uses_lds;
-  int32_t has_dk;        // pass contains 3- or 4-target dense ops (kernel variant without LDS coefficients)
-  int32_t ncoef;         // complex coefficients of this pass (staged in LDS)
+  int32_t has_dk;        // pass contains 3- or 4-target dense ops (kernel variant without LDS coefficients);
+                         // planned in wires: ops of wire_heavy
+  int32_t ncoef;         // complex coefficients of this pass
+  int32_t nstage;        // the first nstage of them are staged in LDS (diagonal tables, read per lane)
   int32_t sync_store;    // store layout differs from the load layout and no relayout ordered the
                          // loads: workgroup barrier before the stores (another wave may still have
                          // to load an address this wave stores to)
@@ -102,6 +133,10 @@ struct PassHdr {
   int32_t rs0[FMAX_RB], ts0[FMAX_TB];  // load layout (tile-local bits)
   int32_t rs1[FMAX_RB], ts1[FMAX_TB];  // store layout
   uint64_t sflip;        // global-index XOR applied to every store address (pending flips)
+  uint64_t sr[FMAX_RB], st[FMAX_TB];  // store address XOR of each register / thread index bit
+  int32_t nsx;           // flips of the store address that depend on the tile: where tile-number bit
+  int32_t sxb[FMAX_SX];  // sxb[i] is 1 ...
+  uint64_t sxm[FMAX_SX]; // ... the address is XORed with sxm[i]
 };
 
 // ---- host planner --------------------------------------------------------------
@@ -120,6 +155,10 @@ struct Config {
   // density matrix (26 instead of 29 passes) is 5% slower, so its calls do
   // not ask for it.
   int remap = 0;
+  // Plan in wires (qsim_wire_plan.hpp): only the bits a gate mixes have to be in
+  // the tile, swaps and flips are relabelings of the whole program, qubits move
+  // between index bits at every store.  `remap` then does not matter.
+  bool wires = false;
 };
 
 static bool gate_diag_like(const qs_gate& g) { return g.kind == QS_GATE_DIAG || g.kind == QS_GATE_PHASE; }
@@ -507,7 +546,8 @@ static bool merge_diag(Built& e, const Built& d, int NR) {
   return true;
 }
 
-static bool uncontrolled(const FOp& o) { return o.creg == 0 && o.cthr == 0; }
+static bool uncontrolled_in_tile(const FOp& o) { return o.creg == 0 && o.cthr == 0; }
+static bool uncontrolled(const FOp& o) { return uncontrolled_in_tile(o) && o.cblk == 0; }
 
 // Dense 4x4 form ((re, im) pairs) of an uncontrolled two-target op.
 static void two_target_dense(const Built& b, double* M) {
@@ -587,7 +627,8 @@ static bool try_merge(std::vector<Built>& out, Built& d, int NR, int RB) {
   if (d.op.kind == F_DIAG && e.op.kind == F_DIAG) return merge_diag(e, d, NR);
   double d2[4], M[8];
   if (d.op.kind == F_DENSE1 && e.op.kind == F_DENSE1 && e.op.pos[0] == d.op.pos[0] && e.op.creg == d.op.creg &&
-      e.op.cregv == d.op.cregv && e.op.cthr == d.op.cthr && e.op.cthrv == d.op.cthrv) {
+      e.op.cregv == d.op.cregv && e.op.cthr == d.op.cthr && e.op.cthrv == d.op.cthrv && e.op.cblk == d.op.cblk &&
+      e.op.cblkv == d.op.cblkv) {
     mat2_mul(d.coef.data(), e.coef.data(), M);
     e.coef.assign(M, M + 8);
     return true;
@@ -1316,6 +1357,8 @@ static int schedule_pass(const qs_gate* gates, PassPlan& p, const Config& c, uin
   }
   for (int b = 0; b < c.RB; ++b) H.rs1[b] = cur.rs[b];
   for (int b = 0; b < c.TB; ++b) H.ts1[b] = cur.ts[b];
+  for (int b = 0; b < c.RB; ++b) H.sr[b] = 1ull << p.tbo[cur.rs[b]];
+  for (int b = 0; b < c.TB; ++b) H.st[b] = 1ull << p.tbo[cur.ts[b]];
   // pending flips go into the store address
   const uint32_t fl = flip_local(cur);
   for (int j = 0; j < K; ++j)
@@ -1329,8 +1372,15 @@ static int schedule_pass(const qs_gate* gates, PassPlan& p, const Config& c, uin
   H.nops = (int)prog.ops.size() - op_start;
   H.coef0 = coef_start;
   H.ncoef = (int)(prog.coef.size() / 2) - coef_start;
+  H.nstage = H.ncoef;
   return QS_OK;
 }
+
+}  // namespace qs
+
+#include "qsim_wire_plan.hpp"
+
+namespace qs {
 
 // Plan and schedule one program (with `remap`: moving qubits onto the low bits).
 // `ready`, when given, sees each fused pass as soon as it is scheduled (its
@@ -1350,7 +1400,17 @@ static int build_one(const qs_gate* gates, int ngates, int n, const Config& c, b
     prog.aux0.push_back(a0);
     if (ready) rc = ready(p);
   };
-  plan_groups(gates, ngates, n, c, remap, prog.plans, prog.pgates, on_pass);
+  if (c.wires) {
+    auto done = [&](const PassHdr& H, int a0, PassPlan& p) -> int {
+      p.hdr = (int)prog.hdrs.size();
+      prog.hdrs.push_back(H);
+      prog.aux0.push_back(a0);
+      return ready ? ready(p) : QS_OK;
+    };
+    rc = plan_wires(gates, ngates, n, c, amp_bytes, prog, done);
+  } else {
+    plan_groups(gates, ngates, n, c, remap, prog.plans, prog.pgates, on_pass);
+  }
   if (rc) return rc;
   prog.hdr_of.assign(prog.plans.size(), -1);
   for (size_t i = 0; i < prog.plans.size(); ++i)
@@ -1365,9 +1425,10 @@ static int check_passes(const FusedProgram& prog, const Config& c, int h0, int h
     const PassHdr& h = prog.hdrs[hi];
     for (int i = 0; i < h.nops; ++i) {
       const FOp& o = prog.ops[(size_t)h.op0 + i];
-      bool ok = o.kind >= F_RELAYOUT && o.kind <= F_XX2;
+      bool ok = o.kind >= F_RELAYOUT && o.kind <= F_ROT;
       switch (o.kind) {
         case F_DENSE1:
+        case F_ROT:
         case F_PERM1:
           ok = o.pos[0] >= 0 && o.pos[0] < c.RB;
           break;
@@ -1384,9 +1445,13 @@ static int check_passes(const FusedProgram& prog, const Config& c, int h0, int h
         case F_DENSE4:
           ok = h.has_dk != 0;
           break;
+        case F_PHASE:
+          ok = o.creg < (1u << c.RB) && o.cregv == o.creg && o.pure >= 0 && o.pure <= 3;
+          break;
         default:
           break;
       }
+      if (c.wires) ok = ok && (!wire_heavy(o) || h.has_dk) && (o.cthr | o.cthrv) < (1u << c.TB);
       if (!ok) {
         set_error("fusion planner: internal error: op outside the tile kernel's encodings");
         return QS_ERR_ARG;
@@ -1414,7 +1479,7 @@ static int build_program_unchecked(const qs_gate* gates, int ngates, int n, cons
   int rc = check_config(c);
   if (rc) return rc;
   rc = build_one(gates, ngates, n, c, false, amp_bytes, prog);
-  if (rc || c.remap == 0 || n < c.RB + c.TB + 2) return rc;
+  if (rc || c.wires || c.remap == 0 || n < c.RB + c.TB + 2) return rc;
   // moving qubits onto the low bits pays when it saves enough passes (the
   // passes that put the qubits back included): the passes get heavier.  Short
   // programs (under 24 passes) rarely save 8%, and a second plan costs host time.
@@ -1503,10 +1568,13 @@ static int build_streamed(const qs_gate* gates, int ngates, int n, const Config&
 static void print_program_stats(const FusedProgram& prog, int n, int K, int L, int ngates) {
   // op counts by kind; dense1 / exchange by control mode (bit 0 register
   // controls, bit 1 thread controls); diagonals lane-mode vs table
-  int nrel = 0, kinds[9] = {0}, d1cm[4] = {0}, p1cm[4] = {0}, dlane = 0, dtab = 0;
+  int nrel = 0, kinds[11] = {0}, d1cm[4] = {0}, p1cm[4] = {0}, dlane = 0, dtab = 0, ph[5] = {0}, outer = 0, d1re = 0;
   for (const FOp& o : prog.ops) {
     if (o.kind == F_RELAYOUT) ++nrel;
-    if (o.kind < 9) ++kinds[o.kind];
+    if (o.kind < 11) ++kinds[o.kind];
+    if (o.kind == F_PHASE) ++ph[__builtin_popcount(o.creg)];
+    if (o.kind == F_DENSE1 && o.pure) ++d1re;
+    outer += o.cblk != 0;
     const int cm = (o.cthr ? 2 : 0) | (o.creg ? 1 : 0);
     if (o.kind == F_DENSE1) ++d1cm[cm];
     if (o.kind == F_PERM1) ++p1cm[cm];
@@ -1517,11 +1585,12 @@ static void print_program_stats(const FusedProgram& prog, int n, int K, int L, i
   fprintf(stderr,
           "[qsim fusion] n=%d K=%d L=%d gates=%d passes=%zu fused=%zu with_lds=%d ops=%zu relayouts=%d "
           "dense1=%d perm1=%d diag=%d dense2=%d xx2=%d swap2=%d dense3=%d dense4=%d "
-          "dense1_cm=%d,%d,%d,%d perm1_cm=%d,%d,%d,%d diag_lane=%d diag_table=%d\n",
+          "dense1_cm=%d,%d,%d,%d perm1_cm=%d,%d,%d,%d diag_lane=%d diag_table=%d real1=%d outer=%d rot=%d "
+          "phase by register bits=%d,%d,%d,%d\n",
           n, K, L, ngates, prog.plans.size(), prog.hdrs.size(), lds, prog.ops.size(), nrel, kinds[F_DENSE1],
           kinds[F_PERM1], kinds[F_DIAG], kinds[F_DENSE2], kinds[F_XX2], kinds[F_SWAP2], kinds[F_DENSE3],
           kinds[F_DENSE4], d1cm[0],
-          d1cm[1], d1cm[2], d1cm[3], p1cm[0], p1cm[1], p1cm[2], p1cm[3], dlane, dtab);
+          d1cm[1], d1cm[2], d1cm[3], p1cm[0], p1cm[1], p1cm[2], p1cm[3], dlane, dtab, d1re, outer, kinds[F_ROT], ph[0], ph[1], ph[2], ph[3]);
 }
 
 }  // namespace qs

@@ -1,0 +1,278 @@
+// The tile pass of programs planned in wires (qsim_wire_plan.hpp): op
+// interpreter and kernel.
+//
+// What bounds it: with 3 to 4 times fewer passes than k_fused each pass carries
+// 30 to 60 ops, and the vector ALU is what a pass waits for (measured with
+// k_fused as the interpreter: 70% of the cycles of a 25-qubit complex64 pass were
+// VALU issue, 6900 instructions a wave for 46 ops).  So the ops are written to
+// need few instructions and no copies of the tile:
+//   * every op changes its registers in place.  A rotation is three shears,
+//     x0 += t x1, x1 += s x0, x0 += t x1 (t = -tan(theta / 2), s = sin(theta),
+//     |theta| <= pi / 2, so |t| <= 1): 3 fused multiply-adds per component pair
+//     instead of 4, and no value outlives its successor, so the compiler keeps one
+//     register set.  k_fused's ops read and write two sets and need 162 VGPRs;
+//   * a phase touches only the amplitudes it changes, again as shears (of the real
+//     and imaginary parts) when its angle is at most pi / 2;
+//   * ops that do not apply to the tile are skipped, one opcode selects the op,
+//     and ops that few circuits need live in a second instance (HEAVY).
+#pragma once
+#include "qsim_fused_kernel.hpp"
+#include "qsim_wires.hpp"
+
+namespace qs {
+
+// ---- ops, in place -----------------------------------------------------------------
+
+template <typename R, int NR, int P>
+__device__ __forceinline__ void wo_rot(cx<R> (&a)[NR], const cx<R>* g) {
+  const R t = g[0].re, s = g[0].im;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (r & (1 << P)) continue;
+    cx<R>&x0 = a[r], &x1 = a[r | (1 << P)];
+    x0.re = rfma(t, x1.re, x0.re);
+    x0.im = rfma(t, x1.im, x0.im);
+    x1.re = rfma(s, x0.re, x1.re);
+    x1.im = rfma(s, x0.im, x1.im);
+    x0.re = rfma(t, x1.re, x0.re);
+    x0.im = rfma(t, x1.im, x0.im);
+  }
+}
+
+// Exchange in place (v_swap_b32).  Written as assignments the exchange would make
+// the compiler rename the pair's registers in this one arm of the op switch, and
+// copy the tile back in all the others.
+__device__ __forceinline__ void swap_bits(float& x, float& y) {
+  asm volatile("v_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+}
+__device__ __forceinline__ void swap_bits(double& x, double& y) {
+  uint64_t u = __builtin_bit_cast(uint64_t, x), w = __builtin_bit_cast(uint64_t, y);
+  uint32_t u0 = (uint32_t)u, u1 = (uint32_t)(u >> 32), w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
+  asm volatile("v_swap_b32 %0, %2\n\tv_swap_b32 %1, %3" : "+v"(u0), "+v"(u1), "+v"(w0), "+v"(w1));
+  x = __builtin_bit_cast(double, (uint64_t)u1 << 32 | u0);
+  y = __builtin_bit_cast(double, (uint64_t)w1 << 32 | w0);
+}
+
+template <typename R, int NR, int P, int C>
+__device__ __forceinline__ void wo_ex(cx<R> (&a)[NR]) {
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if ((r & (1 << P)) || (C >= 0 && !((r >> (C & 31)) & 1))) continue;
+    swap_bits(a[r].re, a[r | (1 << P)].re);
+    swap_bits(a[r].im, a[r | (1 << P)].im);
+  }
+}
+
+// The same where the thread predicate holds.
+template <typename R, int NR, int P>
+__device__ __forceinline__ void wo_ext(cx<R> (&a)[NR], bool on) {
+  if (on) wo_ex<R, NR, P, -1>(a);
+}
+
+// x *= f in place: both cross products before either part changes.
+template <typename R> __device__ __forceinline__ void mul_in_place(cx<R>& x, cx<R> f) {
+  const R u = f.im * x.im, w = f.im * x.re;
+  x.re = rfma(f.re, x.re, -u);
+  x.im = rfma(f.re, x.im, w);
+}
+
+// The amplitudes whose register bits in MASK are all 1 times f (MODE 0), a real
+// factor (1), the unit number of the shear pair f (2) or minus that (3: the signs
+// are operand modifiers).
+template <typename R, int NR, uint32_t MASK, int MODE>
+__device__ __forceinline__ void wo_phase(cx<R> (&a)[NR], cx<R> f) {
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (((uint32_t)r & MASK) != MASK) continue;
+    cx<R>& x = a[r];
+    if constexpr (MODE == 1) {
+      x.re = f.re * x.re;
+      x.im = f.re * x.im;
+    } else if constexpr (MODE == 2) {
+      x.re = rfma(f.re, x.im, x.re);
+      x.im = rfma(f.im, x.re, x.im);
+      x.re = rfma(f.re, x.im, x.re);
+    } else if constexpr (MODE == 3) {
+      x.re = rfma(f.re, x.im, x.re);
+      x.im = rfma(-f.im, x.re, -x.im);
+      x.re = rfma(f.re, x.im, -x.re);
+    } else {
+      mul_in_place(x, f);
+    }
+  }
+}
+
+template <typename R, int NR, int P>
+__device__ __forceinline__ void wo_u2(cx<R> (&a)[NR], const cx<R>* m) {
+  const cx<R> m00 = m[0], m01 = m[1], m10 = m[2], m11 = m[3];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (r & (1 << P)) continue;
+    cx<R>&x0 = a[r], &x1 = a[r | (1 << P)];
+    // the parts that need the other three components first, then each component
+    // times its real diagonal entry, in place
+    R p0r = m01.re * x1.re, p0i = m01.re * x1.im, p1r = m10.re * x0.re, p1i = m10.re * x0.im;
+    p0r = rfma(-m01.im, x1.im, p0r);
+    p0i = rfma(m01.im, x1.re, p0i);
+    p1r = rfma(-m10.im, x0.im, p1r);
+    p1i = rfma(m10.im, x0.re, p1i);
+    p0r = rfma(-m00.im, x0.im, p0r);
+    p0i = rfma(m00.im, x0.re, p0i);
+    p1r = rfma(-m11.im, x1.im, p1r);
+    p1i = rfma(m11.im, x1.re, p1i);
+    x0.re = rfma(m00.re, x0.re, p0r);
+    x0.im = rfma(m00.re, x0.im, p0i);
+    x1.re = rfma(m11.re, x1.re, p1r);
+    x1.im = rfma(m11.re, x1.im, p1i);
+  }
+}
+
+template <typename R, int RB, int TB, bool HEAVY>
+__device__ __forceinline__ void wire_op(cx<R> (&a)[1 << RB], char* lds, const FOpW& e, const cx<R>* __restrict__ C,
+                                        const cx<R>* __restrict__ G, const uint32_t* __restrict__ X, uint32_t tid,
+                                        uint32_t blk) {
+  static_assert(RB == 4, "opcodes are laid out for four register bits");
+  constexpr int NR = 1 << RB;
+  const uint32_t code = e.w[0] & 0xff;
+  const uint32_t cthr = e.w[3] & 0xffff;
+  const bool tok = (tid & cthr) == e.w[3] >> 16;
+  const cx<R>* g = G + e.w[2];  // uniform payloads, through scalar loads
+  switch (code) {
+    case WC_RELAYOUT: {
+      const uint32_t* x = X + e.w[2];
+      const bool tf = e.w[4] != 0;
+      switch (x[0]) {
+        case 0: relayout_half<R, RB, TB, 0>(a, lds, x, tf, tid, blk); break;
+        case 1: relayout_half<R, RB, TB, 1>(a, lds, x, tf, tid, blk); break;
+        case 2: relayout_half<R, RB, TB, 2>(a, lds, x, tf, tid, blk); break;
+        case 3: relayout_half<R, RB, TB, 3>(a, lds, x, tf, tid, blk); break;
+        default: __builtin_unreachable();
+      }
+      break;
+    }
+#define QS_4(X) X(0) X(1) X(2) X(3)
+#define QS_16(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15)
+#define QS_ROT(P) case WC_ROT + P: wo_rot<R, NR, P>(a, g); break;
+    QS_4(QS_ROT)
+#define QS_EX(P) case WC_EX + P: wo_ex<R, NR, P, -1>(a); break;
+    QS_4(QS_EX)
+#define QS_EXT(P) case WC_EXT + P: wo_ext<R, NR, P>(a, tok); break;
+    QS_4(QS_EXT)
+#define QS_EXC(Q)                                                            \
+  case WC_EXC + Q:                                                           \
+    if constexpr (Q / 4 != Q % 4) wo_ex<R, NR, Q / 4, Q % 4>(a);             \
+    else __builtin_unreachable();                                            \
+    break;
+    QS_16(QS_EXC)
+// lanes whose thread bits fail sit these out: a wave all of whose lanes do skips the op
+#define QS_PH(BASE, MODE, M) case BASE + M: if (tok) wo_phase<R, NR, M, MODE>(a, g[0]); break;
+#define QS_PHR(M) QS_PH(WC_PHR, 2, M)
+    QS_16(QS_PHR)
+#define QS_PHS(M) QS_PH(WC_PHS, 3, M)
+    QS_16(QS_PHS)
+#define QS_PHC(M) QS_PH(WC_PHC, 0, M)
+    QS_16(QS_PHC)
+#define QS_PHN(M) QS_PH(WC_PHN, 1, M)
+    QS_16(QS_PHN)
+    case WC_TABLE:
+    case WC_LANE: {
+      const uint32_t s = diag_sel((int)(e.w[0] >> 24), (int)(e.w[1] & 0xff), (int)((e.w[1] >> 8) & 0xff), tid);
+      const cx<R>* T = C + e.w[2] + (code == WC_LANE ? s : s * NR);
+      const int step = code == WC_LANE ? 0 : 1;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) mul_in_place(a[r], ld(T + r * step));
+      break;
+    }
+#define QS_U2(P) case WC_U2 + P: wo_u2<R, NR, P>(a, g); break;
+    QS_4(QS_U2)
+    default: {
+      if constexpr (HEAVY) {
+        const uint32_t creg = (e.w[0] >> 8) & 0xff, cregv = (e.w[0] >> 16) & 0xff;
+        const bool pure = e.w[5] != 0;
+        switch (code) {
+#define QS_U2G(P) case WC_U2G + P: do_dense1<R, NR, P, 3>(a, g, creg, cregv, tok); break;
+          QS_4(QS_U2G)
+#define QS_EXG(P)                                                          \
+  case WC_EXG + P:                                                         \
+    if (pure) do_perm1<R, NR, P, 3, true>(a, g, creg, cregv, tok);         \
+    else do_perm1<R, NR, P, 3, false>(a, g, creg, cregv, tok);             \
+    break;
+          QS_4(QS_EXG)
+#define QS_PAIR(A, B)                                                                            \
+  case WC_D2 + A * (A - 1) / 2 + B: do_dense2<R, NR, A, B, 3>(a, g, creg, cregv, tok); break;    \
+  case WC_XX + A * (A - 1) / 2 + B: do_xx2<R, NR, A, B, false>(a, g); break;                     \
+  case WC_SW + A * (A - 1) / 2 + B:                                                              \
+    if (pure) do_swap2<R, NR, A, B, 3, true>(a, g, creg, cregv, tok);                            \
+    else do_swap2<R, NR, A, B, 3, false>(a, g, creg, cregv, tok);                                \
+    break;
+          QS_PAIR(1, 0) QS_PAIR(2, 0) QS_PAIR(2, 1) QS_PAIR(3, 0) QS_PAIR(3, 1) QS_PAIR(3, 2)
+          case WC_D3 + 0: do_densek<R, NR, 3, 14u>(a, g, creg, cregv, tok); break;
+          case WC_D3 + 1: do_densek<R, NR, 3, 13u>(a, g, creg, cregv, tok); break;
+          case WC_D3 + 2: do_densek<R, NR, 3, 11u>(a, g, creg, cregv, tok); break;
+          case WC_D3 + 3: do_densek<R, NR, 3, 7u>(a, g, creg, cregv, tok); break;
+          case WC_D4: do_densek<R, NR, 4, 15u>(a, g, creg, cregv, tok); break;
+          default: __builtin_unreachable();
+        }
+      } else {
+        __builtin_unreachable();
+      }
+    }
+  }
+}
+
+// One workgroup, one tile: load, ops, store.
+template <typename R, int RB, int TB, bool HEAVY>
+__global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k_wires(cx<R>* __restrict__ v, const PassHdr* __restrict__ H,
+                                                   const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
+                                                   const uint32_t* __restrict__ aux) {
+  constexpr int NR = 1 << RB, K = RB + TB;
+  extern __shared__ __align__(16) char lds_raw[];
+  const uint32_t tid = threadIdx.x, blk = blockIdx.x;
+  const FOpW* P = ops + H->op0;
+  const cx<R>* G = coef + H->coef0;
+  // diagonal tables, read per lane, are staged behind the relayout image
+  cx<R>* C = reinterpret_cast<cx<R>*>(lds_raw) + (H->uses_lds ? (1 << (K - 1)) : 0);
+  if (H->nstage) {
+    for (int i = (int)tid; i < H->nstage; i += (int)blockDim.x) C[i] = G[i];
+    __syncthreads();
+  }
+  cx<R> a[NR];
+  const uint64_t tb = insert_zeros((uint64_t)blk, H->sorted, K);
+  {
+    uint64_t gin = 0;
+#pragma unroll
+    for (int b = 0; b < TB; ++b) gin |= (uint64_t)((tid >> b) & 1u) << H->tbits[H->ts0[b]];
+    const uint64_t base = tb | gin;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      uint64_t g = 0;
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+        if ((r >> b) & 1) g |= 1ull << H->tbits[H->rs0[b]];
+      a[r] = ld_nt(v + (base | g));
+    }
+  }
+  const int nops = H->nops;
+  for (int o = 0; o < nops; ++o) {
+    const FOpW e = P[o];
+    if ((blk & e.w[6]) != e.w[7]) continue;
+    wire_op<R, RB, TB, HEAVY>(a, lds_raw, e, C, G, aux, tid, blk);
+  }
+  if (H->sync_store) __syncthreads();
+  // store: per-lane and per-register address bits, flips that depend on the tile
+  uint64_t base = tb ^ H->sflip;
+#pragma unroll
+  for (int b = 0; b < TB; ++b) base ^= ((tid >> b) & 1u) ? H->st[b] : 0ull;
+  const int nx = H->nsx;
+  for (int i = 0; i < nx; ++i) base ^= ((blk >> H->sxb[i]) & 1u) ? H->sxm[i] : 0ull;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    uint64_t g = 0;
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      if ((r >> b) & 1) g ^= H->sr[b];
+    st_nt(v + (base ^ g), a[r]);
+  }
+}
+
+}  // namespace qs

@@ -1,0 +1,37 @@
+// Tile passes planned in wires: kernel instances and their launch.
+//
+// A translation unit of its own because it is compiled with
+// -structurizecfg-skip-uniform-regions: the op switch is uniform, and without the
+// flag the compiler rebuilds it as nested regions that carry the whole tile from
+// one to the next (two register sets, up to 64 moves an op).
+#include "qsim_wire_kernel.hpp"
+
+namespace qs {
+
+template <typename R, int RB, int TB>
+void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const FOpW* ops, const cx<R>* coef,
+                  const uint32_t* aux, size_t lds, hipStream_t s) {
+  if (hd.has_dk)
+    hipLaunchKernelGGL((k_wires<R, RB, TB, true>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef, aux);
+  else
+    hipLaunchKernelGGL((k_wires<R, RB, TB, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef,
+                       aux);
+}
+
+template <typename R, int RB, int TB> void wires_lds_attr() {
+  const int bytes = (int)((1u << (RB + TB - 1)) * sizeof(cx<R>) + FMAX_PASS_COEF * sizeof(cx<R>));
+  (void)hipFuncSetAttribute((const void*)k_wires<R, RB, TB, true>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  (void)hipFuncSetAttribute((const void*)k_wires<R, RB, TB, false>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
+#define QS_WIRES(R, TB)                                                                                          \
+  template void launch_wires<R, 4, TB>(cx<R>*, uint64_t, const PassHdr&, const PassHdr*, const FOpW*,            \
+                                       const cx<R>*, const uint32_t*, size_t, hipStream_t);                      \
+  template void wires_lds_attr<R, 4, TB>();
+QS_WIRES(double, 7)
+QS_WIRES(double, 8)
+QS_WIRES(double, 9)
+QS_WIRES(float, 8)
+QS_WIRES(float, 9)
+
+}  // namespace qs

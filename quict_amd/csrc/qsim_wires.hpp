@@ -1,0 +1,102 @@
+// Launch of the tile passes planned in wires (kernels in qsim_wires.hip), and their
+// op encoding.
+#pragma once
+#include "qsim_common.hpp"
+#include "qsim_fused_plan.hpp"
+
+namespace qs {
+
+// Opcodes of k_wires.  P, C: register positions; M: mask of register positions.
+enum WCode : uint32_t {
+  WC_RELAYOUT = 0,   // + position that splits the exchange
+  WC_ROT = 4,        // + P: rotation, payload (t, s)
+  WC_EX = 8,         // + P: exchange of the pair, uncontrolled in the tile
+  WC_EXT = 12,       // + P: where the thread predicate holds
+  WC_EXC = 16,       // + 4 P + C: where register bit C is 1
+  WC_PHR = 32,       // + M: phase as shears (t, s)
+  WC_PHS = 48,       // + M: minus that
+  WC_PHC = 64,       // + M: phase f
+  WC_PHN = 80,       // + M: real factor
+  WC_TABLE = 96,     // diagonal table in LDS, per register
+  WC_LANE = 97,      // diagonal table in LDS, one entry per lane
+  WC_U2 = 98,        // + P: complex 2x2
+  WC_HEAVY = 102,    // from here on: only in the HEAVY instance
+  WC_U2G = 102,      // + P: complex 2x2 under register and thread controls
+  WC_EXG = 106,      // + P: exchange under register and thread controls
+  WC_D2 = 110,       // + pair: complex 4x4 under controls
+  WC_XX = 116,       // + pair: diagonal + anti-diagonal
+  WC_SW = 122,       // + pair: exchange of 01 and 10 under controls
+  WC_D3 = 128,       // + missing position: 8x8 (RB = 4)
+  WC_D4 = 132,
+  WC_END = 133
+};
+// register pairs (P0 > P1) in the order 10, 20, 21, 30, 31, 32
+static int wire_pair(int p0, int p1) { return p0 * (p0 - 1) / 2 + p1; }
+
+// Device encoding (32 bytes, one scalar load): code | creg << 8 | cregv << 16 |
+// ntt << 24; tpos[0] | tpos[1] << 8; coef; cthr | cthrv << 16; 0; 0; cblk; cblkv
+static FOpW encode_wire_op(const FOp& o) {
+  uint32_t code = WC_END;
+  const bool ctl = o.creg != 0 || o.cthr != 0;
+  switch (o.kind) {
+    case F_RELAYOUT:
+      code = WC_RELAYOUT;  // the kernel reads the position from the payload
+      break;
+    case F_ROT:
+      code = WC_ROT + o.pos[0];
+      break;
+    case F_PERM1:
+      if (!o.pure) code = WC_EXG + o.pos[0];
+      else if (!ctl) code = WC_EX + o.pos[0];
+      else if (!o.creg) code = WC_EXT + o.pos[0];
+      else if (!o.cthr && __builtin_popcount(o.creg) == 1 && o.cregv == o.creg)
+        code = WC_EXC + 4 * o.pos[0] + __builtin_ctz(o.creg);
+      else code = WC_EXG + o.pos[0];
+      break;
+    case F_PHASE:
+      code = (o.pure == 3 ? WC_PHS : o.pure == 2 ? WC_PHR : o.pure == 1 ? WC_PHN : WC_PHC) + o.creg;
+      break;
+    case F_DIAG:
+      code = o.pure ? WC_LANE : WC_TABLE;
+      break;
+    case F_DENSE1:
+      code = (ctl ? WC_U2G : WC_U2) + o.pos[0];
+      break;
+    case F_DENSE2:
+      code = WC_D2 + wire_pair(o.pos[0], o.pos[1]);
+      break;
+    case F_XX2:
+      code = WC_XX + wire_pair(o.pos[0], o.pos[1]);
+      break;
+    case F_SWAP2:
+      code = WC_SW + wire_pair(o.pos[0], o.pos[1]);
+      break;
+    case F_DENSE3:
+      code = WC_D3 + (6 - o.pos[0] - o.pos[1] - o.pos[2]);
+      break;
+    case F_DENSE4:
+      code = WC_D4;
+      break;
+  }
+  const bool diag = o.kind == F_DIAG;
+  FOpW e;
+  e.w[0] = code | (diag ? 0 : o.creg) << 8 | (diag ? 0 : o.cregv) << 16 | (uint32_t)o.ntt << 24;
+  e.w[1] = (uint32_t)o.tpos[0] | (uint32_t)o.tpos[1] << 8;
+  e.w[2] = (uint32_t)o.coef;
+  e.w[3] = o.cthr | o.cthrv << 16;
+  e.w[4] = (uint32_t)(o.kind == F_RELAYOUT ? o.pure : 0);  // relayout: flips that depend on the tile
+  e.w[5] = (uint32_t)o.pure;
+  e.w[6] = o.cblk;
+  e.w[7] = o.cblkv;
+  return e;
+}
+
+// One pass over the 2^(n-K) tiles of v: header hd, its device copy dh and the
+// program's device arrays.  The caller checks hipGetLastError().
+template <typename R, int RB, int TB>
+void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const FOpW* ops, const cx<R>* coef,
+                  const uint32_t* aux, size_t lds, hipStream_t s);
+// Lets the kernels take their largest LDS allocation (once per process).
+template <typename R, int RB, int TB> void wires_lds_attr();
+
+}  // namespace qs
