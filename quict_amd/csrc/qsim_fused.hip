@@ -90,14 +90,14 @@ template <typename R, int RB, int TB>
 static int launch_fused(qs_ctx* ctx, cx<R>* v, int n, const Config& c, const PassHdr& hd, const PassHdr* dh,
                         const ProgDev<R>& d, hipStream_t s, bool prof) {
   constexpr int K = RB + TB;
-  const uint64_t tiles = 1ull << (n - K);
+  const uint64_t tiles = n > K ? 1ull << (n - K) : 1;
   const size_t lds_bytes = (size_t)(1u << (K - 1)) * sizeof(cx<R>);  // half-tile relayout image
   const size_t lds_relayout = hd.uses_lds ? lds_bytes : 0;
   const size_t lds = hd.has_dk && !c.wires ? lds_relayout : lds_relayout + (size_t)hd.nstage * sizeof(cx<R>);
   int rc = QS_OK;
   if (prof && (rc = prof_begin(ctx, PROF_FUSED, s))) return rc;
   if (c.wires) {
-    launch_wires<R, RB, TB>(v, tiles, hd, dh, d.O, d.C, d.X, lds, s);
+    launch_wires<R, RB, TB>(v, tiles, hd, dh, d.O, d.C, d.X, n < K ? 1u << n : 0u, lds, s);
   } else if (hd.has_dk) {
     hipLaunchKernelGGL((k_fused<R, RB, TB, true, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, d.O,
                        d.C, d.X, tiles);
@@ -363,8 +363,11 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
     set_error("low_bits must not exceed tile_log2 - 4");
     return QS_ERR_ARG;
   }
-  if (n < K + 1 || ngates == 0) {
-    // small registers: every pass is latency-bound anyway; one kernel per gate
+  // Registers of at most a tile run whole programs planned in wires in one launch
+  // (5 qubits, 100 gates: 508 us a run with a kernel per gate, 247 us so); two gates or
+  // fewer are no slower as kernels of their own.  Programs that keep whole gates in
+  // the tile (fused_config) need more than one tile's bits.
+  if (ngates == 0 || (n < K + 1 && (ngates < 3 || !fused_config(4, K - 4, L, gates, ngates).wires))) {
     for (int i = 0; i < ngates; ++i) {
       int rc = apply_gate(ctx, vec, n, dtype, &gates[i], s);
       if (rc) return rc;

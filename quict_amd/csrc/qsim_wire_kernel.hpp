@@ -220,11 +220,12 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[1 << RB], char* lds, const FO
   }
 }
 
-// One workgroup, one tile: load, ops, store.
+// One workgroup, one tile: load, ops, store.  nsmall != 0: a register of nsmall
+// amplitudes, fewer than a tile has; the rest of the tile is zeros.
 template <typename R, int RB, int TB, bool HEAVY>
 __global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k_wires(cx<R>* __restrict__ v, const PassHdr* __restrict__ H,
                                                    const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
-                                                   const uint32_t* __restrict__ aux) {
+                                                   const uint32_t* __restrict__ aux, uint32_t nsmall) {
   constexpr int NR = 1 << RB, K = RB + TB;
   extern __shared__ __align__(16) char lds_raw[];
   const uint32_t tid = threadIdx.x, blk = blockIdx.x;
@@ -249,7 +250,8 @@ __global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k
 #pragma unroll
       for (int b = 0; b < RB; ++b)
         if ((r >> b) & 1) g |= 1ull << H->tbits[H->rs0[b]];
-      a[r] = ld_nt(v + (base | g));
+      if (nsmall == 0) a[r] = ld_nt(v + (base | g));
+      else a[r] = (uint32_t)(base | g) < nsmall ? ld(v + (base | g)) : zero<R>();
     }
   }
   const int nops = H->nops;
@@ -271,7 +273,7 @@ __global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k
 #pragma unroll
     for (int b = 0; b < RB; ++b)
       if ((r >> b) & 1) g ^= H->sr[b];
-    st_nt(v + (base ^ g), a[r]);
+    if (nsmall == 0 || (uint32_t)(base ^ g) < nsmall) st_nt(v + (base ^ g), a[r]);
   }
 }
 

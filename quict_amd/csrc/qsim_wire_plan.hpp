@@ -1069,10 +1069,16 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
 
 // Plans the whole program; every fused pass goes to done(header, first aux word,
 // plan) as soon as it is scheduled and is appended to prog.plans after that.
+//
+// A register of at most K bits is one tile: wires up to K are idle and every store
+// puts all wires home (bits n..K-1 are not there: the kernel neither loads nor
+// stores them).
 template <typename Done>
-static int plan_wires(const qs_gate* gates, int ngates, int n, const Config& c, uint32_t amp_bytes,
+static int plan_wires(const qs_gate* gates, int ngates, int nbits, const Config& c, uint32_t amp_bytes,
                       FusedProgram& prog, const Done& done) {
   const int K = c.RB + c.TB, L = c.L;
+  const int n = std::max(nbits, K);
+  const bool one_tile = n == K;
   WireProgram W;
   {
     WireReducer red(c, W, n);
@@ -1239,7 +1245,7 @@ static int plan_wires(const qs_gate* gates, int ngates, int n, const Config& c, 
       // the head gate runs on its own (nothing precedes it): one the tile kernel
       // cannot take, or one with more bits than a tile has room for
       if (have) {
-        const int rc = finish_pass(PS);
+        const int rc = finish_pass(one_tile ? homing() : PS);
         if (rc) return rc;
         continue;  // its store may have brought bits that let the head gate fit
       }
@@ -1271,7 +1277,7 @@ static int plan_wires(const qs_gate* gates, int ngates, int n, const Config& c, 
         if ((PS >> w) & 1) S |= 1ull << w;
     for (int b = 0; b < n && __builtin_popcountll(S) < K; ++b) S |= 1ull << at[b];
     if (have) {
-      const int rc = finish_pass(S & PS);
+      const int rc = finish_pass(one_tile ? homing() : S & PS);
       if (rc) return rc;
     }
     have = true;

@@ -10,12 +10,13 @@ namespace qs {
 
 template <typename R, int RB, int TB>
 void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const FOpW* ops, const cx<R>* coef,
-                  const uint32_t* aux, size_t lds, hipStream_t s) {
+                  const uint32_t* aux, uint32_t nsmall, size_t lds, hipStream_t s) {
   if (hd.has_dk)
-    hipLaunchKernelGGL((k_wires<R, RB, TB, true>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef, aux);
+    hipLaunchKernelGGL((k_wires<R, RB, TB, true>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef, aux,
+                       nsmall);
   else
     hipLaunchKernelGGL((k_wires<R, RB, TB, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef,
-                       aux);
+                       aux, nsmall);
 }
 
 template <typename R, int RB, int TB> void wires_lds_attr() {
@@ -26,7 +27,7 @@ template <typename R, int RB, int TB> void wires_lds_attr() {
 
 #define QS_WIRES(R, TB)                                                                                          \
   template void launch_wires<R, 4, TB>(cx<R>*, uint64_t, const PassHdr&, const PassHdr*, const FOpW*,            \
-                                       const cx<R>*, const uint32_t*, size_t, hipStream_t);                      \
+                                       const cx<R>*, const uint32_t*, uint32_t, size_t, hipStream_t);            \
   template void wires_lds_attr<R, 4, TB>();
 QS_WIRES(double, 7)
 QS_WIRES(double, 8)

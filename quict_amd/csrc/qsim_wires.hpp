@@ -92,10 +92,10 @@ static FOpW encode_wire_op(const FOp& o) {
 }
 
 // One pass over the 2^(n-K) tiles of v: header hd, its device copy dh and the
-// program's device arrays.  The caller checks hipGetLastError().
+// program's device arrays; nsmall: amplitudes of a register below a tile, else 0.  The caller checks hipGetLastError().
 template <typename R, int RB, int TB>
 void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const FOpW* ops, const cx<R>* coef,
-                  const uint32_t* aux, size_t lds, hipStream_t s);
+                  const uint32_t* aux, uint32_t nsmall, size_t lds, hipStream_t s);
 // Lets the kernels take their largest LDS allocation (once per process).
 template <typename R, int RB, int TB> void wires_lds_attr();
 

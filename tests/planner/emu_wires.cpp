@@ -46,14 +46,16 @@ static void wire_pass(zc* v, int n, int RB, int TB, uint32_t S, const PassHdr& H
   std::vector<zc> a((size_t)NT * NR), lds((size_t)NT * NR), out((size_t)NT * NR);
   std::vector<int> written((size_t)NT * NR);
   auto cz = [&](int i) { return zc(Cd[2 * i], Cd[2 * i + 1]); };
-  for (uint64_t t = 0; t < (1ull << (n - K)); ++t) {
+  // a register below a tile: the amplitudes it lacks are zeros and not stored
+  const uint64_t N = 1ull << n;
+  for (uint64_t t = 0; t < (n > K ? 1ull << (n - K) : 1); ++t) {
     const uint64_t tb = insert_zeros(t, H.sorted, K);
     for (int tid = 0; tid < NT; ++tid)
       for (int r = 0; r < NR; ++r) {
         uint64_t g = tb;
         for (int b = 0; b < TB; ++b) g |= (uint64_t)((tid >> b) & 1) << H.tbits[H.ts0[b]];
         for (int b = 0; b < RB; ++b) g |= (uint64_t)((r >> b) & 1) << H.tbits[H.rs0[b]];
-        a[(size_t)tid * NR + r] = v[g];
+        a[(size_t)tid * NR + r] = g < N ? v[g] : zc(0);
       }
     for (int o = 0; o < H.nops; ++o) {
       const FOp& op = P[o];
@@ -201,7 +203,8 @@ static void wire_pass(zc* v, int n, int RB, int TB, uint32_t S, const PassHdr& H
     for (uint32_t k = 0; k < (uint32_t)(NT * NR); ++k) {
       uint64_t g = tb;
       for (int j = 0; j < K; ++j) g |= (uint64_t)((k >> j) & 1) << H.sorted[j];
-      v[g] = out[k];
+      if (g < N) v[g] = out[k];
+      else if (out[k] != zc(0)) throw std::runtime_error("amplitude outside the register");
     }
   }
 }

@@ -77,6 +77,27 @@ def test_wires_match_per_gate_kernels(case, n, dtype, tol):
     assert both(recs, n, dtype, 2) < tol
 
 
+@pytest.mark.parametrize("dtype,tol", [(nat.QS_C128, 1e-12), (nat.QS_C64, 1e-5)], ids=["c128", "c64"])
+@pytest.mark.parametrize("n", [5, 6, 9, 11, 12])
+def test_registers_within_one_tile(n, dtype, tol):
+    """Fewer amplitudes than a tile: one launch, nothing outside the register written."""
+    import torch
+    print("[case] wires small", n, dtype, flush=True)
+    recs, keep = compile_gates(random_types(n, 150, n).gates, n)
+    assert both(recs, n, dtype, 1) < tol
+    if n >= 9:
+        recs, keep = free_records(n, 60, n)
+        assert both(recs, n, dtype, 1) < tol
+    lib, ctx, s = nat.load_library(), nat.context(0), nat.stream_ptr(0)
+    v = torch.zeros(1 << 13, dtype=torch.complex128 if dtype == nat.QS_C128 else torch.complex64, device="cuda:0")
+    v[1 << n:] = 7
+    v[0] = 1
+    recs, keep = compile_gates(random_types(n, 40, n).gates, n)
+    nat.check(lib.qs_sv_apply_gates(ctx, ctypes.c_void_p(v.data_ptr()), n, dtype, nat.gate_array_ptr(recs), len(recs),
+                                    1, None, s))
+    assert bool((v[1 << n:] == 7).all()) and abs(float(torch.linalg.vector_norm(v[: 1 << n])) - 1) < 1e-5
+
+
 @pytest.mark.parametrize("shape,dtype", [((11, 4), nat.QS_C128), ((13, 4), nat.QS_C128), ((13, 5), nat.QS_C64),
                                          ((12, 8), nat.QS_C64), ((12, 2), nat.QS_C128)])
 def test_wires_in_other_tile_shapes(shape, dtype):

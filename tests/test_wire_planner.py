@@ -100,6 +100,26 @@ def test_all_gate_types(emu, shape, n, ngates, seed):
     check(emu, recs, n, shape)
 
 
+@pytest.mark.parametrize("shape", ["c128", "c64", "c128-k11"])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 8, 11, 12])
+def test_registers_within_one_tile(emu, shape, n):
+    types = [t for t in ALL_TYPES if n >= 3 or t.name in ("h", "x", "y", "s", "rx", "rz", "u3") or
+             (n == 2 and t.name in ("cx", "cz", "swap", "crz"))]
+    recs, keep = compile_gates(random_types(n, 120, n, types).gates, n)
+    st = check(emu, recs, n, shape)
+    assert n > 11 or st[0] == 1 or shape == "c128-k11"
+    if n >= 6:
+        c = random_types(n, 30, n)
+        u, _ = np.linalg.qr(np.random.RandomState(n).randn(32, 32))
+        Unitary(u.astype(complex)) | c(random.Random(n).sample(range(n), 5))
+        Swap | c([0, n - 1])
+        X | c(1)
+        for g in random_types(n, 30, n + 1).gates:
+            c.append(g)
+        recs, keep = compile_gates(c.gates, n)
+        check(emu, recs, n, shape)
+
+
 @pytest.mark.parametrize("L", [2, 3, 5, 8])
 def test_low_bit_counts(emu, L):
     recs, keep = compile_gates(random_types(16, 300, 5).gates, 16)
