@@ -275,6 +275,25 @@ int qs_adjoint_gradient_pauli(qs_ctx* ctx, void* psi, void* lam, int n, int dtyp
                               const qs_gate* dgates, const int32_t* param_slot, double* grads, int nslots,
                               double* energy, void* stream);
 
+/* A variational circuit planned once (no reference counterpart): gate i is the fixed
+   record gates[i] with its inverse inverses[i] when param_slot[i] < 0, else the
+   rotation exp(-i theta[param_slot[i]] P / 2) on bit gates[i].bits[0], P = X, Y, Z for
+   axis[i] = 0, 1, 2 (nothing else of the record is read; a phase diag(1, e^{i theta})
+   is a Z rotation up to a common phase).  The plan does not depend on the angles.
+   QS_ERR_UNSUPPORTED: a gate needs a pass of its own (see qs_graph_capture).
+   qs_var_gradient: energy <psi|H|psi> of psi = circuit |0...0> and its derivatives,
+   added to grads[0..nslots); psi and lam are caller buffers of max(2^n, 4096)
+   amplitudes whose contents are ignored and overwritten.  It waits for the stream.
+   A plan serves one call at a time. */
+typedef struct qs_var qs_var;
+int qs_var_create(qs_ctx* ctx, int n, int dtype, const qs_gate* gates, const qs_gate* inverses, int ngates,
+                  const int32_t* axis, const int32_t* param_slot, int nslots, qs_var** out);
+int qs_var_gradient(qs_var* v, void* psi, void* lam, const double* theta, const qs_pauli_term* terms, int nterms,
+                    double* energy, double* grads, void* stream);
+/* Passes of one forward (backward = 0) or backward sweep (-1 for NULL). */
+int qs_var_passes(const qs_var* v, int backward);
+void qs_var_destroy(qs_var* v);
+
 /* ---- batched variational circuits (no reference counterpart) ------------- */
 /* Launch shape of the batched QNN kernel (picked by the autotuner):
    widths <= lds_max_width keep psi and lam in LDS (2 x 2^w amplitudes),

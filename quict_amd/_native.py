@@ -102,6 +102,10 @@ SIGNATURES = {
     "qs_sv_inner": (_I, [_P, _P, _P, _I, _I, ctypes.POINTER(_D), ctypes.POINTER(_D), _P]),
     "qs_adjoint_gradient": (_I, [_P, _P, _P, _I, _I, _P, _I, _P, _P, _P, _I, _P]),
     "qs_adjoint_gradient_pauli": (_I, [_P, _P, _P, _I, _I, _P, _I, _P, _P, _I, _P, _P, _P, _I, _P, _P]),
+    "qs_var_create": (_I, [_P, _I, _I, _P, _P, _I, _P, _P, _I, ctypes.POINTER(_P)]),
+    "qs_var_gradient": (_I, [_P, _P, _P, _P, _P, _I, ctypes.POINTER(_D), _P, _P]),
+    "qs_var_passes": (_I, [_P, _I]),
+    "qs_var_destroy": (None, [_P]),
     "qs_qnn_batch": (_I, [_P, _I, _I, _P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     "qs_qnn_batch_programs": (_I, [_P, _I, _I, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
 }

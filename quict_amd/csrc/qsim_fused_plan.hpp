@@ -31,6 +31,8 @@ enum FKind : int32_t {
                  // cblk tile-number bits) times one number: pure 0 f, 1 real f, 2 the unit number
                  // given as shears (t, s): re += t im, im += s re, re += t im, 3 minus that number
   F_ROT = 10,    // real rotation of a register pair as shears (t, s): x0 += t x1, x1 += s x0, x0 += t x1
+  F_MEAS = 11,   // two-vector sweeps: column `coef` of the tile's gradient row = Im <lam|P|psi> on register
+                 // bit pos[0], P = Z (pure 0) or Y (pure 1)
 };
 
 constexpr int FMAX_TB = 10;
@@ -58,6 +60,8 @@ struct FOp {
   uint32_t cthrv;   // ... and the values those thread bits must have
   uint32_t cblk;    // control mask in tile-number space (bits outside the tile) ...
   uint32_t cblkv;   // ... and the values those bits must have: other tiles skip the op
+  int sym;          // 0, or 1 + the parameter the payload of this rotation / phase comes from ...
+  double sgn;       // ... times this sign (its matrix is not known when the program is planned)
 };
 
 // Its device encoding for k_fused: eight 32-bit words, read with one scalar load
@@ -114,6 +118,7 @@ static bool wire_heavy(const FOp& o) {
 // pure != 0 a count and that many (tile-number bit, offset) pairs follow: flips
 // of the current layout that depend on the tile.
 constexpr int FMAX_SX = 8;
+constexpr int FMAX_GRAD = 512;  // gradient columns one pass may take (LDS)
 struct PassHdr {
   int32_t nops;
   int32_t op0;
@@ -137,6 +142,7 @@ struct PassHdr {
   int32_t nsx;           // flips of the store address that depend on the tile: where tile-number bit
   int32_t sxb[FMAX_SX];  // sxb[i] is 1 ...
   uint64_t sxm[FMAX_SX]; // ... the address is XORed with sxm[i]
+  int32_t ngrad;         // gradient columns of the pass (two-vector sweeps)
 };
 
 // ---- host planner --------------------------------------------------------------
@@ -971,6 +977,17 @@ static std::vector<int> choose_regs(const std::vector<int>& need, const std::vec
   return regs;
 }
 
+// A gate planned without its matrix: rotation or phase by sgn * theta[slot]; meas != 0:
+// a gradient column of parameter `slot`, sign meas, is taken before it.
+struct WireSym {
+  int slot = -1;
+  double sgn = 1.0, meas = 0.0;
+};
+struct GradCol {
+  int slot;
+  double sgn;
+};
+
 // A whole pass program: headers, ops, complex coefficients and the relayout
 // constants, ready for upload.
 struct FusedProgram {
@@ -982,6 +999,8 @@ struct FusedProgram {
   std::vector<double> coef;  // (re, im)
   std::vector<uint32_t> aux;
   std::vector<int> aux0;     // header -> first aux word of its relayouts
+  std::vector<WireSym> psym;  // parallel to pgates (programs with parameters)
+  std::vector<std::vector<GradCol>> gcols;  // header -> its gradient columns
 };
 
 
@@ -1407,7 +1426,10 @@ static int build_one(const qs_gate* gates, int ngates, int n, const Config& c, b
       prog.aux0.push_back(a0);
       return ready ? ready(p) : QS_OK;
     };
-    rc = plan_wires(gates, ngates, n, c, amp_bytes, prog, done);
+    auto fill = [&](WireReducer& red) {
+      for (int i = 0; i < ngates; ++i) red.add(gates[i]);
+    };
+    rc = plan_wires(fill, ngates, n, c, amp_bytes, prog, done);
   } else {
     plan_groups(gates, ngates, n, c, remap, prog.plans, prog.pgates, on_pass);
   }
@@ -1425,10 +1447,11 @@ static int check_passes(const FusedProgram& prog, const Config& c, int h0, int h
     const PassHdr& h = prog.hdrs[hi];
     for (int i = 0; i < h.nops; ++i) {
       const FOp& o = prog.ops[(size_t)h.op0 + i];
-      bool ok = o.kind >= F_RELAYOUT && o.kind <= F_ROT;
+      bool ok = o.kind >= F_RELAYOUT && o.kind <= F_MEAS;
       switch (o.kind) {
         case F_DENSE1:
         case F_ROT:
+        case F_MEAS:
         case F_PERM1:
           ok = o.pos[0] >= 0 && o.pos[0] < c.RB;
           break;
@@ -1568,10 +1591,10 @@ static int build_streamed(const qs_gate* gates, int ngates, int n, const Config&
 static void print_program_stats(const FusedProgram& prog, int n, int K, int L, int ngates) {
   // op counts by kind; dense1 / exchange by control mode (bit 0 register
   // controls, bit 1 thread controls); diagonals lane-mode vs table
-  int nrel = 0, kinds[11] = {0}, d1cm[4] = {0}, p1cm[4] = {0}, dlane = 0, dtab = 0, ph[5] = {0}, outer = 0, d1re = 0;
+  int nrel = 0, kinds[12] = {0}, d1cm[4] = {0}, p1cm[4] = {0}, dlane = 0, dtab = 0, ph[5] = {0}, outer = 0, d1re = 0;
   for (const FOp& o : prog.ops) {
     if (o.kind == F_RELAYOUT) ++nrel;
-    if (o.kind < 11) ++kinds[o.kind];
+    if (o.kind < 12) ++kinds[o.kind];
     if (o.kind == F_PHASE) ++ph[__builtin_popcount(o.creg)];
     if (o.kind == F_DENSE1 && o.pure) ++d1re;
     outer += o.cblk != 0;

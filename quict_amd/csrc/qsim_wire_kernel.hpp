@@ -63,12 +63,6 @@ __device__ __forceinline__ void wo_ex(cx<R> (&a)[NR]) {
   }
 }
 
-// The same where the thread predicate holds.
-template <typename R, int NR, int P>
-__device__ __forceinline__ void wo_ext(cx<R> (&a)[NR], bool on) {
-  if (on) wo_ex<R, NR, P, -1>(a);
-}
-
 // x *= f in place: both cross products before either part changes.
 template <typename R> __device__ __forceinline__ void mul_in_place(cx<R>& x, cx<R> f) {
   const R u = f.im * x.im, w = f.im * x.re;
@@ -127,10 +121,97 @@ __device__ __forceinline__ void wo_u2(cx<R> (&a)[NR], const cx<R>* m) {
   }
 }
 
-template <typename R, int RB, int TB, bool HEAVY>
-__device__ __forceinline__ void wire_op(cx<R> (&a)[1 << RB], char* lds, const FOpW& e, const cx<R>* __restrict__ C,
+// Relayout in two rounds (see relayout_half) of NV tiles, each through a half-tile
+// image of its own, so that they share the barriers.
+template <typename R, int RB, int TB, int NV, int P>
+__device__ __forceinline__ void wire_relayout(cx<R> (&a)[NV][1 << RB], char* lds, const uint32_t* __restrict__ x,
+                                              bool tile_flips, uint32_t tid, uint32_t blk) {
+  constexpr int NR = 1 << RB;
+  constexpr uint32_t image = (uint32_t)sizeof(cx<R>) << (RB + TB - 1);
+  uint32_t lw[RB], lq[RB];
+#pragma unroll
+  for (int b = 0; b < RB; ++b) lw[b] = x[1 + b];
+  uint32_t w = thr_off<TB>(x + 1 + RB, tid) ^ x[1 + RB + TB];
+  const uint32_t* y = x + 2 + RB + TB;
+  if (tile_flips) {
+    const uint32_t* z = y + RB + TB;
+    const uint32_t nz = z[0];
+    uint32_t f = 0;
+    for (uint32_t i = 0; i < nz; ++i) f ^= ((blk >> z[1 + 2 * i]) & 1u) ? z[2 + 2 * i] : 0u;
+    w ^= f;
+  }
+#pragma unroll
+  for (int b = 0; b < RB; ++b) lq[b] = y[b];
+  const uint32_t rd = thr_off<TB>(y + RB, tid);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (((r >> P) & 1) == k) {
+        const uint32_t o = w ^ reg_off<RB>(r, lw);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) st_lds<R>(lds + v * image, o, a[v][r]);
+      }
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (((r >> P) & 1) == k) {
+        const uint32_t o = rd ^ reg_off<RB>(r, lq);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) a[v][r] = ld_lds<R>(lds + v * image, o);
+      }
+  }
+}
+
+// Lane moves within the 64 lanes of a wave (DPP): lanes without a source add 0.
+template <int CTRL, int ROWS> __device__ __forceinline__ double wave_move(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, ROWS, 0xf, false),
+                          __builtin_amdgcn_update_dpp(0, lo, CTRL, ROWS, 0xf, false));
+}
+// The sum over the wave, in lane 63.
+__device__ __forceinline__ double wave_total(double v) {
+  v += wave_move<0x111, 0xf>(v);  // row_shr:1
+  v += wave_move<0x112, 0xf>(v);  // row_shr:2
+  v += wave_move<0x114, 0xf>(v);  // row_shr:4
+  v += wave_move<0x118, 0xf>(v);  // row_shr:8
+  v += wave_move<0x142, 0xa>(v);  // row_bcast:15
+  v += wave_move<0x143, 0xc>(v);  // row_bcast:31
+  return v;
+}
+
+// This wave's part of Im <lam|P|psi>, P = Z (Y false) or Y on register bit PB, in
+// double for both precisions; lane 63 writes it to its place in the gradient row.
+template <typename R, int NR, int PB, bool Y>
+__device__ __forceinline__ void wo_measure(const cx<R> (&psi)[NR], const cx<R> (&lam)[NR], double* slot, uint32_t tid) {
+  double s0 = 0, s1 = 0;  // two chains
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (r & (1 << PB)) continue;
+    const cx<R> a0 = psi[r], a1 = psi[r | (1 << PB)], b0 = lam[r], b1 = lam[r | (1 << PB)];
+    if constexpr (Y) {  // Y psi = (-i a1, i a0)
+      s0 = rfma((double)b1.re, (double)a0.re, s0);
+      s0 = rfma((double)b1.im, (double)a0.im, s0);
+      s1 = rfma((double)b0.re, (double)a1.re, s1);
+      s1 = rfma((double)b0.im, (double)a1.im, s1);
+    } else {
+      s0 = rfma((double)b0.re, (double)a0.im, s0);
+      s0 = rfma(-(double)b0.im, (double)a0.re, s0);
+      s1 = rfma((double)b1.re, (double)a1.im, s1);
+      s1 = rfma(-(double)b1.im, (double)a1.re, s1);
+    }
+  }
+  const double s = wave_total(s0 - s1);
+  if ((tid & 63) == 63) *slot = s;
+}
+
+// One op on NV vectors (2: psi and lam of a gradient sweep); grad: this wave's column
+// 0 of the tile's gradient row.
+template <typename R, int RB, int TB, int NV, bool HEAVY>
+__device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, const FOpW& e, const cx<R>* __restrict__ C,
                                         const cx<R>* __restrict__ G, const uint32_t* __restrict__ X, uint32_t tid,
-                                        uint32_t blk) {
+                                        uint32_t blk, double* grad) {
   static_assert(RB == 4, "opcodes are laid out for four register bits");
   constexpr int NR = 1 << RB;
   const uint32_t code = e.w[0] & 0xff;
@@ -142,30 +223,34 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[1 << RB], char* lds, const FO
       const uint32_t* x = X + e.w[2];
       const bool tf = e.w[4] != 0;
       switch (x[0]) {
-        case 0: relayout_half<R, RB, TB, 0>(a, lds, x, tf, tid, blk); break;
-        case 1: relayout_half<R, RB, TB, 1>(a, lds, x, tf, tid, blk); break;
-        case 2: relayout_half<R, RB, TB, 2>(a, lds, x, tf, tid, blk); break;
-        case 3: relayout_half<R, RB, TB, 3>(a, lds, x, tf, tid, blk); break;
+        case 0: wire_relayout<R, RB, TB, NV, 0>(a, lds, x, tf, tid, blk); break;
+        case 1: wire_relayout<R, RB, TB, NV, 1>(a, lds, x, tf, tid, blk); break;
+        case 2: wire_relayout<R, RB, TB, NV, 2>(a, lds, x, tf, tid, blk); break;
+        case 3: wire_relayout<R, RB, TB, NV, 3>(a, lds, x, tf, tid, blk); break;
         default: __builtin_unreachable();
       }
       break;
     }
+#define QS_V(...)                                  \
+  _Pragma("unroll") for (int v = 0; v < NV; ++v) { \
+    __VA_ARGS__;                                   \
+  }
 #define QS_4(X) X(0) X(1) X(2) X(3)
 #define QS_16(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15)
-#define QS_ROT(P) case WC_ROT + P: wo_rot<R, NR, P>(a, g); break;
+#define QS_ROT(P) case WC_ROT + P: QS_V(wo_rot<R, NR, P>(a[v], g))  break;
     QS_4(QS_ROT)
-#define QS_EX(P) case WC_EX + P: wo_ex<R, NR, P, -1>(a); break;
+#define QS_EX(P) case WC_EX + P: QS_V(wo_ex<R, NR, P, -1>(a[v])) break;
     QS_4(QS_EX)
-#define QS_EXT(P) case WC_EXT + P: wo_ext<R, NR, P>(a, tok); break;
+#define QS_EXT(P) case WC_EXT + P: if (tok) QS_V(wo_ex<R, NR, P, -1>(a[v])) break;
     QS_4(QS_EXT)
 #define QS_EXC(Q)                                                            \
   case WC_EXC + Q:                                                           \
-    if constexpr (Q / 4 != Q % 4) wo_ex<R, NR, Q / 4, Q % 4>(a);             \
+    if constexpr (Q / 4 != Q % 4) QS_V(wo_ex<R, NR, Q / 4, Q % 4>(a[v]))     \
     else __builtin_unreachable();                                            \
     break;
     QS_16(QS_EXC)
 // lanes whose thread bits fail sit these out: a wave all of whose lanes do skips the op
-#define QS_PH(BASE, MODE, M) case BASE + M: if (tok) wo_phase<R, NR, M, MODE>(a, g[0]); break;
+#define QS_PH(BASE, MODE, M) case BASE + M: if (tok) QS_V(wo_phase<R, NR, M, MODE>(a[v], g[0])) break;
 #define QS_PHR(M) QS_PH(WC_PHR, 2, M)
     QS_16(QS_PHR)
 #define QS_PHS(M) QS_PH(WC_PHS, 3, M)
@@ -180,37 +265,52 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[1 << RB], char* lds, const FO
       const cx<R>* T = C + e.w[2] + (code == WC_LANE ? s : s * NR);
       const int step = code == WC_LANE ? 0 : 1;
 #pragma unroll
-      for (int r = 0; r < NR; ++r) mul_in_place(a[r], ld(T + r * step));
+      for (int r = 0; r < NR; ++r) {
+        const cx<R> f = ld(T + r * step);
+        QS_V(mul_in_place(a[v][r], f))
+      }
       break;
     }
-#define QS_U2(P) case WC_U2 + P: wo_u2<R, NR, P>(a, g); break;
+#define QS_U2(P) case WC_U2 + P: QS_V(wo_u2<R, NR, P>(a[v], g)) break;
     QS_4(QS_U2)
+#define QS_MZ(P)                                                                                        \
+  case WC_MZ + P:                                                                                       \
+    if constexpr (NV == 2) wo_measure<R, NR, P, false>(a[0], a[1], grad + (e.w[2] << (TB - 6)), tid);   \
+    else __builtin_unreachable();                                                                       \
+    break;
+    QS_4(QS_MZ)
+#define QS_MY(P)                                                                                        \
+  case WC_MY + P:                                                                                       \
+    if constexpr (NV == 2) wo_measure<R, NR, P, true>(a[0], a[1], grad + (e.w[2] << (TB - 6)), tid);    \
+    else __builtin_unreachable();                                                                       \
+    break;
+    QS_4(QS_MY)
     default: {
       if constexpr (HEAVY) {
         const uint32_t creg = (e.w[0] >> 8) & 0xff, cregv = (e.w[0] >> 16) & 0xff;
         const bool pure = e.w[5] != 0;
         switch (code) {
-#define QS_U2G(P) case WC_U2G + P: do_dense1<R, NR, P, 3>(a, g, creg, cregv, tok); break;
+#define QS_U2G(P) case WC_U2G + P: QS_V(do_dense1<R, NR, P, 3>(a[v], g, creg, cregv, tok)) break;
           QS_4(QS_U2G)
 #define QS_EXG(P)                                                          \
   case WC_EXG + P:                                                         \
-    if (pure) do_perm1<R, NR, P, 3, true>(a, g, creg, cregv, tok);         \
-    else do_perm1<R, NR, P, 3, false>(a, g, creg, cregv, tok);             \
+    if (pure) QS_V(do_perm1<R, NR, P, 3, true>(a[v], g, creg, cregv, tok)) \
+    else QS_V(do_perm1<R, NR, P, 3, false>(a[v], g, creg, cregv, tok))     \
     break;
           QS_4(QS_EXG)
 #define QS_PAIR(A, B)                                                                            \
-  case WC_D2 + A * (A - 1) / 2 + B: do_dense2<R, NR, A, B, 3>(a, g, creg, cregv, tok); break;    \
-  case WC_XX + A * (A - 1) / 2 + B: do_xx2<R, NR, A, B, false>(a, g); break;                     \
+  case WC_D2 + A * (A - 1) / 2 + B: QS_V(do_dense2<R, NR, A, B, 3>(a[v], g, creg, cregv, tok)) break; \
+  case WC_XX + A * (A - 1) / 2 + B: QS_V(do_xx2<R, NR, A, B, false>(a[v], g)) break;               \
   case WC_SW + A * (A - 1) / 2 + B:                                                              \
-    if (pure) do_swap2<R, NR, A, B, 3, true>(a, g, creg, cregv, tok);                            \
-    else do_swap2<R, NR, A, B, 3, false>(a, g, creg, cregv, tok);                                \
+    if (pure) QS_V(do_swap2<R, NR, A, B, 3, true>(a[v], g, creg, cregv, tok))                    \
+    else QS_V(do_swap2<R, NR, A, B, 3, false>(a[v], g, creg, cregv, tok))                        \
     break;
           QS_PAIR(1, 0) QS_PAIR(2, 0) QS_PAIR(2, 1) QS_PAIR(3, 0) QS_PAIR(3, 1) QS_PAIR(3, 2)
-          case WC_D3 + 0: do_densek<R, NR, 3, 14u>(a, g, creg, cregv, tok); break;
-          case WC_D3 + 1: do_densek<R, NR, 3, 13u>(a, g, creg, cregv, tok); break;
-          case WC_D3 + 2: do_densek<R, NR, 3, 11u>(a, g, creg, cregv, tok); break;
-          case WC_D3 + 3: do_densek<R, NR, 3, 7u>(a, g, creg, cregv, tok); break;
-          case WC_D4: do_densek<R, NR, 4, 15u>(a, g, creg, cregv, tok); break;
+          case WC_D3 + 0: QS_V(do_densek<R, NR, 3, 14u>(a[v], g, creg, cregv, tok)) break;
+          case WC_D3 + 1: QS_V(do_densek<R, NR, 3, 13u>(a[v], g, creg, cregv, tok)) break;
+          case WC_D3 + 2: QS_V(do_densek<R, NR, 3, 11u>(a[v], g, creg, cregv, tok)) break;
+          case WC_D3 + 3: QS_V(do_densek<R, NR, 3, 7u>(a[v], g, creg, cregv, tok)) break;
+          case WC_D4: QS_V(do_densek<R, NR, 4, 15u>(a[v], g, creg, cregv, tok)) break;
           default: __builtin_unreachable();
         }
       } else {
@@ -220,60 +320,127 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[1 << RB], char* lds, const FO
   }
 }
 
-// One workgroup, one tile: load, ops, store.  nsmall != 0: a register of nsmall
-// amplitudes, fewer than a tile has; the rest of the tile is zeros.
-template <typename R, int RB, int TB, bool HEAVY>
-__global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k_wires(cx<R>* __restrict__ v, const PassHdr* __restrict__ H,
-                                                   const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
-                                                   const uint32_t* __restrict__ aux, uint32_t nsmall) {
-  constexpr int NR = 1 << RB, K = RB + TB;
-  extern __shared__ __align__(16) char lds_raw[];
-  const uint32_t tid = threadIdx.x, blk = blockIdx.x;
-  const FOpW* P = ops + H->op0;
-  const cx<R>* G = coef + H->coef0;
-  // diagonal tables, read per lane, are staged behind the relayout image
-  cx<R>* C = reinterpret_cast<cx<R>*>(lds_raw) + (H->uses_lds ? (1 << (K - 1)) : 0);
-  if (H->nstage) {
-    for (int i = (int)tid; i < H->nstage; i += (int)blockDim.x) C[i] = G[i];
-    __syncthreads();
-  }
-  cx<R> a[NR];
-  const uint64_t tb = insert_zeros((uint64_t)blk, H->sorted, K);
-  {
-    uint64_t gin = 0;
+// The wave's tiles from v (NV vectors at the same offsets).
+template <typename R, int RB, int TB, int NV>
+__device__ __forceinline__ void wire_load(cx<R> (&a)[NV][1 << RB], const cx<R>* const (&v)[NV],
+                                          const PassHdr* __restrict__ H, uint64_t tb, uint32_t tid, uint32_t nsmall) {
+  constexpr int NR = 1 << RB;
+  uint64_t gin = 0;
 #pragma unroll
-    for (int b = 0; b < TB; ++b) gin |= (uint64_t)((tid >> b) & 1u) << H->tbits[H->ts0[b]];
-    const uint64_t base = tb | gin;
+  for (int b = 0; b < TB; ++b) gin |= (uint64_t)((tid >> b) & 1u) << H->tbits[H->ts0[b]];
+  const uint64_t base = tb | gin;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       uint64_t g = 0;
 #pragma unroll
       for (int b = 0; b < RB; ++b)
         if ((r >> b) & 1) g |= 1ull << H->tbits[H->rs0[b]];
-      if (nsmall == 0) a[r] = ld_nt(v + (base | g));
-      else a[r] = (uint32_t)(base | g) < nsmall ? ld(v + (base | g)) : zero<R>();
+      if (nsmall == 0) a[i][r] = ld_nt(v[i] + (base | g));
+      else a[i][r] = (uint32_t)(base | g) < nsmall ? ld(v[i] + (base | g)) : zero<R>();
     }
-  }
-  const int nops = H->nops;
-  for (int o = 0; o < nops; ++o) {
-    const FOpW e = P[o];
-    if ((blk & e.w[6]) != e.w[7]) continue;
-    wire_op<R, RB, TB, HEAVY>(a, lds_raw, e, C, G, aux, tid, blk);
-  }
-  if (H->sync_store) __syncthreads();
-  // store: per-lane and per-register address bits, flips that depend on the tile
+}
+
+// Store: per-lane and per-register address bits, flips that depend on the tile.
+template <typename R, int RB, int TB, int NV>
+__device__ __forceinline__ void wire_store(const cx<R> (&a)[NV][1 << RB], cx<R>* const (&v)[NV],
+                                           const PassHdr* __restrict__ H, uint64_t tb, uint32_t tid, uint32_t blk,
+                                           uint32_t nsmall) {
+  constexpr int NR = 1 << RB;
   uint64_t base = tb ^ H->sflip;
 #pragma unroll
   for (int b = 0; b < TB; ++b) base ^= ((tid >> b) & 1u) ? H->st[b] : 0ull;
   const int nx = H->nsx;
   for (int i = 0; i < nx; ++i) base ^= ((blk >> H->sxb[i]) & 1u) ? H->sxm[i] : 0ull;
 #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    uint64_t g = 0;
+  for (int i = 0; i < NV; ++i) {
+    if (v[i] == nullptr) continue;
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
-      if ((r >> b) & 1) g ^= H->sr[b];
-    if (nsmall == 0 || (uint32_t)(base ^ g) < nsmall) st_nt(v + (base ^ g), a[r]);
+    for (int r = 0; r < NR; ++r) {
+      uint64_t g = 0;
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+        if ((r >> b) & 1) g ^= H->sr[b];
+      if (nsmall == 0 || (uint32_t)(base ^ g) < nsmall) st_nt(v[i] + (base ^ g), a[i][r]);
+    }
+  }
+}
+
+// The ops of a pass on the wave's tiles.  Returns the workgroup's gradient row in LDS
+// (NV = 2): per column one entry a wave.
+template <typename R, int RB, int TB, int NV, bool HEAVY>
+__device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, const PassHdr* __restrict__ H,
+                                            const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
+                                            const uint32_t* __restrict__ aux, uint32_t tid, uint32_t blk) {
+  constexpr int K = RB + TB;
+  const FOpW* P = ops + H->op0;
+  const cx<R>* G = coef + H->coef0;
+  // behind the relayout images: diagonal tables (read per lane), the gradient row
+  cx<R>* C = reinterpret_cast<cx<R>*>(lds) + (H->uses_lds ? NV << (K - 1) : 0);
+  if (H->nstage) {
+    for (int i = (int)tid; i < H->nstage; i += (int)blockDim.x) C[i] = G[i];
+    __syncthreads();
+  }
+  double* row = reinterpret_cast<double*>(C + H->nstage);
+  double* grad = row + (tid >> 6);
+  const int nops = H->nops;
+  for (int o = 0; o < nops; ++o) {
+    const FOpW e = P[o];
+    if ((blk & e.w[6]) != e.w[7]) continue;
+    wire_op<R, RB, TB, NV, HEAVY>(a, lds, e, C, G, aux, tid, blk, grad);
+  }
+  return row;
+}
+
+// One workgroup, one tile: load, ops, store.  nsmall != 0: a register of nsmall
+// amplitudes, fewer than a tile has; the rest of the tile is zeros.
+template <typename R, int RB, int TB, bool HEAVY>
+__global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k_wires(
+    cx<R>* __restrict__ v, const PassHdr* __restrict__ H, const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
+    const uint32_t* __restrict__ aux, uint32_t nsmall) {
+  extern __shared__ __align__(16) char lds_raw[];
+  const uint32_t tid = threadIdx.x, blk = blockIdx.x;
+  cx<R> a[1][1 << RB];
+  const uint64_t tb = insert_zeros((uint64_t)blk, H->sorted, RB + TB);
+  wire_load<R, RB, TB, 1>(a, {v}, H, tb, tid, nsmall);
+  wire_ops<R, RB, TB, 1, HEAVY>(a, lds_raw, H, ops, coef, aux, tid, blk);
+  if (H->sync_store) __syncthreads();
+  wire_store<R, RB, TB, 1>(a, {v}, H, tb, tid, blk, nsmall);
+}
+
+// The same for one pass of several programs (jobs), each on its own part of psi (NV
+// = 1) or of psi and lam (NV = 2, with the tile's gradient row).
+template <typename R, int NV, bool HEAVY>
+__global__ __launch_bounds__(256, HEAVY || (NV == 2 && sizeof(R) == 8) ? 2 : NV == 2 ? 3 : sizeof(R) == 8 ? 4 : 7) void k_jobs(
+    cx<R>* __restrict__ psi, cx<R>* __restrict__ lam, const char* __restrict__ image, const WireJobs J,
+    double* __restrict__ partial) {
+  extern __shared__ __align__(16) char lds_raw[];
+  const uint32_t tid = threadIdx.x;
+  int j = 0;
+  while (j + 1 < J.n && blockIdx.x >= J.j[j + 1].blk0) ++j;
+  const WireJob& job = J.j[j];
+  const uint32_t blk = blockIdx.x - job.blk0;
+  const PassHdr* H = reinterpret_cast<const PassHdr*>(image + job.hdr);
+  const uint64_t tb = insert_zeros((uint64_t)blk, H->sorted, 12);
+  cx<R> a[NV][16];
+  if constexpr (NV == 1) {
+    wire_load<R, 4, 8, 1>(a, {psi + job.off}, H, tb, tid, 0);
+  } else {
+    wire_load<R, 4, 8, 2>(a, {psi + job.off, lam + job.off}, H, tb, tid, 0);
+  }
+  double* row = wire_ops<R, 4, 8, NV, HEAVY>(a, lds_raw, H, reinterpret_cast<const FOpW*>(image + job.ops),
+                                              reinterpret_cast<const cx<R>*>(image + job.coef),
+                                              reinterpret_cast<const uint32_t*>(image + job.aux), tid, blk);
+  if (H->sync_store || NV == 2) __syncthreads();
+  if constexpr (NV == 1) {
+    wire_store<R, 4, 8, 1>(a, {psi + job.off}, H, tb, tid, blk, 0);
+  } else {
+    wire_store<R, 4, 8, 2>(a, {job.keep & 1 ? psi + job.off : nullptr, job.keep & 2 ? lam + job.off : nullptr}, H, tb,
+                           tid, blk, 0);
+    const int ng = H->ngrad;
+    double* out = partial + job.part + (uint64_t)blk * ng;
+    for (int i = (int)tid; i < ng; i += 256) out[i] = (row[4 * i] + row[4 * i + 1]) + (row[4 * i + 2] + row[4 * i + 3]);
   }
 }
 

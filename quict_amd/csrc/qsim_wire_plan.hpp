@@ -45,15 +45,17 @@ struct WireProgram {
   std::vector<qs_gate> g;     // bits[] hold wires
   std::vector<char> single;   // a gate the tile kernel cannot take: a pass of its own
   std::vector<int> home;      // wire -> index bit its amplitudes end on
+  std::vector<WireSym> sym;   // parallel to g
 };
 
 // What the scheduler and the grouping need to know of a gate.
-enum WClass : uint8_t { W_REAL, W_PHASE, W_CX, W_FLIP, W_TABLE, W_SINGLE };
+enum WClass : uint8_t { W_REAL, W_PHASE, W_CX, W_FLIP, W_TABLE, W_SINGLE, W_ZMEAS /* phase that is measured */ };
 
 static bool pure_exchange(const qs_gate& g) { return g.m[0] == 1.0 && g.m[1] == 0.0 && g.m[2] == 1.0 && g.m[3] == 0.0; }
 
-static WClass wire_class(const qs_gate& g, bool single) {
+static WClass wire_class(const qs_gate& g, bool single, const WireSym& sym) {
   if (single) return W_SINGLE;
+  if (g.kind == QS_GATE_PHASE && sym.meas != 0.0) return W_ZMEAS;
   if (g.kind == QS_GATE_PHASE) return W_PHASE;
   if (g.kind == QS_GATE_DIAG) return W_TABLE;
   if (g.kind == QS_GATE_XPERM && g.ncontrols == 0 && pure_exchange(g)) return W_FLIP;
@@ -76,6 +78,7 @@ struct WireReducer {
   char touched[64];  // 1: gates diagonal on the wire came after it
   int lastt[64];     // the last gate touching the wire, or -1
   cplx gphase{1.0, 0.0};
+  bool keep_phase = true;  // false: the state is wanted up to a common phase
 
   WireReducer(const Config& cfg, WireProgram& w, int n) : c(cfg), W(w) {
     for (int b = 0; b < 64; ++b) lab[b] = b, last1[b] = -1, touched[b] = 0, lastt[b] = -1;
@@ -83,9 +86,10 @@ struct WireReducer {
   }
 
   // Append a gate (bits already wires) and note which wires it touches.
-  int put(const qs_gate& g, bool single = false) {
+  int put(const qs_gate& g, bool single = false, const WireSym& sym = {}) {
     const int id = (int)W.g.size();
     W.g.push_back(g);
+    W.sym.push_back(sym);
     W.single.push_back(single);
     dead.push_back(0);
     const bool diag = !single && gate_diag_like(g);
@@ -191,6 +195,26 @@ struct WireReducer {
     for (int i = 0; i < k; ++i) g.bits[i] = ws[i];
     g.m[0] = f.first, g.m[1] = f.second;
     put(g);
+  }
+
+  // exp(-i sgn theta[slot] P / 2), P = X, Y, Z (axis 0, 1, 2) on a circuit bit, up to
+  // a common phase; meas: Im <lam|P|psi> is taken before it.
+  void param(int axis, int bit, int slot, double sgn, bool meas) {
+    const int w = lab[bit];
+    const double flip = ((F >> w) & 1) && axis != 0 ? -1.0 : 1.0;  // X Y X = -Y, X Z X = -Z
+    qs_gate g;
+    std::memset(&g, 0, sizeof(g));
+    g.ntargets = 1;
+    g.bits[0] = w;
+    g.kind = axis == 2 ? QS_GATE_PHASE : QS_GATE_DENSE;
+    WireSym s;
+    s.slot = slot;
+    s.sgn = sgn * flip;
+    s.meas = meas ? flip : 0.0;
+    const double P[8] = {1, 0, 0, 0, 0, 0, 0, 1}, Q[8] = {1, 0, 0, 0, 0, 0, 0, -1};
+    if (axis == 0) one_qubit(w, P, true);  // X = S^dagger Y S
+    put(g, false, s);
+    if (axis == 0) one_qubit(w, Q, true);
   }
 
   // Turn a frame flip into an X gate.
@@ -300,16 +324,19 @@ struct WireReducer {
     for (int b = 0; b < n; ++b) W.home[lab[b]] = b;
     std::vector<qs_gate> in;
     std::vector<char> ins;
+    std::vector<WireSym> insym;
     in.swap(W.g);
     ins.swap(W.single);
+    insym.swap(W.sym);
     W.g.reserve(in.size() + 16);
     cplx pend[64];
     for (int w = 0; w < 64; ++w) pend[w] = {1.0, 0.0};
     const double eps = 5e-16;  // rounding of the factors: not an op
     auto is_one = [&](cplx f) { return std::fabs(f.first - 1.0) <= eps && std::fabs(f.second) <= eps; };
-    auto push = [&](const qs_gate& g, bool single) {
+    auto push = [&](const qs_gate& g, bool single, const WireSym& sym = {}) {
       W.g.push_back(g);
       W.single.push_back(single);
+      W.sym.push_back(sym);
     };
     auto flush = [&](int w) {
       if (!is_one(pend[w])) {
@@ -327,6 +354,11 @@ struct WireReducer {
       if (dead[k]) continue;
       const qs_gate& g = in[k];
       const int nb = g.ncontrols + g.ntargets;
+      if (insym[k].slot >= 0) {
+        if (g.kind == QS_GATE_DENSE) flush(g.bits[0]);
+        push(g, false, insym[k]);
+        continue;
+      }
       if (!ins[k] && g.kind == QS_GATE_PHASE && nb == 1) {
         pend[g.bits[0]] = cm_(pend[g.bits[0]], {g.m[0], g.m[1]});
         continue;
@@ -356,7 +388,7 @@ struct WireReducer {
       push(g, ins[k]);
     }
     for (int w = 0; w < n; ++w) flush(w);
-    if (!is_one(gphase)) {  // the common factor multiplies whole tiles, in one pass
+    if (keep_phase && !is_one(gphase)) {  // the common factor multiplies whole tiles, in one pass
       qs_gate g;
       std::memset(&g, 0, sizeof(g));
       g.kind = QS_GATE_PHASE;
@@ -442,7 +474,8 @@ static double unit_tolerance(uint32_t amp_bytes) { return amp_bytes == 16 ? 1e-1
 // that may go to the low index bits at the store (at least L of them); home[j]:
 // the index bit where tile-local bit j ends, to be taken where it is free.
 static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Config& c, uint32_t amp_bytes,
-                          uint32_t allowed, const std::vector<int>& home, PassHdr& H, FusedProgram& prog) {
+                          uint32_t allowed, const std::vector<int>& home, PassHdr& H, FusedProgram& prog,
+                          std::vector<GradCol>& gcols) {
   const int RB = c.RB, TB = c.TB, K = RB + TB, L = c.L, NR = 1 << RB;
   const uint32_t full = (1u << K) - 1;
   const double tol = unit_tolerance(amp_bytes);
@@ -467,7 +500,7 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
     l.cls = cls[gi];
     l.all = l.mix = l.ctl = l.outer = 0;
     const int nb = g.ncontrols + g.ntargets;
-    const bool diag = l.cls == W_PHASE || l.cls == W_TABLE;
+    const bool diag = l.cls == W_PHASE || l.cls == W_TABLE || l.cls == W_ZMEAS;
     l.loc.resize(nb);
     for (int i = 0; i < nb; ++i) {
       const int j = g2l[g.bits[i]];
@@ -528,12 +561,33 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
     const bool two = b.op.kind == F_DENSE2 || b.op.kind == F_XX2 || b.op.kind == F_DIAG;
     if (l.outer != 0 || !two || !try_merge(built, b, NR, RB)) built.push_back(std::move(b));
   };
+  // Gradient column before a measured gate, its sign with the wire's pending flip.
+  auto emit_meas = [&](const LocalGate& l, int y) {
+    const WireSym& sym = prog.psym[l.idx];
+    Built b;
+    std::memset(&b.op, 0, sizeof(b.op));
+    b.op.kind = F_MEAS;
+    b.op.pure = y;
+    b.op.pos[0] = slot_of(cur, __builtin_ctz(l.all));
+    b.op.coef = (int)gcols.size();
+    b.slots = 1u << b.op.pos[0];
+    gcols.push_back({sym.slot, (l.all & aff) ? -sym.meas : sym.meas});
+    built.push_back(std::move(b));
+  };
   auto emit_phase = [&](const LocalGate& l) {
     const qs_gate& g = prog.pgates[l.idx];
+    const WireSym& sym = prog.psym[l.idx];
     OpBuild ob;
     std::memset(&ob.op, 0, sizeof(ob.op));
     ob.op.kind = F_PHASE;
-    phase_payload({g.m[0], g.m[1]}, tol, ob);
+    if (sym.slot >= 0) {
+      ob.op.sym = 1 + sym.slot;
+      ob.op.sgn = (l.all & aff) ? -sym.sgn : sym.sgn;
+      ob.op.pure = 2;
+      ob.coef = {0.0, 0.0};
+    } else {
+      phase_payload({g.m[0], g.m[1]}, tol, ob);
+    }
     for (uint32_t m = l.all; m; m &= m - 1) {
       const int s = slot_of(cur, __builtin_ctz(m));
       if (s < RB) ob.op.creg |= 1u << s;
@@ -546,7 +600,20 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
   auto emit_gate = [&](const LocalGate& l) -> int {
     // controls outside the tile are the op's tile predicate: drop them here
     const qs_gate& g = prog.pgates[l.idx];
+    const WireSym& sym = prog.psym[l.idx];
     OpBuild ob;
+    if (sym.slot >= 0) {  // rotation about Y
+      if (sym.meas != 0.0) emit_meas(l, 1);
+      std::memset(&ob.op, 0, sizeof(ob.op));
+      ob.op.kind = F_ROT;
+      ob.op.npos = 1;
+      ob.op.pos[0] = slot_of(cur, __builtin_ctz(l.mix));
+      ob.op.sym = 1 + sym.slot;
+      ob.op.sgn = (l.all & aff) ? -sym.sgn : sym.sgn;
+      ob.coef = {0.0, 0.0};
+      add_op(ob, l);
+      return QS_OK;
+    }
     set_flips();
     int rc;
     if (l.outer == 0) {
@@ -642,6 +709,9 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
           case W_PHASE:
             if ((last || (l.all & regs)) && !(l.all & aff) && mask_row_clean(l.all)) emit_phase(l), ran = true;
             break;
+          case W_ZMEAS:
+            if (!(l.all & ~regs) && mask_row_clean(l.all)) emit_meas(l, 0), emit_phase(l), ran = true;
+            break;
           case W_TABLE:
             if (__builtin_popcount(l.all & ~regs) <= 2 && mask_row_clean(l.all)) scan_rc = emit_gate(l), ran = true;
             break;
@@ -683,6 +753,10 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
           case W_PHASE:
             ran = (l.all & R) && !(l.all & dv);
             break;
+          case W_ZMEAS:
+            ran = !(l.all & ~R) && !(l.all & dv);
+            if (ran) score += 4;
+            break;
           case W_TABLE:
             ran = __builtin_popcount(l.all & ~R) <= 2 && !(l.all & dv);
             if (ran) score += 4;
@@ -717,7 +791,8 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
         // candidates: what the unblocked gates with missing register bits need
         if (!((l.all & wm) | (l.mix & wa))) {
           uint32_t need = 0;
-          if (l.cls != W_PHASE && l.cls != W_TABLE) need = l.mix & ~R;
+          if (l.cls == W_ZMEAS) need = l.all & ~R;
+          else if (l.cls != W_PHASE && l.cls != W_TABLE) need = l.mix & ~R;
           else if (l.cls == W_TABLE) {
             uint32_t m = l.all & ~R;
             for (int k = __builtin_popcount(m); k > 2; --k, m &= m - 1) need |= m & (~m + 1);
@@ -1023,7 +1098,7 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
   for (size_t i = 0; i < nb; ++i) {
     Built& b = built[i];
     if (b.op.kind == F_DIAG && b.op.creg == 0) continue;  // the merged product is the identity
-    if (b.op.kind != F_DIAG && b.op.kind != F_RELAYOUT) put_coef(b);
+    if (b.op.kind != F_DIAG && b.op.kind != F_RELAYOUT && b.op.kind != F_MEAS) put_coef(b);
     prog.ops.push_back(b.op);
   }
   for (int b = 0; b < RB; ++b) H.rs1[b] = cur.rs[b];
@@ -1067,14 +1142,14 @@ static int schedule_wires(const std::vector<WClass>& cls, PassPlan& p, const Con
 
 // ---- grouping --------------------------------------------------------------------
 
-// Plans the whole program; every fused pass goes to done(header, first aux word,
+// Plans the whole program, whose gates fill(reducer) adds; every fused pass goes to done(header, first aux word,
 // plan) as soon as it is scheduled and is appended to prog.plans after that.
 //
 // A register of at most K bits is one tile: wires up to K are idle and every store
 // puts all wires home (bits n..K-1 are not there: the kernel neither loads nor
 // stores them).
-template <typename Done>
-static int plan_wires(const qs_gate* gates, int ngates, int nbits, const Config& c, uint32_t amp_bytes,
+template <typename Fill, typename Done>
+static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, uint32_t amp_bytes,
                       FusedProgram& prog, const Done& done) {
   const int K = c.RB + c.TB, L = c.L;
   const int n = std::max(nbits, K);
@@ -1083,7 +1158,7 @@ static int plan_wires(const qs_gate* gates, int ngates, int nbits, const Config&
   {
     WireReducer red(c, W, n);
     W.g.reserve(ngates + 8);
-    for (int i = 0; i < ngates; ++i) red.add(gates[i]);
+    fill(red);
     red.finish(n, unit_tolerance(amp_bytes));
   }
   const int G = (int)W.g.size();
@@ -1095,16 +1170,17 @@ static int plan_wires(const qs_gate* gates, int ngates, int nbits, const Config&
   std::vector<int> rw(G);
   for (int i = 0; i < G; ++i) {
     const qs_gate& g = W.g[i];
-    cls[i] = wire_class(g, W.single[i]);
+    cls[i] = wire_class(g, W.single[i], W.sym[i]);
     ra[i] = gate_mask(g);
     uint64_t t = 0;
     for (int k = 0; k < g.ntargets; ++k) t |= 1ull << g.bits[g.ncontrols + k];
-    rm[i] = cls[i] == W_SINGLE ? ra[i] : cls[i] == W_PHASE || cls[i] == W_TABLE ? 0 : t;
-    rn[i] = cls[i] == W_TABLE ? ra[i] : rm[i];
+    rm[i] = cls[i] == W_SINGLE ? ra[i] : cls[i] == W_PHASE || cls[i] == W_TABLE || cls[i] == W_ZMEAS ? 0 : t;
+    rn[i] = cls[i] == W_TABLE || cls[i] == W_ZMEAS ? ra[i] : rm[i];
     rid[i] = i;
     rw[i] = cls[i] == W_PHASE ? 1 : cls[i] == W_FLIP ? 0 : 2;
   }
   prog.pgates = W.g;
+  prog.psym = W.sym;
   std::vector<int> pos(n), at(n);  // wire -> index bit, index bit -> wire
   for (int b = 0; b < n; ++b) pos[b] = at[b] = b;
   auto translate = [&](int gi) {
@@ -1122,12 +1198,13 @@ static int plan_wires(const qs_gate* gates, int ngates, int nbits, const Config&
   // gates need besides (in order, each once); taken: the gates (positions).
   auto scan = [&](uint64_t S, std::vector<uint64_t>* cand, std::vector<int>* taken) -> int {
     uint64_t wa = 0, wm = 0;
-    int w = 0, tables = 0;
+    int w = 0, tables = 0, meas = 0;
     for (int k = 0; k < R; ++k) {
       const uint64_t a = ra[k], m = rm[k];
       if (!((a & wm) | (m & wa))) {
         const uint64_t need = rn[k] & ~S;
-        const bool room = cls[rid[k]] != W_TABLE || ++tables <= max_tables;
+        bool room = cls[rid[k]] != W_TABLE || ++tables <= max_tables;
+        if (W.sym[rid[k]].meas != 0.0) room = ++meas <= FMAX_GRAD;
         if (!need && room && cls[rid[k]] != W_SINGLE) {
           w += rw[k];
           if (taken) taken->push_back(k);
@@ -1164,8 +1241,11 @@ static int plan_wires(const qs_gate* gates, int ngates, int nbits, const Config&
     for (int gi : p.gates) translate(gi);
     const int a0 = (int)prog.aux.size();
     PassHdr H;
-    int rc = schedule_wires(cls, p, c, amp_bytes, al, home, H, prog);
+    std::vector<GradCol> cols;
+    int rc = schedule_wires(cls, p, c, amp_bytes, al, home, H, prog, cols);
     if (rc) return rc;
+    H.ngrad = (int)cols.size();
+    prog.gcols.push_back(std::move(cols));
     std::vector<int> wires(K);
     for (int j = 0; j < K; ++j) wires[j] = at[p.tbits[j]];
     for (int j = 0; j < K; ++j) {
@@ -1316,6 +1396,68 @@ static int plan_wires(const qs_gate* gates, int ngates, int nbits, const Config&
     if (rc) return rc;
   }
   return QS_OK;
+}
+
+}  // namespace qs
+
+namespace qs {
+
+// ---- programs with parameters ------------------------------------------------------
+
+// One gate of a variational circuit: a fixed gate with its inverse, or a rotation
+// exp(-i theta[slot] P / 2), P = X, Y, Z (axis 0, 1, 2), on a circuit bit.
+struct VarOp {
+  int axis = -1;  // -1: fixed
+  int bit = 0, slot = -1;
+  qs_gate g, inv;
+};
+
+// Plans the circuit (or, backward: its inverse, with a gradient column before every
+// rotation's inverse) without its angles.  QS_ERR_UNSUPPORTED for circuits with a
+// gate that needs a pass of its own.
+static int build_var(const std::vector<VarOp>& ops, bool backward, int n, const Config& c, uint32_t amp_bytes,
+                     FusedProgram& prog) {
+  auto fill = [&](WireReducer& red) {
+    red.keep_phase = false;
+    for (size_t i = 0; i < ops.size(); ++i) {
+      const VarOp& o = ops[backward ? ops.size() - 1 - i : i];
+      if (o.axis < 0) red.add(backward ? o.inv : o.g);
+      else red.param(o.axis, o.bit, o.slot, backward ? -1.0 : 1.0, backward);
+    }
+  };
+  auto done = [&](const PassHdr& H, int a0, PassPlan& p) -> int {
+    p.hdr = (int)prog.hdrs.size();
+    prog.hdrs.push_back(H);
+    prog.aux0.push_back(a0);
+    return QS_OK;
+  };
+  const int rc = plan_wires(fill, (int)ops.size(), n, c, amp_bytes, prog, done);
+  if (rc) return rc;
+  for (const PassPlan& p : prog.plans)
+    if (!p.fused) {
+      set_error("a gate of the circuit needs a pass of its own");
+      return QS_ERR_UNSUPPORTED;
+    }
+  return QS_OK;
+}
+
+// Shear payload of a rotation by sgn * theta, from cos and sin of theta / 2: |t| <= 1
+// (a rotation by more than a half turn is taken with a minus sign, which a
+// state known up to a phase does not notice).
+static void rot_payload(double ch, double sh, double sgn, double* out) {
+  sh *= sgn;
+  if (ch < 0.0) ch = -ch, sh = -sh;
+  out[0] = -sh / (1.0 + ch);
+  out[1] = sh;
+}
+// The same for the phase exp(i sgn theta); returns the op's `pure`.
+static int phase_payload_sym(double c, double s, double sgn, double* out) {
+  s *= sgn;
+  const bool neg = c < 0.0;
+  if (neg) c = -c, s = -s;
+  out[0] = -s / (1.0 + c);
+  out[1] = s;
+  return neg ? 3 : 2;
 }
 
 }  // namespace qs

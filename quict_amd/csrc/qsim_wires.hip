@@ -25,6 +25,30 @@ template <typename R, int RB, int TB> void wires_lds_attr() {
   (void)hipFuncSetAttribute((const void*)k_wires<R, RB, TB, false>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
+template <typename R>
+void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs, uint32_t blocks, bool heavy, double* partial,
+                 size_t lds, hipStream_t s) {
+  static bool attr = false;  // two images, tables and gradient rows can pass 64 KiB
+  if (!attr) {
+    const int bytes = 150 * 1024;
+    (void)hipFuncSetAttribute((const void*)k_jobs<R, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute((const void*)k_jobs<R, 1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute((const void*)k_jobs<R, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute((const void*)k_jobs<R, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    attr = true;
+  }
+  const dim3 g(blocks), t(256);
+  if (!lam && heavy) hipLaunchKernelGGL((k_jobs<R, 1, true>), g, t, lds, s, psi, lam, image, jobs, partial);
+  else if (!lam) hipLaunchKernelGGL((k_jobs<R, 1, false>), g, t, lds, s, psi, lam, image, jobs, partial);
+  else if (heavy) hipLaunchKernelGGL((k_jobs<R, 2, true>), g, t, lds, s, psi, lam, image, jobs, partial);
+  else hipLaunchKernelGGL((k_jobs<R, 2, false>), g, t, lds, s, psi, lam, image, jobs, partial);
+}
+
+template void launch_jobs<double>(cx<double>*, cx<double>*, const char*, const WireJobs&, uint32_t, bool, double*,
+                                  size_t, hipStream_t);
+template void launch_jobs<float>(cx<float>*, cx<float>*, const char*, const WireJobs&, uint32_t, bool, double*, size_t,
+                                 hipStream_t);
+
 #define QS_WIRES(R, TB)                                                                                          \
   template void launch_wires<R, 4, TB>(cx<R>*, uint64_t, const PassHdr&, const PassHdr*, const FOpW*,            \
                                        const cx<R>*, const uint32_t*, uint32_t, size_t, hipStream_t);            \

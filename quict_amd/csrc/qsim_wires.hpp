@@ -20,15 +20,17 @@ enum WCode : uint32_t {
   WC_TABLE = 96,     // diagonal table in LDS, per register
   WC_LANE = 97,      // diagonal table in LDS, one entry per lane
   WC_U2 = 98,        // + P: complex 2x2
-  WC_HEAVY = 102,    // from here on: only in the HEAVY instance
-  WC_U2G = 102,      // + P: complex 2x2 under register and thread controls
-  WC_EXG = 106,      // + P: exchange under register and thread controls
-  WC_D2 = 110,       // + pair: complex 4x4 under controls
-  WC_XX = 116,       // + pair: diagonal + anti-diagonal
-  WC_SW = 122,       // + pair: exchange of 01 and 10 under controls
-  WC_D3 = 128,       // + missing position: 8x8 (RB = 4)
-  WC_D4 = 132,
-  WC_END = 133
+  WC_MZ = 102,       // + P: gradient column Im <lam|Z|psi> (two vectors)
+  WC_MY = 106,       // + P: Im <lam|Y|psi>
+  WC_HEAVY = 110,    // from here on: only in the HEAVY instance
+  WC_U2G = 110,      // + P: complex 2x2 under register and thread controls
+  WC_EXG = 114,      // + P: exchange under register and thread controls
+  WC_D2 = 118,       // + pair: complex 4x4 under controls
+  WC_XX = 124,       // + pair: diagonal + anti-diagonal
+  WC_SW = 130,       // + pair: exchange of 01 and 10 under controls
+  WC_D3 = 136,       // + missing position: 8x8 (RB = 4)
+  WC_D4 = 140,
+  WC_END = 141
 };
 // register pairs (P0 > P1) in the order 10, 20, 21, 30, 31, 32
 static int wire_pair(int p0, int p1) { return p0 * (p0 - 1) / 2 + p1; }
@@ -44,6 +46,9 @@ static FOpW encode_wire_op(const FOp& o) {
       break;
     case F_ROT:
       code = WC_ROT + o.pos[0];
+      break;
+    case F_MEAS:
+      code = (o.pure ? WC_MY : WC_MZ) + o.pos[0];
       break;
     case F_PERM1:
       if (!o.pure) code = WC_EXG + o.pos[0];
@@ -90,6 +95,27 @@ static FOpW encode_wire_op(const FOp& o) {
   e.w[7] = o.cblkv;
   return e;
 }
+
+// One pass of one program in a launch of several (12-bit tiles): byte offsets into
+// the images (see VarImage), and where its amplitudes are.
+struct WireJob {
+  uint32_t hdr, ops, aux, coef;
+  uint64_t off;    // first amplitude
+  uint64_t part;   // first entry of the gradient rows (tile by tile, ngrad each)
+  uint32_t blk0;   // first block; the jobs are in block order
+  uint32_t keep;   // two vectors: store psi (1), lam (2)
+};
+constexpr int WIRE_MAX_JOBS = 20;  // the widths of a QNN batch
+struct WireJobs {
+  int n;
+  WireJob j[WIRE_MAX_JOBS];
+};
+// lam == nullptr: one vector.  The kernel reads the programs through one pointer
+// argument, which it never writes: pointers inside the jobs would make every
+// descriptor a vector load.
+template <typename R>
+void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs, uint32_t blocks, bool heavy, double* partial,
+                 size_t lds, hipStream_t s);
 
 // One pass over the 2^(n-K) tiles of v: header hd, its device copy dh and the
 // program's device arrays; nsmall: amplitudes of a register below a tile, else 0.  The caller checks hipGetLastError().

@@ -23,7 +23,7 @@ import numpy as np
 from ..core import GateType, GATE_TYPE_TO_CLASS, Circuit
 from ..core import exception as qerr
 from .. import _native as nat
-from ..simulation.gate_compiler import compile_gate
+from ..simulation.gate_compiler import compile_gate, compile_gates
 
 _PAULI = {
     "I": np.eye(2, dtype=np.complex128),
@@ -95,6 +95,7 @@ class ParameterizedCircuit:
         self.nparams = 0
         self._template = None   # record templates, rebuilt after every add()
         self._work = None       # working copies of the templates' records
+        self._plans = {}        # (precision, device) -> planned circuit (or None), dropped by add()
 
     def add(self, gtype: GateType, qubits, param: Optional[int] = None, value=None):
         qubits = [qubits] if isinstance(qubits, int) else list(qubits)
@@ -105,7 +106,12 @@ class ParameterizedCircuit:
         vals = None if value is None else (list(value) if isinstance(value, (list, tuple)) else [value])
         self.ops.append((gtype, qubits, param, vals))
         self._template = None
+        self._plans = {}
         return self
+
+    def __getstate__(self):
+        # plans hold native handles and device memory: a copy makes its own
+        return {**self.__dict__, "_plans": {}}
 
     @staticmethod
     def hea(n: int, layers: int) -> "ParameterizedCircuit":
@@ -300,6 +306,97 @@ def _records_generic(pc: ParameterizedCircuit, theta: np.ndarray):
     return fwd, inv, der, slot, keep
 
 
+_AXES = {GateType.rx: 0, GateType.ry: 1, GateType.rz: 2, GateType.u1: 2, GateType.phase: 2}
+
+
+def _plan_records(pc: ParameterizedCircuit):
+    """Records of the fixed gates and of their inverses, rotation axes and slots; of
+    a trainable gate's record only the bit is set."""
+    G, n = len(pc.ops), pc.n
+    fwd = np.zeros(G, dtype=nat.QS_GATE_DTYPE)
+    axis = np.full(G, -1, dtype=np.int32)
+    slot = np.full(G, -1, dtype=np.int32)
+    fixed, made = [], {}
+    for j, (t, qubits, param, vals) in enumerate(pc.ops):
+        if param is not None:
+            axis[j], slot[j] = _AXES[t], param
+            fwd[j]["bits"][0] = n - 1 - qubits[0]
+            continue
+        g = made.get(t) if vals is None else None
+        if g is None:
+            g = GATE_TYPE_TO_CLASS[t]()
+            if vals is None:
+                made[t] = g
+            else:
+                g = g(*vals)
+        g = g.copy()
+        g.cargs, g.targs = qubits[: g.controls], qubits[g.controls:]
+        fixed.append((j, g))
+    recs, keep = compile_gates([g for _, g in fixed], n)
+    if len(recs) != len(fixed):  # a gate without a record (identity, barrier)
+        raise qerr.GateAlgorithmNotImplementError("circuit with gates that have no record")
+    rows = np.array([j for j, _ in fixed], dtype=np.int64)
+    inv = fwd.copy()
+    if len(rows):
+        fwd[rows] = recs
+        back = recs.copy()
+        m = back["m"].view(np.complex128)
+        m[:] = m.conj()
+        ex = (recs["kind"] == nat.GATE_XPERM) | (recs["kind"] == nat.GATE_SWAP)
+        m[ex, 0], m[ex, 1] = m[ex, 1].copy(), m[ex, 0].copy()
+        for t in (1, 2):
+            d = np.nonzero((recs["kind"] == nat.GATE_DENSE) & (recs["ntargets"] == t))[0]
+            D = 1 << t
+            m[d, : D * D] = m[d, : D * D].reshape(-1, D, D).transpose(0, 2, 1).reshape(-1, D * D)
+        for i in np.nonzero((recs["kind"] == nat.GATE_DENSE) & (recs["ntargets"] > 2))[0]:
+            compile_gate(fixed[i][1], n, back[i], keep, dagger=True)
+        inv[rows] = back
+    return fwd, inv, axis, slot, keep
+
+
+class _Plan:
+    """A circuit planned once for the energy gradient (qs_var_create)."""
+
+    def __init__(self, pc: ParameterizedCircuit, precision: str, device: int):
+        self.lib = nat.load_library()
+        self.nparams = pc.nparams
+        self.handle = ctypes.c_void_p(0)
+        fwd, inv, axis, slot, keep = _plan_records(pc)
+        P = ctypes.c_void_p
+        rc = self.lib.qs_var_create(nat.context(device), pc.n, nat.QS_C128 if precision == "double" else nat.QS_C64,
+                                    nat.gate_array_ptr(fwd), nat.gate_array_ptr(inv), len(fwd), axis.ctypes.data_as(P),
+                                    slot.ctypes.data_as(P), pc.nparams, ctypes.byref(self.handle))
+        del keep  # wide matrices are read during the call
+        nat.check(rc, "qs_var_create")
+
+    def __del__(self):
+        try:
+            if self.handle:
+                self.lib.qs_var_destroy(self.handle)
+                self.handle = None
+        except Exception:
+            pass
+
+
+def _plan_of(pc: ParameterizedCircuit, precision: str, device: int) -> Optional["_Plan"]:
+    """The circuit's plan, kept with the circuit until a gate is added.  None for
+    circuits the planned sweep does not take (trainable gates other than one-qubit
+    rotations and phases, gates that need a pass of their own, angles set by hand
+    to more parameters than the gates name): their gradients come from the gate
+    records."""
+    plans = pc.__dict__.setdefault("_plans", {})
+    key = (precision, device, pc.n, pc.nparams, len(pc.ops))
+    if key not in plans:
+        plan = None
+        if pc.ops and all(p is None or t in _AXES for t, _, p, _ in pc.ops):
+            try:
+                plan = _Plan(pc, precision, device)
+            except qerr.GateAlgorithmNotImplementError:
+                plan = None
+        plans[key] = plan
+    return plans[key]
+
+
 class _Engine:
     def __init__(self, n: int, precision: str, device: int):
         import torch
@@ -310,7 +407,8 @@ class _Engine:
         self.dcode = nat.QS_C128 if precision == "double" else nat.QS_C64
         self.lib = nat.load_library()
         self.ctx = nat.context(device)
-        self.psi = torch.empty(1 << n, dtype=self.tdtype, device=f"cuda:{device}")
+        # (at least one tile, see qs_var_gradient)
+        self.psi = torch.empty(max(1 << n, 4096), dtype=self.tdtype, device=f"cuda:{device}")
         self.lam = torch.empty_like(self.psi)
 
     def ptr(self, t):
@@ -357,10 +455,20 @@ def adjoint_gradient(pc: ParameterizedCircuit, theta: np.ndarray, H: PauliSum, p
                      device: int = 0) -> Tuple[float, np.ndarray]:
     theta = np.asarray(theta, dtype=np.float64)
     eng = _engine(pc.n, precision, device)
-    fwd, inv, der, slot, keep = _records(pc, theta, reuse=True)
     grads = np.zeros(max(pc.nparams, 1), dtype=np.float64)
     if not H.terms:
         return 0.0, grads[: pc.nparams]
+    plan = _plan_of(pc, precision, device) if theta.ndim == 1 and len(theta) >= pc.nparams else None
+    if plan is not None:
+        theta = np.ascontiguousarray(theta)
+        recs = H.records()
+        E = ctypes.c_double(0)
+        nat.check(eng.lib.qs_var_gradient(plan.handle, eng.ptr(eng.psi), eng.ptr(eng.lam),
+                                          theta.ctypes.data_as(ctypes.c_void_p),
+                                          ctypes.cast(recs, ctypes.c_void_p), len(recs), ctypes.byref(E),
+                                          grads.ctypes.data_as(ctypes.c_void_p), eng.stream()), "qs_var_gradient")
+        return E.value, grads[: pc.nparams]
+    fwd, inv, der, slot, keep = _records(pc, theta, reuse=True)
     # the fused forward passes are launched while they are planned; the sweep
     # below is planned while they run (measured on MI355X at 20 qubits, 480
     # parameters: 2.52 ms against 2.56 ms with the forward computed inside the

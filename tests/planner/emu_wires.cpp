@@ -250,3 +250,96 @@ extern "C" int wires_apply(double* vec, int n, const qs_gate* gates, int ngates,
     return -99;
   }
 }
+
+// Energy-gradient sweep of a variational circuit: psi runs the planned circuit from
+// |0...0>, lam = Z on index bit zbit of it, both run the planned inverse.  ops: axis,
+// bit, slot per gate and, for fixed gates, records g and their inverses inv.
+// grads[slot] receives Im <lam|P|psi> summed over the gates of the slot; psi the
+// state swept back to |0...0>; fwd the forward state (up to a phase).  stats: forward
+// and backward passes.
+extern "C" int wires_gradient(int n, int nops, const int* axis, const int* bit, const int* slot, const qs_gate* g,
+                              const qs_gate* inv, const double* theta, int zbit, int amp_bytes, double* fwd,
+                              double* psi_out, double* grads, int* stats) {
+  using namespace qs;
+  try {
+    Config c{4, 8, 4};
+    c.wires = true;
+    std::vector<VarOp> ops(nops);
+    for (int i = 0; i < nops; ++i) {
+      ops[i].axis = axis[i], ops[i].bit = bit[i], ops[i].slot = slot[i];
+      if (axis[i] < 0) ops[i].g = g[i], ops[i].inv = inv[i];
+    }
+    const uint64_t N = 1ull << n;
+    std::vector<zc> psi(N), lam(N);
+    psi[0] = 1.0;
+    for (int back = 0; back < 2; ++back) {
+      FusedProgram prog;
+      const int rc = build_var(ops, back, n, c, (uint32_t)amp_bytes, prog);
+      if (rc) return rc;
+      const int rc2 = check_passes(prog, c, 0, (int)prog.hdrs.size());
+      if (rc2) return rc2;
+      stats[back] = (int)prog.hdrs.size();
+      for (size_t h = 0; h < prog.hdrs.size(); ++h) {
+        PassHdr& H = prog.hdrs[h];
+        for (int i = 0; i < H.nops; ++i) {
+          FOp& o = prog.ops[H.op0 + i];
+          if (!o.sym) continue;
+          const double t = theta[o.sym - 1];
+          double* p = &prog.coef[2 * (size_t)(H.coef0 + o.coef)];
+          if (o.kind == F_ROT) rot_payload(std::cos(t / 2), std::sin(t / 2), o.sgn, p);
+          else o.pure = phase_payload_sym(std::cos(t), std::sin(t), o.sgn, p);
+        }
+        std::vector<double> cols(H.ngrad, 0.0);
+        const FOp* P = prog.ops.data() + H.op0;
+        const double* C = prog.coef.data() + 2 * (size_t)H.coef0;
+        if (!back) {
+          wire_pass(psi.data(), n, 4, 8, (uint32_t)amp_bytes, H, P, C, prog.aux.data());
+        } else {
+          // run both vectors op by op up to each measurement: as passes that stop there
+          std::vector<zc> a = psi, b = lam;
+          for (int i = 0; i <= H.nops; ++i) {
+            if (i < H.nops && P[i].kind != F_MEAS) continue;
+            if (i == H.nops) break;
+            std::vector<zc> x = psi, y = lam;
+            PassHdr S = H;  // the ops before i, stored where the layout stands (register bit pos[0] known)
+            std::vector<FOp> pre;
+            for (int k = 0; k < i; ++k)
+              if (P[k].kind != F_MEAS) pre.push_back(P[k]);
+            S.nops = (int)pre.size();
+            // store register r, thread t at the tile-local index (r | t << RB)
+            for (int q = 0; q < 4; ++q) S.sr[q] = 1ull << H.sorted[q];
+            for (int q = 0; q < 8; ++q) S.st[q] = 1ull << H.sorted[4 + q];
+            S.sflip = 0, S.nsx = 0;
+            wire_pass(x.data(), n, 4, 8, (uint32_t)amp_bytes, S, pre.data(), C, prog.aux.data());
+            wire_pass(y.data(), n, 4, 8, (uint32_t)amp_bytes, S, pre.data(), C, prog.aux.data());
+            const uint64_t m = 1ull << H.sorted[P[i].pos[0]];
+            double s = 0;
+            for (uint64_t k = 0; k < N; ++k) {
+              const zc z = P[i].pure ? ((k & m) ? zc(0, 1) : zc(0, -1)) * x[k ^ m] : ((k & m) ? -1.0 : 1.0) * x[k];
+              s += (std::conj(y[k]) * z).imag();
+            }
+            if (P[i].coef >= H.ngrad) throw std::runtime_error("gradient column out of range");
+            cols[P[i].coef] += s;
+          }
+          std::vector<FOp> all;
+          for (int k = 0; k < H.nops; ++k)
+            if (P[k].kind != F_MEAS) all.push_back(P[k]);
+          PassHdr S = H;
+          S.nops = (int)all.size();
+          wire_pass(psi.data(), n, 4, 8, (uint32_t)amp_bytes, S, all.data(), C, prog.aux.data());
+          wire_pass(lam.data(), n, 4, 8, (uint32_t)amp_bytes, S, all.data(), C, prog.aux.data());
+          for (int k = 0; k < H.ngrad; ++k) grads[prog.gcols[h][k].slot] += prog.gcols[h][k].sgn * cols[k];
+        }
+      }
+      if (!back) {
+        std::memcpy(fwd, psi.data(), N * sizeof(zc));
+        for (uint64_t k = 0; k < N; ++k) lam[k] = ((k >> zbit) & 1) ? -psi[k] : psi[k];
+      }
+    }
+    std::memcpy(psi_out, psi.data(), N * sizeof(zc));
+    return 0;
+  } catch (const std::exception& e) {
+    g_err = e.what();
+    return -99;
+  }
+}

@@ -204,3 +204,75 @@ def test_fewer_passes_than_whole_gates_in_the_tile(emu):
     recs, keep = compile_gates(QFT(4).gates if hasattr(QFT(4), "gates") else hea(16, 1, 1).gates, 16)
     check(emu, compile_gates(qft(16).gates, 16)[0], 16)
     check(emu, compile_gates(hea(16, 6, 2).gates, 16)[0], 16)
+
+
+def variational(n, nops, seed, hea_layers=0):
+    """(axis, bit, slot) per gate and the fixed gates: random rotations among CX, X,
+    Swap, CZ, H, Toffoli, or the hardware-efficient ansatz."""
+    from quict_amd.core import CZ, GateType
+    from quict_amd.gradient.adjoint import ParameterizedCircuit
+    rng = random.Random(seed)
+    if hea_layers:
+        return ParameterizedCircuit.hea(n, hea_layers)
+    pc = ParameterizedCircuit(n)
+    k = 0
+    for _ in range(nops):
+        t = rng.choice([GateType.rx, GateType.ry, GateType.rz, GateType.rx, GateType.cx, GateType.x, GateType.swap,
+                        GateType.cz, GateType.h, GateType.ccx, GateType.s])
+        nq = {GateType.cx: 2, GateType.swap: 2, GateType.cz: 2, GateType.ccx: 3}.get(t, 1)
+        rot = t in (GateType.rx, GateType.ry, GateType.rz)
+        pc.add(t, rng.sample(range(n), nq), param=(k if rng.random() < 0.8 else rng.randrange(k + 1)) if rot else None)
+        k += rot
+    return pc
+
+
+@pytest.mark.parametrize("n,nops,seed,layers", [(13, 90, 1, 0), (14, 140, 2, 0), (13, 0, 3, 2), (5, 60, 4, 0),
+                                                (8, 0, 5, 3)])
+def test_sweep_programs_give_the_shift_gradient(emu, n, nops, seed, layers):
+    """Planned forward program, planned inverse with gradient columns: the state, the
+    state swept back and d<Z>/d theta by the parameter-shift rule (two terms per gate
+    occurrence, so parameters used twice count twice)."""
+    from quict_amd.core import GateType
+    from quict_amd.gradient.adjoint import _records
+    pc = variational(n, nops, seed, layers)
+    theta = np.random.RandomState(seed).uniform(-7, 7, pc.nparams)
+    fwd, inv, _, slot, keep = _records(pc, theta)
+    axes = {GateType.rx: 0, GateType.ry: 1, GateType.rz: 2}
+    axis = np.array([axes[t] if p is not None else -1 for t, _, p, _ in pc.ops], dtype=np.int32)
+    bit = np.array([n - 1 - q[-1] for _, q, _, _ in pc.ops], dtype=np.int32)
+    zbit, N = n - 2, 1 << n
+    state, back, grads, st = np.zeros(N, complex), np.zeros(N, complex), np.zeros(pc.nparams), np.zeros(2, np.int32)
+    ptr = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    rc = emu.wires_gradient(n, len(pc.ops), ptr(axis), ptr(bit), ptr(slot), nat.gate_array_ptr(fwd),
+                            nat.gate_array_ptr(inv), ptr(theta), zbit, 16, ptr(state), ptr(back), ptr(grads), ptr(st))
+    assert rc == 0, emu.wires_last_error()
+
+    def run(recs):
+        v = np.zeros(N, complex)
+        v[0] = 1
+        emu.cpu_apply_gates(ptr(v), n, nat.gate_array_ptr(recs), len(recs), 4)
+        return v
+
+    sign = 1 - 2.0 * ((np.arange(N) >> zbit) & 1)
+    energy = lambda recs: float(np.sum(sign * np.abs(run(recs)) ** 2))
+    ref = run(fwd)
+    assert abs(abs(np.vdot(ref, state)) - 1) < 1e-12
+    assert abs(back[0]) > 1 - 1e-12
+    from quict_amd.simulation.gate_compiler import compile_gate
+    want = np.zeros(pc.nparams)
+    rotations = [j for j in range(len(pc.ops)) if axis[j] >= 0]
+    check_ = set(random.Random(0).sample(rotations, min(len(rotations), 12)))
+    by_slot = {}
+    for j in rotations:
+        by_slot.setdefault(int(slot[j]), []).append(j)
+    for s, js in by_slot.items():
+        if not check_ & set(js):
+            continue
+        for j in js:
+            for sh, w in ((np.pi / 2, 0.5), (-np.pi / 2, -0.5)):
+                r = fwd.copy()
+                t2 = theta.copy()
+                t2[s] += sh
+                compile_gate(pc.gate(j, t2), n, r[j], keep)
+                want[s] += w * energy(r)
+        assert abs(grads[s] - want[s]) < 1e-11
