@@ -57,16 +57,27 @@ struct ProgImage {
 template <typename R> static void pack_program(const FusedProgram& prog, const Config& c, ProgImage& im) {
   auto al = [](uint64_t b) { return (b + 255) & ~255ull; };
   im.hb = al(prog.hdrs.size() * sizeof(PassHdr));
-  im.ob = al(prog.ops.size() * sizeof(FOpW));
+  const uint64_t op_bytes = c.wires ? sizeof(WireOp<R>) : sizeof(FOpW);
+  im.ob = al((prog.ops.size() + 1) * op_bytes);  // (k_wires fetches one op ahead)
   im.xb = al(prog.aux.size() * sizeof(uint32_t));
   const uint64_t ncoef = prog.coef.size() / 2;
   im.cb = al(ncoef * sizeof(cx<R>));
   im.host.assign(im.hb + im.ob + im.xb + im.cb, 0);
   char* h = im.host.data();
   if (!prog.hdrs.empty()) std::memcpy(h, prog.hdrs.data(), prog.hdrs.size() * sizeof(PassHdr));
-  for (size_t i = 0; i < prog.ops.size(); ++i) {
-    const FOpW e = c.wires ? encode_wire_op(prog.ops[i]) : encode_op(prog.ops[i]);
-    std::memcpy(h + im.hb + i * sizeof(FOpW), &e, sizeof(FOpW));
+  if (c.wires) {
+    WireOp<R>* w = reinterpret_cast<WireOp<R>*>(h + im.hb);
+    for (const PassHdr& H : prog.hdrs)
+      for (int i = H.op0; i < H.op0 + H.nops; ++i) {
+        const bool payload = prog.ops[i].kind == F_ROT || prog.ops[i].kind == F_PHASE;
+        w[i] = encode_wire_op<R>(prog.ops[i],
+                                 payload ? prog.coef.data() + 2 * ((size_t)H.coef0 + prog.ops[i].coef) : nullptr);
+      }
+  } else {
+    for (size_t i = 0; i < prog.ops.size(); ++i) {
+      const FOpW e = encode_op(prog.ops[i]);
+      std::memcpy(h + im.hb + i * sizeof(FOpW), &e, sizeof(FOpW));
+    }
   }
   if (!prog.aux.empty()) std::memcpy(h + im.hb + im.ob, prog.aux.data(), prog.aux.size() * sizeof(uint32_t));
   cx<R>* hc = reinterpret_cast<cx<R>*>(h + im.hb + im.ob + im.xb);
@@ -97,7 +108,7 @@ static int launch_fused(qs_ctx* ctx, cx<R>* v, int n, const Config& c, const Pas
   int rc = QS_OK;
   if (prof && (rc = prof_begin(ctx, PROF_FUSED, s))) return rc;
   if (c.wires) {
-    launch_wires<R, RB, TB>(v, tiles, hd, dh, d.O, d.C, d.X, n < K ? 1u << n : 0u, lds, s);
+    launch_wires<R, RB, TB>(v, tiles, hd, dh, (const WireOp<R>*)d.O, d.C, d.X, n < K ? 1u << n : 0u, lds, s);
   } else if (hd.has_dk) {
     hipLaunchKernelGGL((k_fused<R, RB, TB, true, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, d.O,
                        d.C, d.X, tiles);

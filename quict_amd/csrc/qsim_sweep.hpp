@@ -53,7 +53,7 @@ class VarImage {
     }
     auto al = [](uint64_t b) { return (b + 255) & ~255ull; };
     ob = al(nh * sizeof(PassHdr));
-    xb = ob + al(no * sizeof(FOpW));
+    xb = ob + al((no + 1) * sizeof(WireOp<R>));  // (k_jobs fetches one op ahead)
     cb = xb + al(nx * sizeof(uint32_t));
     host.assign(cb + al(nc * sizeof(cx<R>)), 0);
     uint32_t h0 = 0, o0 = 0, x0 = 0, c0 = 0;
@@ -63,11 +63,11 @@ class VarImage {
         PassHdr H = p.hdrs[h];
         for (int i = 0; i < H.nops; ++i) {
           FOp o = p.ops[H.op0 + i];
-          if (o.sym) refs.push_back({o0 + (uint32_t)(H.op0 + i), c0 + (uint32_t)(H.coef0 + o.coef), o.sym - 1, o.sgn,
-                                     o.kind == F_ROT, o.creg});
+          if (o.sym) refs.push_back({o0 + (uint32_t)(H.op0 + i), o.sym - 1, o.sgn, o.kind == F_ROT, o.creg});
           if (o.kind == F_RELAYOUT) o.coef += (int)x0;
-          const FOpW w = encode_wire_op(o);
-          std::memcpy(host.data() + ob + (o0 + (uint64_t)H.op0 + i) * sizeof(FOpW), &w, sizeof(w));
+          const bool payload = o.kind == F_ROT || o.kind == F_PHASE;
+          op<R>(o0 + (uint64_t)H.op0 + i) =
+              encode_wire_op<R>(o, payload ? p.coef.data() + 2 * ((size_t)H.coef0 + o.coef) : nullptr);
         }
         const int nv = d + 1;
         const size_t image = (size_t)nv * 2048 * sizeof(cx<R>);
@@ -79,7 +79,8 @@ class VarImage {
         std::memcpy(host.data() + (h0 + h) * sizeof(PassHdr), &H, sizeof(H));
       }
       if (!p.aux.empty()) std::memcpy(host.data() + xb + (uint64_t)x0 * 4, p.aux.data(), p.aux.size() * 4);
-      for (size_t i = 0; i < p.coef.size() / 2; ++i) put<R>(c0 + i, p.coef[2 * i], p.coef[2 * i + 1]);
+      cx<R>* cf = reinterpret_cast<cx<R>*>(host.data() + cb) + c0;
+      for (size_t i = 0; i < p.coef.size() / 2; ++i) cf[i] = mk<R>((R)p.coef[2 * i], (R)p.coef[2 * i + 1]);
       h0 += (uint32_t)p.hdrs.size(), o0 += (uint32_t)p.ops.size(), x0 += (uint32_t)p.aux.size();
       c0 += (uint32_t)(p.coef.size() / 2);
     }
@@ -88,7 +89,6 @@ class VarImage {
 
   // Payloads of the parameterised ops; at(slot) is the slot's row of the angle table.
   template <typename R, typename At> void bind(const AngleTable& t, const At& at) {
-    FOpW* ops = reinterpret_cast<FOpW*>(host.data() + ob);
     for (const Ref& r : refs) {
       const double* v = &t.v[4 * (size_t)at(r.slot)];
       double p[2];
@@ -96,26 +96,23 @@ class VarImage {
         rot_payload(v[0], v[1], r.sgn, p);
       } else {
         const int pure = phase_payload_sym(v[2], v[3], r.sgn, p);
-        FOpW& w = ops[r.op];
-        w.w[0] = (w.w[0] & ~0xffu) | ((pure == 3 ? WC_PHS : WC_PHR) + r.mask);
+        uint32_t& w0 = op<R>(r.op).w[0];
+        w0 = (w0 & ~0xffu) | ((pure == 3 ? WC_PHS : WC_PHR) + r.mask);
       }
-      put<R>(r.coef, p[0], p[1]);
+      op<R>(r.op).f = mk<R>((R)p[0], (R)p[1]);
     }
   }
 
  private:
   struct Ref {
-    uint32_t op, coef;
+    uint32_t op;
     int slot;
     double sgn;
     bool rot;
     uint32_t mask;
   };
   std::vector<Ref> refs;
-  template <typename R> void put(uint64_t i, double re, double im) {
-    cx<R>* c = reinterpret_cast<cx<R>*>(host.data() + cb);
-    c[i] = mk<R>((R)re, (R)im);
-  }
+  template <typename R> WireOp<R>& op(uint64_t i) { return reinterpret_cast<WireOp<R>*>(host.data() + ob)[i]; }
 };
 
 // Column sums of gradient rows: out[i] = sum over rows of partial[off + row * stride].

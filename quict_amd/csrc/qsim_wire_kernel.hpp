@@ -24,8 +24,8 @@ namespace qs {
 // ---- ops, in place -----------------------------------------------------------------
 
 template <typename R, int NR, int P>
-__device__ __forceinline__ void wo_rot(cx<R> (&a)[NR], const cx<R>* g) {
-  const R t = g[0].re, s = g[0].im;
+__device__ __forceinline__ void wo_rot(cx<R> (&a)[NR], cx<R> ts) {
+  const R t = ts.re, s = ts.im;
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     if (r & (1 << P)) continue;
@@ -209,7 +209,7 @@ __device__ __forceinline__ void wo_measure(const cx<R> (&psi)[NR], const cx<R> (
 // One op on NV vectors (2: psi and lam of a gradient sweep); grad: this wave's column
 // 0 of the tile's gradient row.
 template <typename R, int RB, int TB, int NV, bool HEAVY>
-__device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, const FOpW& e, const cx<R>* __restrict__ C,
+__device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, const WireOp<R>& e, const cx<R>* __restrict__ C,
                                         const cx<R>* __restrict__ G, const uint32_t* __restrict__ X, uint32_t tid,
                                         uint32_t blk, double* grad) {
   static_assert(RB == 4, "opcodes are laid out for four register bits");
@@ -237,7 +237,7 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, cons
   }
 #define QS_4(X) X(0) X(1) X(2) X(3)
 #define QS_16(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15)
-#define QS_ROT(P) case WC_ROT + P: QS_V(wo_rot<R, NR, P>(a[v], g))  break;
+#define QS_ROT(P) case WC_ROT + P: QS_V(wo_rot<R, NR, P>(a[v], e.f))  break;
     QS_4(QS_ROT)
 #define QS_EX(P) case WC_EX + P: QS_V(wo_ex<R, NR, P, -1>(a[v])) break;
     QS_4(QS_EX)
@@ -250,7 +250,7 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, cons
     break;
     QS_16(QS_EXC)
 // lanes whose thread bits fail sit these out: a wave all of whose lanes do skips the op
-#define QS_PH(BASE, MODE, M) case BASE + M: if (tok) QS_V(wo_phase<R, NR, M, MODE>(a[v], g[0])) break;
+#define QS_PH(BASE, MODE, M) case BASE + M: if (tok) QS_V(wo_phase<R, NR, M, MODE>(a[v], e.f)) break;
 #define QS_PHR(M) QS_PH(WC_PHR, 2, M)
     QS_16(QS_PHR)
 #define QS_PHS(M) QS_PH(WC_PHS, 3, M)
@@ -371,10 +371,10 @@ __device__ __forceinline__ void wire_store(const cx<R> (&a)[NV][1 << RB], cx<R>*
 // (NV = 2): per column one entry a wave.
 template <typename R, int RB, int TB, int NV, bool HEAVY>
 __device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, const PassHdr* __restrict__ H,
-                                            const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
+                                            const WireOp<R>* __restrict__ ops, const cx<R>* __restrict__ coef,
                                             const uint32_t* __restrict__ aux, uint32_t tid, uint32_t blk) {
   constexpr int K = RB + TB;
-  const FOpW* P = ops + H->op0;
+  const WireOp<R>* P = ops + H->op0;
   const cx<R>* G = coef + H->coef0;
   // behind the relayout images: diagonal tables (read per lane), the gradient row
   cx<R>* C = reinterpret_cast<cx<R>*>(lds) + (H->uses_lds ? NV << (K - 1) : 0);
@@ -385,10 +385,11 @@ __device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, 
   double* row = reinterpret_cast<double*>(C + H->nstage);
   double* grad = row + (tid >> 6);
   const int nops = H->nops;
+  WireOp<R> e = P[0];
   for (int o = 0; o < nops; ++o) {
-    const FOpW e = P[o];
-    if ((blk & e.w[6]) != e.w[7]) continue;
-    wire_op<R, RB, TB, NV, HEAVY>(a, lds, e, C, G, aux, tid, blk, grad);
+    const WireOp<R> nx = P[o + 1];  // (past the last op: what follows in the program's memory)
+    if ((blk & e.w[6]) == e.w[7]) wire_op<R, RB, TB, NV, HEAVY>(a, lds, e, C, G, aux, tid, blk, grad);
+    e = nx;
   }
   return row;
 }
@@ -397,7 +398,7 @@ __device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, 
 // amplitudes, fewer than a tile has; the rest of the tile is zeros.
 template <typename R, int RB, int TB, bool HEAVY>
 __global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k_wires(
-    cx<R>* __restrict__ v, const PassHdr* __restrict__ H, const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
+    cx<R>* __restrict__ v, const PassHdr* __restrict__ H, const WireOp<R>* __restrict__ ops, const cx<R>* __restrict__ coef,
     const uint32_t* __restrict__ aux, uint32_t nsmall) {
   extern __shared__ __align__(16) char lds_raw[];
   const uint32_t tid = threadIdx.x, blk = blockIdx.x;
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(256, HEAVY || (NV == 2 && sizeof(R) == 8) ? 2 : NV 
   } else {
     wire_load<R, 4, 8, 2>(a, {psi + job.off, lam + job.off}, H, tb, tid, 0);
   }
-  double* row = wire_ops<R, 4, 8, NV, HEAVY>(a, lds_raw, H, reinterpret_cast<const FOpW*>(image + job.ops),
+  double* row = wire_ops<R, 4, 8, NV, HEAVY>(a, lds_raw, H, reinterpret_cast<const WireOp<R>*>(image + job.ops),
                                               reinterpret_cast<const cx<R>*>(image + job.coef),
                                               reinterpret_cast<const uint32_t*>(image + job.aux), tid, blk);
   if (H->sync_store || NV == 2) __syncthreads();

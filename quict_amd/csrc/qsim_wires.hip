@@ -9,7 +9,7 @@
 namespace qs {
 
 template <typename R, int RB, int TB>
-void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const FOpW* ops, const cx<R>* coef,
+void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const WireOp<R>* ops, const cx<R>* coef,
                   const uint32_t* aux, uint32_t nsmall, size_t lds, hipStream_t s) {
   if (hd.has_dk)
     hipLaunchKernelGGL((k_wires<R, RB, TB, true>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef, aux,
@@ -50,7 +50,7 @@ template void launch_jobs<float>(cx<float>*, cx<float>*, const char*, const Wire
                                  hipStream_t);
 
 #define QS_WIRES(R, TB)                                                                                          \
-  template void launch_wires<R, 4, TB>(cx<R>*, uint64_t, const PassHdr&, const PassHdr*, const FOpW*,            \
+  template void launch_wires<R, 4, TB>(cx<R>*, uint64_t, const PassHdr&, const PassHdr*, const WireOp<R>*,       \
                                        const cx<R>*, const uint32_t*, uint32_t, size_t, hipStream_t);            \
   template void wires_lds_attr<R, 4, TB>();
 QS_WIRES(double, 7)

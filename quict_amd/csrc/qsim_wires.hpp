@@ -4,6 +4,8 @@
 #include "qsim_common.hpp"
 #include "qsim_fused_plan.hpp"
 
+#include <cstring>
+
 namespace qs {
 
 // Opcodes of k_wires.  P, C: register positions; M: mask of register positions.
@@ -35,9 +37,20 @@ enum WCode : uint32_t {
 // register pairs (P0 > P1) in the order 10, 20, 21, 30, 31, 32
 static int wire_pair(int p0, int p1) { return p0 * (p0 - 1) / 2 + p1; }
 
-// Device encoding (32 bytes, one scalar load): code | creg << 8 | cregv << 16 |
-// ntt << 24; tpos[0] | tpos[1] << 8; coef; cthr | cthrv << 16; 0; 0; cblk; cblkv
-static FOpW encode_wire_op(const FOp& o) {
+// Device encoding, one cache line: words code | creg << 8 | cregv << 16 | ntt << 24;
+// tpos[0] | tpos[1] << 8; coef; cthr | cthrv << 16; relayout with tile flips; pure;
+// cblk; cblkv; then the payload of a rotation or a phase.  The interpreter loads the
+// next op while it runs one: with the payload elsewhere (a second dependent load) and
+// nothing fetched ahead an op of a 20-qubit pass, one wave a SIMD, took 0.7 us.
+template <typename R> struct WireOp {
+  uint32_t w[8];
+  cx<R> f;
+  uint32_t pad[8 - sizeof(cx<R>) / 4];
+};
+static_assert(sizeof(WireOp<double>) == 64 && sizeof(WireOp<float>) == 64, "WireOp layout");
+
+// f: the op's first coefficient.
+template <typename R> static WireOp<R> encode_wire_op(const FOp& o, const double* f) {
   uint32_t code = WC_END;
   const bool ctl = o.creg != 0 || o.cthr != 0;
   switch (o.kind) {
@@ -84,7 +97,9 @@ static FOpW encode_wire_op(const FOp& o) {
       break;
   }
   const bool diag = o.kind == F_DIAG;
-  FOpW e;
+  WireOp<R> e;
+  std::memset((void*)&e, 0, sizeof(e));
+  if (o.kind == F_ROT || o.kind == F_PHASE) e.f = mk<R>((R)f[0], (R)f[1]);
   e.w[0] = code | (diag ? 0 : o.creg) << 8 | (diag ? 0 : o.cregv) << 16 | (uint32_t)o.ntt << 24;
   e.w[1] = (uint32_t)o.tpos[0] | (uint32_t)o.tpos[1] << 8;
   e.w[2] = (uint32_t)o.coef;
@@ -120,7 +135,7 @@ void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs
 // One pass over the 2^(n-K) tiles of v: header hd, its device copy dh and the
 // program's device arrays; nsmall: amplitudes of a register below a tile, else 0.  The caller checks hipGetLastError().
 template <typename R, int RB, int TB>
-void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const FOpW* ops, const cx<R>* coef,
+void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const WireOp<R>* ops, const cx<R>* coef,
                   const uint32_t* aux, uint32_t nsmall, size_t lds, hipStream_t s);
 // Lets the kernels take their largest LDS allocation (once per process).
 template <typename R, int RB, int TB> void wires_lds_attr();
