@@ -142,6 +142,7 @@ struct PassHdr {
   int32_t nsx;           // flips of the store address that depend on the tile: where tile-number bit
   int32_t sxb[FMAX_SX];  // sxb[i] is 1 ...
   uint64_t sxm[FMAX_SX]; // ... the address is XORed with sxm[i]
+  int32_t aux0, naux;    // its relayout constants in the aux table (planned in wires)
   int32_t ngrad;         // gradient columns of the pass (two-vector sweeps)
 };
 
@@ -1532,6 +1533,7 @@ static void chunk_program(const FusedProgram& prog, int h0, int h1, FusedProgram
   for (PassHdr& h : sub.hdrs) {
     h.op0 -= o0;
     h.coef0 -= c0;
+    h.aux0 -= x0;
   }
   sub.ops.assign(prog.ops.begin() + o0, prog.ops.begin() + o1);
   for (FOp& o : sub.ops)

@@ -76,6 +76,7 @@ class VarImage {
         if (d) cols.insert(cols.end(), p.gcols[h].begin(), p.gcols[h].end());
         H.op0 += (int)o0;
         H.coef0 += (int)c0;
+        H.aux0 += (int)x0;
         std::memcpy(host.data() + (h0 + h) * sizeof(PassHdr), &H, sizeof(H));
       }
       if (!p.aux.empty()) std::memcpy(host.data() + xb + (uint64_t)x0 * 4, p.aux.data(), p.aux.size() * 4);

@@ -1244,6 +1244,8 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
     std::vector<GradCol> cols;
     int rc = schedule_wires(cls, p, c, amp_bytes, al, home, H, prog, cols);
     if (rc) return rc;
+    H.aux0 = a0;
+    H.naux = (int)prog.aux.size() - a0;
     H.ngrad = (int)cols.size();
     prog.gcols.push_back(std::move(cols));
     std::vector<int> wires(K);
