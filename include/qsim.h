@@ -295,8 +295,9 @@ int qs_var_passes(const qs_var* v, int backward);
 void qs_var_destroy(qs_var* v);
 
 /* ---- batched variational circuits (no reference counterpart) ------------- */
-/* Launch shape of the batched QNN kernel (picked by the autotuner):
-   widths <= lds_max_width keep psi and lam in LDS (2 x 2^w amplitudes),
+/* Launch shape of the batched QNN kernel (picked by the autotuner).  complex128
+   batches of qs_qnn_batch run as planned tile passes: the values are checked and the
+   shape is the library's.  Otherwise widths <= lds_max_width keep psi and lam in LDS (2 x 2^w amplitudes),
    wider circuits use a global slot per workgroup; block_threads threads per
    workgroup; blocks_per_cu persistent workgroups per CU; use_graph != 0
    captures the launch in a hipGraph on first use and replays it for every
@@ -309,16 +310,17 @@ typedef struct qs_qnn_config {
   int32_t fuse_qubits; /* rotations of this many qubits (1..3) per pass over a circuit's state; 0 means 1 */
 } qs_qnn_config;
 
-/* Hardware-efficient-ansatz QNN batch, one persistent launch for forward and
-   adjoint backward of every circuit.  Circuit c has width widths[c] (<= 20),
+/* Hardware-efficient-ansatz QNN batch, forward and adjoint backward of every circuit
+   (complex64: one persistent launch; complex128: a few launches, each one tile pass of
+   all circuits, on up to two vectors of 4 GiB that the context keeps).  Circuit c has width widths[c] (<= 20),
    angle-encodes x[c*nfeat + j] with Ry on qubit j mod width, then `layers`
    layers of (Ry(theta), Rz(theta) on every qubit; CX(i, i+1) ladder).  theta is
    shared: theta[(l*2 + g)*max_width + q].  Loss: mean over circuits of
    (<Z_0> - target[c])^2.  Outputs (host): expval[c], loss, grad_theta
    (d loss / d theta), grad_x (per circuit, nfeat; may be NULL).  dtype selects
    complex64 / complex128 amplitudes (reductions in double).  cfg may be NULL.
-   grad_theta is the sum of per-circuit terms taken in circuit order, so it is
-   bit-identical across runs and launch shapes of the same block_threads. */
+   grad_theta is summed in a fixed order: bit-identical across runs and launch
+   shapes of the same block_threads. */
 int qs_qnn_batch(qs_ctx* ctx, int dtype, int ncirc, const int32_t* widths, int nfeat, const double* x,
                  const double* target, int layers, int max_width, const double* theta, double* expval,
                  double* loss, double* grad_theta, double* grad_x, const qs_qnn_config* cfg, void* stream);

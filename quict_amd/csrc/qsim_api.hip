@@ -381,6 +381,7 @@ qs_ctx* qs_ctx_create(int device) {
     delete ctx;
     return nullptr;
   }
+  ctx->qnn = qnn_state_create();
   return ctx;
 }
 
@@ -389,6 +390,7 @@ void qs_ctx_destroy(qs_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipDeviceSynchronize();
   if (ctx->scratch) (void)hipFree(ctx->scratch);
+  qnn_state_destroy(ctx->qnn);
   for (auto& S : ctx->prog_slot) {
     if (S.dev) (void)hipFree(S.dev);
     if (S.host) (void)hipHostFree(S.host);

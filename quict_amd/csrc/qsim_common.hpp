@@ -96,6 +96,9 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 }  // namespace qs
 
 // ---- context -------------------------------------------------------------------
+namespace qs {
+struct QnnState;
+}
 struct qs_ctx {
   int device = 0;
   int tile_log2 = 0;   // 0 = default per dtype
@@ -125,6 +128,7 @@ struct qs_ctx {
   };
   ProgSlot prog_slot[2];
   int prog_next = 0;
+  qs::QnnState* qnn = nullptr;  // batches of variational circuits (qsim_qnn_planned.hip)
   // kernel timing (HIP events recorded on the launch stream around each launch)
   int profile = 0;
   double prof_ms[4] = {0, 0, 0, 0};       // per kernel class, see qs_profile_read

@@ -45,6 +45,13 @@ int pauli_sum_async(qs_ctx* ctx, const void* vec, void* out, int n, int dtype, c
 int inner_async(const void* a, const void* b, int n, int dtype, double* part, double* res, hipStream_t s);
 int inner_partial_blocks();
 
+// qs_qnn_batch in complex128, arguments checked (qsim_qnn_planned.hip), and what a
+// context keeps for it.
+int qnn_planned(qs_ctx* ctx, int ncirc, const int32_t* widths, int nfeat, const double* x, const double* target, int layers,
+                int max_width, const double* theta, double* expval, double* loss, double* grad_theta, double* grad_x);
+QnnState* qnn_state_create();
+void qnn_state_destroy(QnnState* S);
+
 inline size_t amp_bytes(int dtype) { return dtype == QS_C128 ? 16 : 8; }
 
 }  // namespace qs

@@ -1,5 +1,6 @@
 """Batched QNN: many uneven-width parameterised circuits, forward + adjoint
-backward in one persistent, graph-captured launch (qs_qnn_batch).
+backward in one call (qs_qnn_batch): complex128 as planned tile passes over all
+circuits, complex64 in one persistent, graph-captured launch.
 
 The circuit family (angle encoding, hardware-efficient ansatz, <Z_0> readout,
 squared loss) is documented in quict_amd/csrc/qsim_qnn.hip.  ``QNNBatch``
@@ -8,7 +9,8 @@ per-circuit <Z_0>, d loss / d theta and d loss / d x.
 
 ``autotune`` times every launch shape of a small search space on the real
 batch (LDS width limit, workgroup size, workgroups per CU) and caches the
-winner per (dtype, width histogram, layers, features) in a JSON file.
+winner per (dtype, width histogram, layers, features) in a JSON file.  The shape
+matters to complex64; complex128 batches take the library's own.
 """
 import ctypes
 import json
