@@ -295,23 +295,21 @@ int qs_var_passes(const qs_var* v, int backward);
 void qs_var_destroy(qs_var* v);
 
 /* ---- batched variational circuits (no reference counterpart) ------------- */
-/* Launch shape of the batched QNN kernel (picked by the autotuner).  complex128
-   batches of qs_qnn_batch run as planned tile passes: the values are checked and the
-   shape is the library's.  Otherwise widths <= lds_max_width keep psi and lam in LDS (2 x 2^w amplitudes),
-   wider circuits use a global slot per workgroup; block_threads threads per
-   workgroup; blocks_per_cu persistent workgroups per CU; use_graph != 0
-   captures the launch in a hipGraph on first use and replays it for every
-   later batch of the same shape. */
+/* Launch shape of qs_qnn_batch_programs: widths <= lds_max_width keep psi and lam in
+   LDS (2 x 2^w amplitudes), wider circuits use a global slot per workgroup;
+   block_threads threads per workgroup; blocks_per_cu persistent workgroups per CU.
+   qs_qnn_batch checks the values and takes its launch shapes from the widths;
+   fuse_qubits is what the order of rounding of complex64 results depends on. */
 typedef struct qs_qnn_config {
   int32_t lds_max_width;
   int32_t block_threads;
   int32_t blocks_per_cu;
   int32_t use_graph;
-  int32_t fuse_qubits; /* rotations of this many qubits (1..3) per pass over a circuit's state; 0 means 1 */
+  int32_t fuse_qubits; /* 1..3; 0 means 1 */
 } qs_qnn_config;
 
 /* Hardware-efficient-ansatz QNN batch, forward and adjoint backward of every circuit
-   (complex64: one persistent launch; complex128: a few launches, each one tile pass of
+   (complex64: a workgroup a circuit; complex128: a few launches, each one tile pass of
    all circuits, on up to two vectors of 4 GiB that the context keeps).  Circuit c has width widths[c] (<= 20),
    angle-encodes x[c*nfeat + j] with Ry on qubit j mod width, then `layers`
    layers of (Ry(theta), Rz(theta) on every qubit; CX(i, i+1) ladder).  theta is
@@ -319,8 +317,7 @@ typedef struct qs_qnn_config {
    (<Z_0> - target[c])^2.  Outputs (host): expval[c], loss, grad_theta
    (d loss / d theta), grad_x (per circuit, nfeat; may be NULL).  dtype selects
    complex64 / complex128 amplitudes (reductions in double).  cfg may be NULL.
-   grad_theta is summed in a fixed order: bit-identical across runs and launch
-   shapes of the same block_threads. */
+   grad_theta is summed in a fixed order: bit-identical across runs. */
 int qs_qnn_batch(qs_ctx* ctx, int dtype, int ncirc, const int32_t* widths, int nfeat, const double* x,
                  const double* target, int layers, int max_width, const double* theta, double* expval,
                  double* loss, double* grad_theta, double* grad_x, const qs_qnn_config* cfg, void* stream);
@@ -350,8 +347,8 @@ typedef struct qs_qnn_op {
    widths[c] (1..20) and runs ops[prog_offsets[c] .. prog_offsets[c+1]) from
    |0..0>; E_c = <Z_0>, loss = mean over circuits of (E_c - target[c])^2.
    theta (nparams values) is shared by every circuit.  Outputs (host):
-   expval[c], loss, grad_theta (d loss / d theta, summed over circuits in
-   circuit order: bit-identical across runs), grad_x (ncirc x nfeat, d loss /
+   expval[c], loss, grad_theta (d loss / d theta, summed over circuits in a
+   fixed order: bit-identical across runs), grad_x (ncirc x nfeat, d loss /
    d x for the encoding ops; may be NULL).  cfg: lds_max_width, block_threads,
    blocks_per_cu (use_graph and fuse_qubits are ignored: one rotation per
    pass); NULL for defaults.  Replaces no reference function. */

@@ -1,67 +1,46 @@
-// Batched variational circuits: one persistent launch runs forward + adjoint
-// backward for every circuit of a batch (no reference counterpart).  k_qnn takes the
-// complex64 batches; complex128 ones run as planned tile passes (qsim_qnn_planned.hip),
-// 9.3 times as fast, which apply the gates of different qubits in another order: in 32
-// bits that moves the results by 1e-6, and complex64 callers keep the order they have.
+// Batched variational circuits, forward + adjoint backward (no reference counterpart).
 //
 // Circuit c (width w = widths[c], qubit 0 = most significant amplitude bit):
 //   angle encoding   Ry(x[c, j]) on qubit j mod w, j < nfeat
 //   `layers` times   Ry(theta[l,0,q]) Rz(theta[l,1,q]) on every qubit q, then CX(q, q+1), q = 0..w-2
 //   readout          E_c = <Z_0>,  loss_c = (E_c - target_c)^2,  loss = mean_c loss_c
 //
-// Mechanism.  Ry rotations about one axis add, so the encoding is the product
-// state prod_q (cos(phi_q/2)|0> + sin(phi_q/2)|1>) with phi_q = sum_{j = q mod w} x_j:
-// one pass.  A CX ladder is the GF(2)-linear permutation "prefix xor" of the
-// qubit bits, so no amplitude is moved: the kernel keeps, per logical qubit q,
-// the physical index mask c_q = P(e_q) and the parity mask r_q (logical bit q of
-// a physical index p is parity(p & r_q)), and updates both after every ladder.
-// A rotation on logical qubit q then pairs physical p with p ^ c_q.  Every
-// circuit therefore costs w rotation passes per layer forward and w fused
-// (gradient + inverse) passes per layer backward, on a state that lives in LDS
-// (psi and lam, 2 x 2^w amplitudes) when w <= lds_max_width, otherwise in a
-// per-workgroup global slot.  Workgroups pull circuits from an atomic queue
-// ordered by decreasing width, so the widest circuits start first.
+// complex128 batches run as planned tile passes (qsim_qnn_planned.hip), which apply the
+// gates of different qubits in another order.  In 32 bits that would move the results
+// by 1e-6, and complex64 callers keep the order they have: k_qnn takes a circuit per
+// workgroup and a layer's qubits one after another.
 //
-// Fusion depth D (1..3, a launch parameter the autotuner picks): the rotations
-// of D consecutive qubits of a layer run in one pass over groups of 2^D
-// amplitudes (a coset of the span of their D column masks, enumerated by
-// inserting zeros at the masks' elimination pivots), so a layer costs
-// ceil(w / D) passes forward and backward instead of w: D times fewer sweeps
-// of a wide circuit's state through the memory of its slot.
+// k_qnn.  Ry rotations about one axis add, so the encoding is the product state
+// prod_q (cos(phi_q/2)|0> + sin(phi_q/2)|1>) with phi_q = sum_{j = q mod w} x_j: one
+// pass.  A CX ladder is the GF(2)-linear permutation "prefix xor" of the qubit bits, so
+// no amplitude is moved: every wave keeps, in lane q, the physical index mask c_q =
+// P(e_q) and the parity mask r_q (logical bit q of a physical index p is parity(p &
+// r_q)), and updates both after every ladder.  A rotation on logical qubit q then pairs
+// physical p with p ^ c_q.  The rotations of four consecutive qubits run in one sweep
+// over groups of 16 amplitudes (a coset of the span of their masks, enumerated by
+// inserting zeros at the masks' elimination pivots).  psi and lam are in LDS up to 13
+// qubits (128 KiB), above that in a slot of device memory a workgroup.
+//
+// What bounds it: one workgroup's chain of sweeps, barriers and LDS round trips.  192
+// circuits of 5..13 qubits, 4 layers: the kernel 214 us against 690 us with two qubits
+// a sweep, states above 11 qubits in device memory, every thread taking the sines of
+// every angle, and two barriers a qubit for its two derivatives; the call
+// 841 -> 257 us.  1024 circuits of 8..18 qubits, 6 layers: 46.8 -> 18.7 ms.
+// The launch shape follows from the widths (qnn_c64): the caller's is checked only.
 #include "qsim_common.hpp"
 #include "qsim_internal.hpp"
+#include "qsim_qnn.hpp"
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <numeric>
 #include <vector>
 
 namespace qs {
 
-constexpr int QNN_MAX_W = 20;
 constexpr int QNN_MAX_LAYERS = 16;
-
-struct QnnArgs {
-  int fuse;               // rotations of `fuse` qubits per pass (1..3)
-  int ncirc;
-  int nfeat;
-  int layers;
-  int max_width;
-  int lds_max_width;
-  const int32_t* order;    // circuits, widest first
-  const int32_t* widths;
-  const double* x;         // ncirc x nfeat
-  const double* target;    // ncirc
-  const double* theta;     // layers x 2 x max_width
-  double* expval;          // ncirc
-  double* loss_terms;      // ncirc
-  double* grad_circ;       // ncirc x (layers x 2 x max_width): each circuit's term of d(loss)/d(theta)
-  double* grad_x;          // ncirc x nfeat
-  void* slots;             // global per-workgroup state slots (2 x 2^max_width amplitudes each)
-  int* counter;
-  double inv_ncirc;
-};
 
 __device__ __forceinline__ int parity64(uint64_t v) { return __popcll(v) & 1; }
 
@@ -116,294 +95,374 @@ __device__ __forceinline__ void pair_of(uint64_t h, uint64_t m, uint64_t r, uint
   }
 }
 
-// Coset representatives of span{m_0..m_{D-1}}: indices with zeros at the
-// masks' elimination pivots (ascending in piv); returns D.
-template <int D>
-__device__ __forceinline__ void group_pivots(const uint64_t* m, int* piv) {
-  uint64_t red[D];
+// ---- one circuit family, complex64 --------------------------------------------
+struct QnnArgs {
+  int n;                   // circuits of this launch, and the first of them
+  int first;
+  uint32_t alt;            // qubits with the other order of rounding (prod)
+  int nfeat, layers, max_width;
+  const int32_t* widths;   // per circuit, widest first
+  const double* x;         // nfeat each
+  const double* target;
+  const double* trig;      // (layer, qubit): cos, sin of half the Ry angle, of half the Rz angle
+  double* expval;
+  double* loss_terms;
+  double* grad_circ;       // layers x 2 x max_width each: the circuit's term of d(loss)/d(theta)
+  double* grad_x;          // nfeat each
+  cx<float>* slots;        // per workgroup 2 x 2^slot_width amplitudes (states in device memory)
+  int slot_width;
+  int* counter;
+  double inv_ncirc;
+};
+
+// The angles' cosines and sines, once for the batch, and the launches' queues.
+__global__ void k_qnn_trig(const double* __restrict__ theta, int layers, int max_width, double* __restrict__ trig,
+                           int* counters, int ncounters) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < ncounters) counters[i] = 0;
+  if (i >= layers * max_width) return;
+  const int l = i / max_width, q = i % max_width;
+  const double ty = theta[(l * 2 + 0) * max_width + q], tz = theta[(l * 2 + 1) * max_width + q];
+  trig[4 * i] = cos(0.5 * ty);
+  trig[4 * i + 1] = sin(0.5 * ty);
+  trig[4 * i + 2] = cos(0.5 * tz);
+  trig[4 * i + 3] = sin(0.5 * tz);
+}
+
+// Where amplitude p of a state is.  In LDS, sweeps along the lowest bits would put a
+// wave's lanes 128 bytes apart; xor-ing bits 5..9 onto the banks spreads them, and
+// being linear it goes through the masks: at(p ^ q) = at(p) ^ at(q).
+template <bool INLDS> __device__ __forceinline__ uint32_t at(uint32_t p) { return INLDS ? p ^ ((p >> 5) & 31) : p; }
+
+// D qubits' masks: offsets of a group's members and the pivots, ascending, where a
+// group's number gets zeros inserted.
+template <int D, bool INLDS> struct Sweep {
+  uint32_t off[1 << D], r[D];
+  int piv[D];
+  __device__ __forceinline__ Sweep(uint32_t cm, uint32_t rm, int q0) {
+    uint32_t m[D], red[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      m[i] = __builtin_amdgcn_readlane(cm, q0 + i);
+      r[i] = __builtin_amdgcn_readlane(rm, q0 + i);
+      uint32_t v = m[i];
+#pragma unroll
+      for (int j = 0; j < i; ++j)
+        if ((v >> piv[j]) & 1) v ^= red[j];
+      red[i] = v;
+      piv[i] = 31 - __clz(v);
+    }
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+#pragma unroll
+      for (int j = i + 1; j < D; ++j) {
+        const int lo = min(piv[i], piv[j]), hi = max(piv[i], piv[j]);
+        piv[i] = lo, piv[j] = hi;
+      }
+#pragma unroll
+    for (int s = 0; s < 1 << D; ++s) {
+      uint32_t o = 0;
+#pragma unroll
+      for (int i = 0; i < D; ++i)
+        if ((s >> i) & 1) o ^= m[i];
+      off[s] = at<INLDS>(o);
+    }
+  }
+  __device__ __forceinline__ uint32_t base(uint32_t h) const {
+#pragma unroll
+    for (int i = 0; i < D; ++i) h = ((h >> piv[i]) << (piv[i] + 1)) | (h & ((1u << piv[i]) - 1));
+    return h;
+  }
+};
+
+// (By value: a choice between two array elements is a choice between addresses, which
+// puts the array into scratch memory.)
+__device__ __forceinline__ float pick(bool f, float x, float y) { return f ? x : y; }
+__device__ __forceinline__ cx<float> pick(bool f, cx<float> x, cx<float> y) {
+  return mk<float>(pick(f, x.re, y.re), pick(f, x.im, y.im));
+}
+
+// Products with the order of rounding that complex64 results have had: which of two
+// products is rounded and which one the fused multiply-add takes exactly, moves results
+// by 1e-7 and is otherwise the compiler's choice.  prod: u x, with the imaginary part's
+// products the other way round (ALT) on qubits that are not a multiple of fuse_qubits;
+// turn, turn_back: e^{+-i t/2} x; mix: c x + s y.
+template <bool ALT> __device__ __forceinline__ cx<float> prod(cx<float> u, cx<float> x) {
+  return mk<float>(rfma(u.re, x.re, -(u.im * x.im)),
+                   ALT ? rfma(u.im, x.re, u.re * x.im) : rfma(u.re, x.im, u.im * x.re));
+}
+template <int D, int I, bool ALT>
+__device__ __forceinline__ void qnn_rotate(cx<float> (&a)[1 << D], const cx<float>* u, bool flip) {
+#pragma unroll
+  for (int s = 0; s < 1 << D; ++s) {
+    if ((s >> I) & 1) continue;
+    const int s1 = s | (1 << I);
+    const cx<float> x0 = pick(flip, a[s1], a[s]), x1 = pick(flip, a[s], a[s1]);
+    const cx<float> y0 = cfma(prod<ALT>(u[0], x0), u[1], x1), y1 = cfma(prod<ALT>(u[2], x0), u[3], x1);
+    a[s] = pick(flip, y1, y0);
+    a[s1] = pick(flip, y0, y1);
+  }
+}
+template <int D, int I>
+__device__ __forceinline__ void qnn_rotations(cx<float> (&a)[1 << D], const cx<float>* u, const uint32_t* r, uint32_t p,
+                                              uint32_t alt) {
+  if constexpr (I < D) {
+    const bool flip = __popc(p & r[I]) & 1;  // the member with bit I of s set holds logical 0
+    if ((alt >> I) & 1) qnn_rotate<D, I, true>(a, u + 4 * I, flip);
+    else qnn_rotate<D, I, false>(a, u + 4 * I, flip);
+    qnn_rotations<D, I + 1>(a, u, r, p, alt);
+  }
+}
+__device__ __forceinline__ cx<float> turn(float c, float s, cx<float> x) {
+  return mk<float>(rfma(c, x.re, -(s * x.im)), rfma(s, x.re, c * x.im));
+}
+__device__ __forceinline__ cx<float> turn_back(float c, float s, cx<float> x) {
+  return mk<float>(rfma(c, x.re, s * x.im), rfma(c, x.im, -(s * x.re)));
+}
+__device__ __forceinline__ cx<float> mix(float c, cx<float> x, float s, cx<float> y) {
+  return mk<float>(rfma(c, x.re, s * y.re), rfma(c, x.im, s * y.im));
+}
+
+// Forward: U_i = Rz Ry on logical qubit q0 + i, i < D; t: the qubits' rows of the trig table.
+template <int D, bool INLDS>
+__device__ __forceinline__ void qnn_fwd(cx<float>* psi, uint32_t N, uint32_t cm, uint32_t rm, int q0,
+                                        const double* __restrict__ t, uint32_t alt, int tid, int nt) {
+  using R = float;
+  constexpr int G = 1 << D;
+  const Sweep<D, INLDS> S(cm, rm, q0);
+  cx<R> u[4 * D];
 #pragma unroll
   for (int i = 0; i < D; ++i) {
-    uint64_t v = m[i];
-#pragma unroll
-    for (int j = 0; j < i; ++j)
-      if ((v >> piv[j]) & 1) v ^= red[j];
-    red[i] = v;
-    piv[i] = 63 - __clzll(v);
+    const double cy = t[4 * i], sy = t[4 * i + 1], cz = t[4 * i + 2], sz = t[4 * i + 3];
+    // U = Rz(tz) Ry(ty) = [[e^{-i tz/2} cy, -e^{-i tz/2} sy], [e^{i tz/2} sy, e^{i tz/2} cy]]
+    u[4 * i] = mk<R>((R)(cz * cy), (R)(-sz * cy));
+    u[4 * i + 1] = mk<R>((R)(-cz * sy), (R)(sz * sy));
+    u[4 * i + 2] = mk<R>((R)(cz * sy), (R)(sz * sy));
+    u[4 * i + 3] = mk<R>((R)(cz * cy), (R)(sz * cy));
   }
-  // ascending order for zero insertion
-#pragma unroll
-  for (int i = 0; i < D; ++i)
-#pragma unroll
-    for (int j = i + 1; j < D; ++j)
-      if (piv[j] < piv[i]) {
-        const int t = piv[i];
-        piv[i] = piv[j];
-        piv[j] = t;
-      }
-}
-
-__device__ __forceinline__ uint64_t insert0(uint64_t h, int p) {
-  return ((h >> p) << (p + 1)) | (h & ((1ull << p) - 1));
-}
-
-// Forward: apply U_i (2x2, row-major u[4 i .. 4 i + 3]) on logical qubit i of
-// the group, i < D, to every group of psi.
-template <typename R, int D>
-__device__ __forceinline__ void qnn_fwd_group(cx<R>* psi, uint64_t ngroups, const uint64_t* m, const uint64_t* r,
-                                              const cx<R>* u, int tid, int nt) {
-  constexpr int G = 1 << D;
-  int piv[D];
-  group_pivots<D>(m, piv);
-  uint64_t off[G];
-#pragma unroll
-  for (int sI = 0; sI < G; ++sI) {
-    uint64_t o = 0;
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-      if ((sI >> i) & 1) o ^= m[i];
-    off[sI] = o;
-  }
-  for (uint64_t h = tid; h < ngroups; h += nt) {
-    uint64_t base = h;
-#pragma unroll
-    for (int i = 0; i < D; ++i) base = insert0(base, piv[i]);
+#pragma unroll 1
+  for (uint32_t h = tid; h < N >> D; h += nt) {
+    const uint32_t p = S.base(h), g = at<INLDS>(p);
     cx<R> a[G];
 #pragma unroll
-    for (int sI = 0; sI < G; ++sI) a[sI] = ld(psi + (base ^ off[sI]));
+    for (int s = 0; s < G; ++s) a[s] = ld(psi + (g ^ S.off[s]));
+    qnn_rotations<D, 0>(a, u, S.r, p, alt);
 #pragma unroll
-    for (int i = 0; i < D; ++i) {
-      const bool flip = parity64(base & r[i]);  // member with s_i = 1 holds logical 0
-#pragma unroll
-      for (int sI = 0; sI < G; ++sI) {
-        if ((sI >> i) & 1) continue;
-        const int s1 = sI | (1 << i);
-        const cx<R> x0 = flip ? a[s1] : a[sI], x1 = flip ? a[sI] : a[s1];
-        const cx<R> y0 = cfma(mul(u[4 * i], x0), u[4 * i + 1], x1), y1 = cfma(mul(u[4 * i + 2], x0), u[4 * i + 3], x1);
-        a[sI] = flip ? y1 : y0;
-        a[s1] = flip ? y0 : y1;
-      }
-    }
-#pragma unroll
-    for (int sI = 0; sI < G; ++sI) st(psi + (base ^ off[sI]), a[sI]);
+    for (int s = 0; s < G; ++s) st(psi + (g ^ S.off[s]), a[s]);
   }
 }
 
-// Backward over one group of D qubits: for each qubit i the Rz step (gradient
-// gz_i = Im <lam|Z|psi>, then Rz^dagger on both) and the Ry step (gy_i =
-// Im <lam|Y|psi>, then Ry^dagger); different qubits commute.
-template <typename R, int D>
-__device__ __forceinline__ void qnn_bwd_group(cx<R>* psi, cx<R>* lam, uint64_t ngroups, const uint64_t* m,
-                                              const uint64_t* r, const double* cy, const double* sy,
-                                              const double* cz, const double* sz, double* gy, double* gz, int tid,
-                                              int nt) {
+// Backward: for each qubit the Rz step (gradient gz = Im <lam|Z|psi>, v[4 + i]; then
+// Rz^dagger = diag(e^{i tz/2}, e^{-i tz/2}) on both) and the Ry step (gy = Im <lam|Y|psi>
+// with Y psi = (-i a1, i a0), v[i]; then Ry^dagger = [[cy, sy], [-sy, cy]]).  ENC: gy
+// alone, nothing is applied.
+template <int D, bool INLDS, bool ENC>
+__device__ __forceinline__ void qnn_bwd(cx<float>* psi, cx<float>* lam, uint32_t N, uint32_t cm, uint32_t rm, int q0,
+                                        const double* __restrict__ t, double (&v)[8], int tid, int nt) {
+  using R = float;
   constexpr int G = 1 << D;
-  int piv[D];
-  group_pivots<D>(m, piv);
-  uint64_t off[G];
-#pragma unroll
-  for (int sI = 0; sI < G; ++sI) {
-    uint64_t o = 0;
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-      if ((sI >> i) & 1) o ^= m[i];
-    off[sI] = o;
-  }
-  for (uint64_t h = tid; h < ngroups; h += nt) {
-    uint64_t base = h;
-#pragma unroll
-    for (int i = 0; i < D; ++i) base = insert0(base, piv[i]);
+  const Sweep<D, INLDS> S(cm, rm, q0);
+#pragma unroll 1
+  for (uint32_t h = tid; h < N >> D; h += nt) {
+    const uint32_t p = S.base(h), g = at<INLDS>(p);
     cx<R> a[G], b[G];
 #pragma unroll
-    for (int sI = 0; sI < G; ++sI) {
-      a[sI] = ld(psi + (base ^ off[sI]));
-      b[sI] = ld(lam + (base ^ off[sI]));
+    for (int s = 0; s < G; ++s) {
+      a[s] = ld(psi + (g ^ S.off[s]));
+      b[s] = ld(lam + (g ^ S.off[s]));
     }
 #pragma unroll
     for (int i = 0; i < D; ++i) {
-      const bool flip = parity64(base & r[i]);
-      const cx<R> ep = mk<R>((R)cz[i], (R)sz[i]), em = mk<R>((R)cz[i], (R)-sz[i]);
+      const bool flip = __popc(p & S.r[i]) & 1;
+      const R cy = ENC ? (R)0 : (R)t[4 * i], sy = ENC ? (R)0 : (R)t[4 * i + 1];
+      const R cz = ENC ? (R)0 : (R)t[4 * i + 2], sz = ENC ? (R)0 : (R)t[4 * i + 3];
 #pragma unroll
-      for (int sI = 0; sI < G; ++sI) {
-        if ((sI >> i) & 1) continue;
-        const int s1 = sI | (1 << i);
-        const int j0 = flip ? s1 : sI, j1 = flip ? sI : s1;  // logical 0 / 1 members
-        cx<R> a0 = a[j0], a1 = a[j1], b0 = b[j0], b1 = b[j1];
-        gz[i] += ((double)b0.re * a0.im - (double)b0.im * a0.re) - ((double)b1.re * a1.im - (double)b1.im * a1.re);
-        a0 = mul(ep, a0);
-        b0 = mul(ep, b0);
-        a1 = mul(em, a1);
-        b1 = mul(em, b1);
-        gy[i] += -((double)b0.re * a1.re + (double)b0.im * a1.im) + ((double)b1.re * a0.re + (double)b1.im * a0.im);
-        const R c = (R)cy[i], sn = (R)sy[i];
-        a[j0] = mk<R>(c * a0.re + sn * a1.re, c * a0.im + sn * a1.im);
-        a[j1] = mk<R>(-sn * a0.re + c * a1.re, -sn * a0.im + c * a1.im);
-        b[j0] = mk<R>(c * b0.re + sn * b1.re, c * b0.im + sn * b1.im);
-        b[j1] = mk<R>(-sn * b0.re + c * b1.re, -sn * b0.im + c * b1.im);
+      for (int s = 0; s < G; ++s) {
+        if ((s >> i) & 1) continue;
+        const int s1 = s | (1 << i);
+        cx<R> a0 = pick(flip, a[s1], a[s]), a1 = pick(flip, a[s], a[s1]);  // logical 0 / 1
+        cx<R> b0 = pick(flip, b[s1], b[s]), b1 = pick(flip, b[s], b[s1]);
+        if (!ENC) {
+          v[4 + i] +=
+              ((double)b0.re * a0.im - (double)b0.im * a0.re) - ((double)b1.re * a1.im - (double)b1.im * a1.re);
+          a0 = turn(cz, sz, a0);
+          b0 = turn(cz, sz, b0);
+          a1 = turn_back(cz, sz, a1);
+          b1 = turn_back(cz, sz, b1);
+        }
+        v[i] += -((double)b0.re * a1.re + (double)b0.im * a1.im) + ((double)b1.re * a0.re + (double)b1.im * a0.im);
+        if (!ENC) {
+          const cx<R> c0 = mix(cy, a0, sy, a1), c1 = mix(cy, a1, -sy, a0);
+          const cx<R> d0 = mix(cy, b0, sy, b1), d1 = mix(cy, b1, -sy, b0);
+          a[s] = pick(flip, c1, c0);
+          a[s1] = pick(flip, c0, c1);
+          b[s] = pick(flip, d1, d0);
+          b[s1] = pick(flip, d0, d1);
+        }
       }
     }
+    if (!ENC) {
 #pragma unroll
-    for (int sI = 0; sI < G; ++sI) {
-      st(psi + (base ^ off[sI]), a[sI]);
-      st(lam + (base ^ off[sI]), b[sI]);
+      for (int s = 0; s < G; ++s) {
+        st(psi + (g ^ S.off[s]), a[s]);
+        st(lam + (g ^ S.off[s]), b[s]);
+      }
     }
   }
 }
 
-template <typename R>
-__global__ __launch_bounds__(1024) void k_qnn(QnnArgs A) {
-  extern __shared__ __align__(16) char lds_raw[];
-  __shared__ double red[64];
-  __shared__ uint64_t cm[QNN_MAX_W], rm[QNN_MAX_W];
-  __shared__ double gacc[QNN_MAX_LAYERS * 2 * QNN_MAX_W];
-  __shared__ double enc_c[QNN_MAX_W], enc_s[QNN_MAX_W];
-  __shared__ int cur;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  cx<R>* slot_psi = reinterpret_cast<cx<R>*>(A.slots) + (uint64_t)blockIdx.x * 2 * (1ull << A.max_width);
-  cx<R>* slot_lam = slot_psi + (1ull << A.max_width);
+// The wave's sums of eight values, sum k in the lanes 8 k .. 8 k + 7: halves are
+// exchanged first, so ten exchanges instead of 48.
+__device__ __forceinline__ double wave_sums(double (&v)[8], int lane) {
+#pragma unroll
+  for (int o = 32, n = 4; n >= 1; o >>= 1, n >>= 1) {
+    const bool hi = lane & o;
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const double keep = hi ? v[i + n] : v[i], send = hi ? v[i] : v[i + n];
+      v[i] = keep + __shfl_xor(send, o, 64);
+    }
+  }
+  double s = v[0];
+  s += __shfl_xor(s, 4, 64);
+  s += __shfl_xor(s, 2, 64);
+  s += __shfl_xor(s, 1, 64);
+  return s;
+}
 
+template <int NT, bool INLDS>
+__global__ __launch_bounds__(NT) void k_qnn(QnnArgs A) {
+  using R = float;
+  constexpr int NW = NT / 64;
+  extern __shared__ __align__(16) char lds_raw[];
+  __shared__ double red[2][8][NW];  // two buffers in turn: one barrier a sweep covers both uses
+  __shared__ double enc[QNN_MAX_W][2];
+  __shared__ int cur;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int MW = A.max_width, nth = A.layers * 2 * MW;
   for (;;) {
     if (tid == 0) cur = atomicAdd(A.counter, 1);
     __syncthreads();
-    const int k = cur;
+    const int k = __builtin_amdgcn_readfirstlane(cur);
     __syncthreads();
-    if (k >= A.ncirc) break;
-    const int c = A.order[k];
-    const int w = A.widths[c];
-    const uint64_t N = 1ull << w, half = N >> 1;
-    cx<R>* psi;
-    cx<R>* lam;
-    if (w <= A.lds_max_width) {
+    if (k >= A.n) break;
+    const int c = A.first + k;
+    const int w = __builtin_amdgcn_readfirstlane(A.widths[c]);
+    const uint32_t N = 1u << w;
+    cx<R>*psi, *lam;
+    if constexpr (INLDS) {
       psi = reinterpret_cast<cx<R>*>(lds_raw);
       lam = psi + N;
     } else {
-      psi = slot_psi;
-      lam = slot_lam;
+      psi = A.slots + ((uint64_t)blockIdx.x << (A.slot_width + 1));
+      lam = psi + (1u << A.slot_width);
     }
-    const double* th = A.theta;
-    const int MW = A.max_width;
     // encoding angles and product state
-    for (int i = tid; i < 2 * A.layers * MW; i += nt) gacc[i] = 0;
     if (tid < w) {
-      cm[tid] = 1ull << (w - 1 - tid);
-      rm[tid] = 1ull << (w - 1 - tid);
       double phi = 0;
       for (int j = tid; j < A.nfeat; j += w) phi += A.x[(uint64_t)c * A.nfeat + j];
-      enc_c[tid] = cos(0.5 * phi);
-      enc_s[tid] = sin(0.5 * phi);
+      enc[tid][0] = cos(0.5 * phi);
+      enc[tid][1] = sin(0.5 * phi);
     }
+    double* grow = A.grad_circ + (uint64_t)c * nth;
+    for (int i = tid; i < nth; i += NT)
+      if (i % MW >= w) grow[i] = 0.0;
     __syncthreads();
-    for (uint64_t i = tid; i < N; i += nt) {
+    for (uint32_t i = tid; i < N; i += NT) {
       double re = 1;
-      for (int q = 0; q < w; ++q) re *= ((i >> (w - 1 - q)) & 1) ? enc_s[q] : enc_c[q];
-      st(psi + i, mk<R>((R)re, (R)0));
+      for (int q = 0; q < w; ++q) re *= enc[q][(i >> (w - 1 - q)) & 1];
+      st(psi + at<INLDS>(i), mk<R>((R)re, (R)0));
     }
+    uint32_t cm = lane < w ? 1u << (w - 1 - lane) : 0, rm = cm;
     __syncthreads();
-    // forward
     for (int l = 0; l < A.layers; ++l) {
-      for (int q0 = 0; q0 < w; q0 += A.fuse) {
-        const int d = min(A.fuse, w - q0);
-        uint64_t m[3], r[3];
-        cx<R> u[12];
-        for (int i = 0; i < d; ++i) {
-          const int q = q0 + i;
-          const double ty = th[(l * 2 + 0) * MW + q], tz = th[(l * 2 + 1) * MW + q];
-          const double cy = cos(0.5 * ty), sy = sin(0.5 * ty), cz = cos(0.5 * tz), sz = sin(0.5 * tz);
-          // U = Rz(tz) Ry(ty) = [[e^{-i tz/2} cy, -e^{-i tz/2} sy], [e^{i tz/2} sy, e^{i tz/2} cy]]
-          u[4 * i] = mk<R>((R)(cz * cy), (R)(-sz * cy));
-          u[4 * i + 1] = mk<R>((R)(-cz * sy), (R)(sz * sy));
-          u[4 * i + 2] = mk<R>((R)(cz * sy), (R)(sz * sy));
-          u[4 * i + 3] = mk<R>((R)(cz * cy), (R)(sz * cy));
-          m[i] = cm[q];
-          r[i] = rm[q];
+      for (int q0 = 0; q0 < w; q0 += 4) {
+        const double* t = A.trig + 4 * (l * MW + q0);
+        const uint32_t alt = A.alt >> q0;
+        switch (min(4, w - q0)) {
+          case 1: qnn_fwd<1, INLDS>(psi, N, cm, rm, q0, t, alt, tid, NT); break;
+          case 2: qnn_fwd<2, INLDS>(psi, N, cm, rm, q0, t, alt, tid, NT); break;
+          case 3: qnn_fwd<3, INLDS>(psi, N, cm, rm, q0, t, alt, tid, NT); break;
+          default: qnn_fwd<4, INLDS>(psi, N, cm, rm, q0, t, alt, tid, NT);
         }
-        if (d == 1) qnn_fwd_group<R, 1>(psi, N >> 1, m, r, u, tid, nt);
-        else if (d == 2) qnn_fwd_group<R, 2>(psi, N >> 2, m, r, u, tid, nt);
-        else qnn_fwd_group<R, 3>(psi, N >> 3, m, r, u, tid, nt);
         __syncthreads();
       }
-      // CX ladder: r'_k = r_0 ^ .. ^ r_k ; c'_q = c_q ^ c_{q+1}
-      if (tid == 0) {
-        for (int q = 1; q < w; ++q) rm[q] ^= rm[q - 1];
-        for (int q = 0; q + 1 < w; ++q) cm[q] ^= cm[q + 1];
+      // CX ladder: r'_q = r_0 ^ .. ^ r_q, c'_q = c_q ^ c_{q+1}
+#pragma unroll
+      for (int o = 1; o < 32; o <<= 1) {
+        const uint32_t v = __shfl_up(rm, o, 64);
+        if (lane >= o) rm ^= v;
       }
-      __syncthreads();
+      if (lane >= w) rm = 0;
+      cm ^= __shfl_down(cm, 1, 64);
     }
     // E = <Z_0>, lam = Z_0 psi
     double e = 0;
     {
-      const uint64_t r0 = rm[0];
-      for (uint64_t i = tid; i < N; i += nt) {
-        const cx<R> a = ld(psi + i);
+      const uint32_t r0 = __builtin_amdgcn_readlane(rm, 0);
+      for (uint32_t i = tid; i < N; i += NT) {
+        const cx<R> a = ld(psi + at<INLDS>(i));
         const double p = (double)a.re * a.re + (double)a.im * a.im;
-        const bool one = parity64(i & r0);
+        const bool one = __popc(i & r0) & 1;
         e += one ? -p : p;
-        st(lam + i, one ? mk<R>(-a.re, -a.im) : a);
+        st(lam + at<INLDS>(i), one ? mk<R>(-a.re, -a.im) : a);
       }
     }
-    e = block_reduce<R>(e, red);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+    if (lane == 0) red[0][0][wave] = e;
+    __syncthreads();
+    e = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) e += red[0][0][i];
     const double tgt = A.target[c];
     const double dl = 2.0 * (e - tgt) * A.inv_ncirc;  // d(mean loss)/dE_c
-    // backward
-    for (int l = A.layers - 1; l >= 0; --l) {
-      if (tid == 0) {
-        for (int q = w - 1; q >= 1; --q) rm[q] ^= rm[q - 1];
-        for (int q = w - 2; q >= 0; --q) cm[q] ^= cm[q + 1];
-      }
-      __syncthreads();
-      for (int q0 = 0; q0 < w; q0 += A.fuse) {
-        const int d = min(A.fuse, w - q0);
-        uint64_t m[3], r[3];
-        double cy[3], sy[3], cz[3], sz[3], gy[3] = {0, 0, 0}, gz[3] = {0, 0, 0};
-        for (int i = 0; i < d; ++i) {
-          const int q = q0 + i;
-          const double ty = th[(l * 2 + 0) * MW + q], tz = th[(l * 2 + 1) * MW + q];
-          cy[i] = cos(0.5 * ty);
-          sy[i] = sin(0.5 * ty);
-          cz[i] = cos(0.5 * tz);
-          sz[i] = sin(0.5 * tz);
-          m[i] = cm[q];
-          r[i] = rm[q];
-        }
-        // per qubit: gz = Im <lam|Z|psi>, Rz^dagger = diag(e^{i tz/2}, e^{-i tz/2}) on both,
-        // gy = Im <lam|Y|psi> (Y psi = (-i a1, i a0)), Ry^dagger = [[cy, sy], [-sy, cy]] on both
-        if (d == 1) qnn_bwd_group<R, 1>(psi, lam, N >> 1, m, r, cy, sy, cz, sz, gy, gz, tid, nt);
-        else if (d == 2) qnn_bwd_group<R, 2>(psi, lam, N >> 2, m, r, cy, sy, cz, sz, gy, gz, tid, nt);
-        else qnn_bwd_group<R, 3>(psi, lam, N >> 3, m, r, cy, sy, cz, sz, gy, gz, tid, nt);
-        for (int i = 0; i < d; ++i) {
-          block_reduce2<R>(gz[i], gy[i], red);
-          if (tid == 0) {
-            gacc[(l * 2 + 0) * MW + q0 + i] += gy[i];
-            gacc[(l * 2 + 1) * MW + q0 + i] += gz[i];
-          }
-        }
-        __syncthreads();
-      }
-    }
-    // encoding gradient: dE/dphi_q = Im <lam| Y_q |psi> (identity map again)
-    for (int q = 0; q < w; ++q) {
-      const uint64_t m = 1ull << (w - 1 - q);
-      double gy = 0, dummy = 0;
-      for (uint64_t h = tid; h < half; h += nt) {
-        uint64_t p0, p1;
-        pair_of(h, m, m, p0, p1);
-        const cx<R> a0 = ld(psi + p0), a1 = ld(psi + p1), b0 = ld(lam + p0), b1 = ld(lam + p1);
-        gy += -((double)b0.re * a1.re + (double)b0.im * a1.im) + ((double)b1.re * a0.re + (double)b1.im * a0.im);
-      }
-      block_reduce2<R>(gy, dummy, red);
-      if (tid == 0)
-        for (int j = q; j < A.nfeat; j += w) A.grad_x[(uint64_t)c * A.nfeat + j] = dl * gy;
-      __syncthreads();
-    }
     if (tid == 0) {
       A.expval[c] = e;
       A.loss_terms[c] = (e - tgt) * (e - tgt);
     }
-    // this circuit's row of the per-circuit gradient terms (summed in circuit
-    // order by k_qnn_reduce: the result does not depend on which workgroup ran
-    // which circuit)
-    for (int i = tid; i < A.layers * 2 * MW; i += nt) {
-      const int q = i % MW;
-      A.grad_circ[(uint64_t)c * A.layers * 2 * MW + i] = q < w ? dl * gacc[i] : 0.0;
+    int buf = 1;
+    // backward; l = -1: the encoding, d E / d phi_q = Im <lam|Y_q|psi> with the identity map again
+    for (int l = A.layers - 1; l >= -1; --l) {
+      if (l >= 0) {
+        const uint32_t v = __shfl_up(rm, 1, 64);
+        if (lane >= 1 && lane < w) rm ^= v;
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) cm ^= __shfl_down(cm, o, 64);
+      }
+      for (int q0 = 0; q0 < w; q0 += 4) {
+        const int d = min(4, w - q0);
+        const double* t = A.trig + 4 * (max(l, 0) * MW + q0);
+        double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (l >= 0) {
+          switch (d) {
+            case 1: qnn_bwd<1, INLDS, false>(psi, lam, N, cm, rm, q0, t, v, tid, NT); break;
+            case 2: qnn_bwd<2, INLDS, false>(psi, lam, N, cm, rm, q0, t, v, tid, NT); break;
+            case 3: qnn_bwd<3, INLDS, false>(psi, lam, N, cm, rm, q0, t, v, tid, NT); break;
+            default: qnn_bwd<4, INLDS, false>(psi, lam, N, cm, rm, q0, t, v, tid, NT);
+          }
+        } else {
+          switch (d) {
+            case 1: qnn_bwd<1, INLDS, true>(psi, lam, N, cm, rm, q0, t, v, tid, NT); break;
+            case 2: qnn_bwd<2, INLDS, true>(psi, lam, N, cm, rm, q0, t, v, tid, NT); break;
+            case 3: qnn_bwd<3, INLDS, true>(psi, lam, N, cm, rm, q0, t, v, tid, NT); break;
+            default: qnn_bwd<4, INLDS, true>(psi, lam, N, cm, rm, q0, t, v, tid, NT);
+          }
+        }
+        const double s = wave_sums(v, lane);
+        if ((lane & 7) == 0) red[buf][lane >> 3][wave] = s;
+        __syncthreads();
+        if (tid < 8 && (tid & 3) < d) {
+          double g = 0;
+#pragma unroll
+          for (int i = 0; i < NW; ++i) g += red[buf][tid][i];
+          const int q = q0 + (tid & 3);
+          if (l >= 0) grow[(l * 2 + (tid >> 2)) * MW + q] = dl * g;
+          else if (tid < 4)
+            for (int j = q; j < A.nfeat; j += w) A.grad_x[(uint64_t)c * A.nfeat + j] = dl * g;
+        }
+        buf ^= 1;
+      }
     }
     __syncthreads();
   }
@@ -413,13 +472,54 @@ __global__ void k_qnn_clear(int* counter) {
   if (threadIdx.x == 0) *counter = 0;
 }
 
-// grad_theta[i] = sum over circuits c = 0, 1, ... (in that order) of grad_circ[c][i]
-__global__ void k_qnn_reduce(const double* __restrict__ grad_circ, int ncirc, int nth, double* __restrict__ g) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nth) return;
+// grad_theta[i] = sum over circuits of grad_circ[c][i]: 32 columns a block, eight
+// threads a column, in a fixed order.  (One thread a column: 43 us for 192 circuits.)
+__global__ __launch_bounds__(256) void k_qnn_reduce(const double* __restrict__ grad_circ, int ncirc, int nth,
+                                                    double* __restrict__ g) {
+  __shared__ double red[8][32];
+  const int q = threadIdx.x & 31, r = threadIdx.x >> 5, i = blockIdx.x * 32 + q;
   double s = 0;
-  for (int c = 0; c < ncirc; ++c) s += grad_circ[(uint64_t)c * nth + i];
-  g[i] = s;
+  if (i < nth)
+    for (int c = r; c < ncirc; c += 8) s += grad_circ[(uint64_t)c * nth + i];
+  red[r][q] = s;
+  __syncthreads();
+  if (r == 0 && i < nth)
+    g[i] = ((red[0][q] + red[1][q]) + (red[2][q] + red[3][q])) + ((red[4][q] + red[5][q]) + (red[6][q] + red[7][q]));
+}
+
+QnnState* qnn_state_create() { return new QnnState(); }
+void qnn_state_destroy(QnnState* S) {
+  if (!S) return;
+  if (S->dev) (void)hipFree(S->dev);
+  if (S->host) (void)hipHostFree(S->host);
+  if (S->stream) (void)hipStreamDestroy(S->stream);
+  delete S;
+}
+int QnnState::open(int device) {
+  QS_CHECK_HIP(hipSetDevice(device));
+  if (!stream) QS_CHECK_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+  return QS_OK;
+}
+int QnnState::room(uint64_t dev_need, uint64_t host_need) {
+  if (dev_bytes < dev_need) {
+    if (dev) QS_CHECK_HIP(hipFree(dev));
+    dev = nullptr, dev_bytes = 0;
+    const hipError_t err = hipMalloc((void**)&dev, dev_need);
+    if (err != hipSuccess) {
+      (void)hipGetLastError();
+      dev = nullptr;
+      set_error(std::string("batch of variational circuits: ") + hipGetErrorString(err));
+      return QS_ERR_UNSUPPORTED;
+    }
+    dev_bytes = dev_need;
+  }
+  if (host_bytes < host_need) {
+    if (host) QS_CHECK_HIP(hipHostFree(host));
+    host = nullptr, host_bytes = 0;
+    QS_CHECK_HIP(hipHostMalloc((void**)&host, host_need, hipHostMallocDefault));
+    host_bytes = host_need;
+  }
+  return QS_OK;
 }
 
 static int qnn_check(const qs_qnn_config* cfg, int dtype) {
@@ -434,154 +534,106 @@ static int qnn_check(const qs_qnn_config* cfg, int dtype) {
   return QS_OK;
 }
 
-struct QnnPlan {
-  int dtype = -1, ncirc = 0, nfeat = 0, layers = 0, max_width = 0, lds_max_width = 0, threads = 0, blocks = 0,
-      fuse = 0;
-  bool slots = false;  // the buffer holds the global state slots (some circuit wider than the LDS limit)
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
-  hipStream_t stream = nullptr;
-  void* buf = nullptr;
-  uint64_t buf_bytes = 0;
-};
-
-static QnnPlan g_plan;  // one cached plan (graph + buffers) per process
-
-template <typename R>
-static int qnn_t(qs_ctx* ctx, int dtype, int ncirc, const int32_t* widths, int nfeat, const double* x,
-                 const double* target, int layers, int max_width, const double* theta, double* expval, double* loss,
-                 double* grad_theta, double* grad_x, const qs_qnn_config* cfg, hipStream_t user_stream) {
-  int lds_w = cfg ? cfg->lds_max_width : 11;
-  int threads = cfg ? cfg->block_threads : 256;
-  int per_cu = cfg ? cfg->blocks_per_cu : 2;
-  const int use_graph = cfg ? cfg->use_graph : 1;
-  const int fuse = (cfg && cfg->fuse_qubits) ? cfg->fuse_qubits : 1;
-  const size_t lds_bytes = lds_w > 0 ? (size_t)2 * (1ull << lds_w) * sizeof(cx<R>) : 0;
-  int dev = ctx->device, cus = 0;
-  QS_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int blocks = std::max(1, cus * per_cu);
-  // device buffers: order, widths, x, target, theta, expval, loss, grad_theta, grad_x, counter,
-  // per-circuit gradient terms, slots
-  // global state slots only when some circuit is wider than the LDS limit
-  int wmax = 0;
-  for (int i = 0; i < ncirc; ++i) wmax = std::max(wmax, (int)widths[i]);
-  const uint64_t slot_bytes = wmax > lds_w ? (uint64_t)blocks * 2 * (1ull << max_width) * sizeof(cx<R>) : 0;
-  auto al = [](uint64_t b) { return (b + 255) & ~255ull; };
-  const uint64_t nth = (uint64_t)layers * 2 * max_width;
-  const uint64_t sz_i = al(ncirc * sizeof(int32_t)), sz_x = al((uint64_t)ncirc * nfeat * sizeof(double)),
-                 sz_c = al(ncirc * sizeof(double)), sz_t = al(nth * sizeof(double));
-  const uint64_t sz_gc = al((uint64_t)ncirc * nth * sizeof(double));
-  const uint64_t total = 2 * sz_i + 2 * sz_x + 3 * sz_c + 2 * sz_t + 256 + sz_gc + slot_bytes;
-  QnnPlan& P = g_plan;
-  const bool same = P.exec && P.dtype == dtype && P.ncirc == ncirc && P.nfeat == nfeat && P.layers == layers &&
-                    P.max_width == max_width && P.lds_max_width == lds_w && P.threads == threads &&
-                    P.blocks == blocks && P.fuse == fuse && P.slots == (slot_bytes != 0);
-  if (!same) {
-    if (P.exec) (void)hipGraphExecDestroy(P.exec);
-    if (P.graph) (void)hipGraphDestroy(P.graph);
-    P.exec = nullptr;
-    P.graph = nullptr;
-    if (!P.stream) QS_CHECK_HIP(hipStreamCreateWithFlags(&P.stream, hipStreamNonBlocking));
-    if (P.buf_bytes < total) {
-      if (P.buf) QS_CHECK_HIP(hipFree(P.buf));
-      P.buf = nullptr;
-      QS_CHECK_HIP(hipMalloc(&P.buf, total));
-      P.buf_bytes = total;
-    }
-  }
-  char* b = (char*)P.buf;
-  int32_t* d_order = (int32_t*)b;
-  int32_t* d_w = (int32_t*)(b + sz_i);
-  double* d_x = (double*)(b + 2 * sz_i);
-  double* d_gx = (double*)(b + 2 * sz_i + sz_x);
-  double* d_t = (double*)(b + 2 * sz_i + 2 * sz_x);
-  double* d_e = (double*)(b + 2 * sz_i + 2 * sz_x + sz_c);
-  double* d_l = (double*)(b + 2 * sz_i + 2 * sz_x + 2 * sz_c);
-  double* d_th = (double*)(b + 2 * sz_i + 2 * sz_x + 3 * sz_c);
-  double* d_gth = (double*)(b + 2 * sz_i + 2 * sz_x + 3 * sz_c + sz_t);
-  int* d_cnt = (int*)(b + 2 * sz_i + 2 * sz_x + 3 * sz_c + 2 * sz_t);
-  double* d_gc = (double*)(b + 2 * sz_i + 2 * sz_x + 3 * sz_c + 2 * sz_t + 256);
-  void* d_slots = b + 2 * sz_i + 2 * sz_x + 3 * sz_c + 2 * sz_t + 256 + sz_gc;
-
-  // widest first
+// Launch shapes, one launch each, the widest circuits first.  A sweep has 2^(w-4) groups
+// and takes 240 registers a thread, eight waves a CU: 512 threads from 14 qubits on (a
+// workgroup a CU, each with its slot) and for 12 and 13 (a workgroup's LDS), 128 up to 11
+// (32 KiB: four workgroups a CU).  Up to one circuit a CU the last two go as one
+// launch: they run side by side, and only the widest counts.
+static int qnn_c64(qs_ctx* ctx, int fuse, int ncirc, const int32_t* widths, int nfeat, const double* x, const double* target,
+                   int layers, int max_width, const double* theta, double* expval, double* loss, double* grad_theta,
+                   double* grad_x) {
+  QnnState* S = ctx->qnn;
+  std::lock_guard<std::mutex> lock(S->mu);
+  int rc = S->open(ctx->device);
+  if (rc) return rc;
   std::vector<int32_t> order(ncirc);
   std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int a, int c2) { return widths[a] > widths[c2]; });
-  hipStream_t s = P.stream;
-  QS_CHECK_HIP(hipMemcpyAsync(d_order, order.data(), ncirc * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  QS_CHECK_HIP(hipMemcpyAsync(d_w, widths, ncirc * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  QS_CHECK_HIP(hipMemcpyAsync(d_x, x, (uint64_t)ncirc * nfeat * sizeof(double), hipMemcpyHostToDevice, s));
-  QS_CHECK_HIP(hipMemcpyAsync(d_t, target, ncirc * sizeof(double), hipMemcpyHostToDevice, s));
-  QS_CHECK_HIP(hipMemcpyAsync(d_th, theta, nth * sizeof(double), hipMemcpyHostToDevice, s));
-
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return widths[a] > widths[b]; });
+  auto wider = [&](int w) {  // circuits of more than w qubits
+    return (int)(std::partition_point(order.begin(), order.end(), [&](int c) { return widths[c] > w; }) - order.begin());
+  };
+  const int cus = ctx->num_cus;
+  int end[3] = {wider(13), wider(11), ncirc};
+  if (ncirc - end[0] <= cus && end[1] > end[0]) end[1] = ncirc;
+  const int wmax = widths[order[0]];
+  auto al = [](uint64_t b) { return (b + 255) & ~255ull; };
+  const uint64_t n = ncirc, nth = (uint64_t)layers * 2 * max_width, nx = n * nfeat;
+  // up: theta, x, target, widths; down: <Z_0>, loss terms, grad_theta, grad_x
+  const uint64_t x_off = al(nth * sizeof(double)), t_off = al(x_off + nx * sizeof(double)),
+                 w_off = al(t_off + n * sizeof(double)), up = w_off + n * sizeof(int32_t), res_off = al(up),
+                 nres = 2 * n + nth + nx, trig_off = al(res_off + nres * sizeof(double)),
+                 cnt_off = al(trig_off + 2 * nth * sizeof(double)), gc_off = cnt_off + 256,
+                 slot_off = al(gc_off + n * nth * sizeof(double));
+  int slots = std::min(end[0], cus);
+  for (;;) {  // fewer states in device memory at a time if it has not so much to give
+    rc = S->room(slot_off + ((uint64_t)slots << (wmax + 1)) * sizeof(cx<float>), res_off + nres * sizeof(double));
+    if (rc != QS_ERR_UNSUPPORTED || slots <= 1) break;
+    slots /= 2;
+  }
+  if (rc) return rc == QS_ERR_UNSUPPORTED ? QS_ERR_DEVICE : rc;
+  std::memcpy(S->host, theta, nth * sizeof(double));
+  double* hx = (double*)(S->host + x_off);
+  double* ht = (double*)(S->host + t_off);
+  int32_t* hw = (int32_t*)(S->host + w_off);
+  for (int i = 0; i < ncirc; ++i) {
+    if (nfeat) std::memcpy(hx + (uint64_t)i * nfeat, x + (uint64_t)order[i] * nfeat, nfeat * sizeof(double));
+    ht[i] = target[order[i]];
+    hw[i] = widths[order[i]];
+  }
+  hipStream_t s = S->stream;
+  char* d = S->dev;
+  QS_CHECK_HIP(hipMemcpyAsync(d, S->host, up, hipMemcpyHostToDevice, s));
   QnnArgs A;
-  A.fuse = fuse;
-  A.ncirc = ncirc;
-  A.nfeat = nfeat;
-  A.layers = layers;
-  A.max_width = max_width;
-  A.lds_max_width = lds_w;
-  A.order = d_order;
-  A.widths = d_w;
-  A.x = d_x;
-  A.target = d_t;
-  A.theta = d_th;
-  A.expval = d_e;
-  A.loss_terms = d_l;
-  A.grad_circ = d_gc;
-  A.grad_x = d_gx;
-  A.slots = d_slots;
-  A.counter = d_cnt;
+  A.nfeat = nfeat, A.layers = layers, A.max_width = max_width;
+  A.alt = 0;
+  for (int q = 0; q < QNN_MAX_W; ++q) A.alt |= (uint32_t)(q % fuse != 0) << q;
+  A.widths = (const int32_t*)(d + w_off);
+  A.x = (const double*)(d + x_off);
+  A.target = (const double*)(d + t_off);
+  A.trig = (const double*)(d + trig_off);
+  double* res = (double*)(d + res_off);
+  A.expval = res, A.loss_terms = res + n, A.grad_x = res + 2 * n + nth;
+  A.grad_circ = (double*)(d + gc_off);
+  A.slots = (cx<float>*)(d + slot_off);
+  A.slot_width = wmax;
   A.inv_ncirc = 1.0 / ncirc;
-  if (lds_bytes > 64 * 1024)
-    QS_CHECK_HIP(hipFuncSetAttribute((const void*)k_qnn<R>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)lds_bytes));
-  int rc = prof_begin(ctx, PROF_QNN, s);
-  if (rc) return rc;
-  if (use_graph) {
-    if (!same) {
-      // queue reset + persistent kernel + ordered reduction, captured once and
-      // replayed for every batch of this shape
-      QS_CHECK_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      hipLaunchKernelGGL(k_qnn_clear, dim3(1), dim3(64), 0, s, d_cnt);
-      hipLaunchKernelGGL(k_qnn<R>, dim3(blocks), dim3(threads), lds_bytes, s, A);
-      hipLaunchKernelGGL(k_qnn_reduce, dim3((unsigned)((nth + 255) / 256)), dim3(256), 0, s, d_gc, ncirc, (int)nth,
-                         d_gth);
-      QS_CHECK_HIP(hipStreamEndCapture(s, &P.graph));
-      QS_CHECK_HIP(hipGraphInstantiate(&P.exec, P.graph, nullptr, nullptr, 0));
+  int* counters = (int*)(d + cnt_off);
+  if ((rc = prof_begin(ctx, PROF_QNN, s))) return rc;
+  hipLaunchKernelGGL(k_qnn_trig, dim3((unsigned)((layers * max_width + 63) / 64)), dim3(64), 0, s, (const double*)d, layers,
+                     max_width, (double*)(d + trig_off), counters, 3);
+  QS_CHECK_HIP(hipGetLastError());
+  for (int i = 0, first = 0; i < 3; first = end[i], ++i) {
+    A.first = first, A.n = end[i] - first, A.counter = counters + i;
+    if (A.n <= 0) continue;
+    const size_t lds = (size_t)2 << std::max((int)widths[order[first]], 1) << 3;
+    if (i == 0) {
+      hipLaunchKernelGGL((k_qnn<512, false>), dim3((unsigned)slots), dim3(512), 0, s, A);
+    } else if (i == 1) {
+      QS_CHECK_HIP(hipFuncSetAttribute((const void*)k_qnn<512, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       128 * 1024));
+      hipLaunchKernelGGL((k_qnn<512, true>), dim3((unsigned)std::min(A.n, 2 * cus)), dim3(512), lds, s, A);
+    } else {
+      hipLaunchKernelGGL((k_qnn<128, true>), dim3((unsigned)std::min(A.n, 16 * cus)), dim3(128), lds, s, A);
     }
-    QS_CHECK_HIP(hipGraphLaunch(P.exec, s));
-  } else {
-    hipLaunchKernelGGL(k_qnn_clear, dim3(1), dim3(64), 0, s, d_cnt);
-    QS_CHECK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_qnn<R>, dim3(blocks), dim3(threads), lds_bytes, s, A);
-    QS_CHECK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_qnn_reduce, dim3((unsigned)((nth + 255) / 256)), dim3(256), 0, s, d_gc, ncirc, (int)nth,
-                       d_gth);
     QS_CHECK_HIP(hipGetLastError());
   }
-  rc = prof_end(ctx, s);
-  if (rc) return rc;
-  P.dtype = dtype;
-  P.ncirc = ncirc;
-  P.nfeat = nfeat;
-  P.layers = layers;
-  P.max_width = max_width;
-  P.lds_max_width = lds_w;
-  P.threads = threads;
-  P.blocks = blocks;
-  P.fuse = fuse;
-  P.slots = slot_bytes != 0;
-  std::vector<double> lt(ncirc);
-  QS_CHECK_HIP(hipMemcpyAsync(expval, d_e, ncirc * sizeof(double), hipMemcpyDeviceToHost, s));
-  QS_CHECK_HIP(hipMemcpyAsync(lt.data(), d_l, ncirc * sizeof(double), hipMemcpyDeviceToHost, s));
-  QS_CHECK_HIP(hipMemcpyAsync(grad_theta, d_gth, nth * sizeof(double), hipMemcpyDeviceToHost, s));
-  if (grad_x)
-    QS_CHECK_HIP(hipMemcpyAsync(grad_x, d_gx, (uint64_t)ncirc * nfeat * sizeof(double), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_qnn_reduce, dim3((unsigned)((nth + 31) / 32)), dim3(256), 0, s, A.grad_circ, ncirc, (int)nth,
+                     res + 2 * n);
+  QS_CHECK_HIP(hipGetLastError());
+  if ((rc = prof_end(ctx, s))) return rc;
+  const double* r = (const double*)(S->host + res_off);
+  QS_CHECK_HIP(hipMemcpyAsync((void*)r, res, (grad_x ? nres : nres - nx) * sizeof(double), hipMemcpyDeviceToHost, s));
   QS_CHECK_HIP(hipStreamSynchronize(s));
-  (void)user_stream;
+  std::vector<double> terms(ncirc);
+  for (int i = 0; i < ncirc; ++i) {
+    expval[order[i]] = r[i];
+    terms[order[i]] = r[n + i];
+    if (grad_x && nfeat)
+      std::memcpy(grad_x + (uint64_t)order[i] * nfeat, r + 2 * n + nth + (uint64_t)i * nfeat, nfeat * sizeof(double));
+  }
+  std::copy(r + 2 * n, r + 2 * n + nth, grad_theta);
   double L = 0;
-  for (int i = 0; i < ncirc; ++i) L += lt[i];
+  for (int i = 0; i < ncirc; ++i) L += terms[i];
   *loss = L / ncirc;
   return QS_OK;
 }
@@ -876,7 +928,7 @@ static int qnn_prog_t(qs_ctx* ctx, int ncirc, const int32_t* widths, const int32
   hipLaunchKernelGGL(k_qnn_prog<R>, dim3(blocks), dim3(threads), lds_bytes, s, A);
   QS_CHECK_HIP(hipGetLastError());
   if (nparams) {
-    hipLaunchKernelGGL(k_qnn_reduce, dim3((unsigned)((nparams + 255) / 256)), dim3(256), 0, s, d_gc, ncirc, nparams,
+    hipLaunchKernelGGL(k_qnn_reduce, dim3((unsigned)((nparams + 31) / 32)), dim3(256), 0, s, d_gc, ncirc, nparams,
                        d_gth);
     QS_CHECK_HIP(hipGetLastError());
   }
@@ -910,10 +962,15 @@ extern "C" int qs_qnn_batch(qs_ctx* ctx, int dtype, int ncirc, const int32_t* wi
   for (int i = 0; i < ncirc; ++i) QS_REQUIRE(widths[i] >= 2 && widths[i] <= max_width, "width out of range");
   int rc = qnn_check(cfg, dtype);
   if (rc) return rc;
-  if (dtype == QS_C128)
-    return qnn_planned(ctx, ncirc, widths, nfeat, x, target, layers, max_width, theta, expval, loss, grad_theta, grad_x);
-  return qnn_t<float>(ctx, dtype, ncirc, widths, nfeat, x, target, layers, max_width, theta, expval, loss, grad_theta,
-                      grad_x, cfg, as_stream(stream));
+  try {
+    return dtype == QS_C128 ? qnn_planned(ctx, ncirc, widths, nfeat, x, target, layers, max_width, theta, expval, loss,
+                                          grad_theta, grad_x)
+                            : qnn_c64(ctx, cfg && cfg->fuse_qubits ? cfg->fuse_qubits : 1, ncirc, widths, nfeat, x, target, layers, max_width, theta, expval, loss,
+                                      grad_theta, grad_x);
+  } catch (const std::exception& e) {
+    set_error(std::string("batch of variational circuits: ") + e.what());
+    return QS_ERR_DEVICE;
+  }
 }
 
 extern "C" int qs_qnn_batch_programs(qs_ctx* ctx, int dtype, int ncirc, const int32_t* widths,

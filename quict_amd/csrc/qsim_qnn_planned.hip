@@ -17,20 +17,15 @@
 // time (k_qnn), which swept the state w / 2 times a layer forward and w / 2 back, in LDS
 // up to 11 qubits and in memory above; here 18 qubits take 4 passes forward and 3 back.
 #include "qsim_internal.hpp"
-#include "qsim_sweep.hpp"
+#include "qsim_qnn.hpp"
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <exception>
-#include <map>
-#include <mutex>
 #include <numeric>
 #include <vector>
 
 namespace qs {
-
-constexpr int QNN_MAX_W = 20;
 
 // The circuits of one width.  Their kernels outside the sweeps take a block of 256
 // threads per unit: 2^12 amplitudes of a circuit, or all of a narrower one's.
@@ -257,27 +252,7 @@ __global__ __launch_bounds__(256) void k_qnn_gradx_sum(const QnnGroups G, const 
   }
 }
 
-// What a context keeps for its batches: a stream (inputs and outputs are in host
-// memory, so nothing orders it with the caller's), buffers that grow on demand and are
-// given back with the context, and the planned programs.  One batch at a time.
-struct QnnState {
-  std::mutex mu;
-  hipStream_t stream = nullptr;
-  char* dev = nullptr;
-  char* host = nullptr;  // pinned
-  uint64_t dev_bytes = 0, host_bytes = 0;
-  std::map<std::pair<int, int>, VarImage> images;  // (width, layers)
-};
-constexpr size_t QNN_MAX_IMAGES = 64;  // 0.1..0.6 MB each; a batch has at most 19 widths
-
-QnnState* qnn_state_create() { return new QnnState(); }
-void qnn_state_destroy(QnnState* S) {
-  if (!S) return;
-  if (S->dev) (void)hipFree(S->dev);
-  if (S->host) (void)hipHostFree(S->host);
-  if (S->stream) (void)hipStreamDestroy(S->stream);
-  delete S;
-}
+constexpr size_t QNN_MAX_IMAGES = 64;  // planned programs kept, 0.1..0.6 MB each; a batch has at most 19 widths
 
 static int qnn_image(QnnState* S, int w, int layers, VarImage** out) {
   const auto key = std::make_pair(w, layers);
@@ -364,25 +339,8 @@ static int qnn_part(qs_ctx* ctx, QnnState* S, const int32_t* order, int n, int n
                  part_off = al(g_off + (grad_x ? units * QNN_MAX_W * sizeof(double) : 0)),
                  psi_off = al(part_off + part * sizeof(double)), lam_off = al(psi_off + amps * sizeof(cx<double>)),
                  total = lam_off + amps * sizeof(cx<double>);
-  if (S->dev_bytes < total) {
-    if (S->dev) QS_CHECK_HIP(hipFree(S->dev));
-    S->dev = nullptr, S->dev_bytes = 0;
-    const hipError_t err = hipMalloc((void**)&S->dev, total);
-    if (err != hipSuccess) {
-      (void)hipGetLastError();
-      S->dev = nullptr;
-      set_error(std::string("batch of variational circuits: ") + hipGetErrorString(err));
-      return QS_ERR_UNSUPPORTED;
-    }
-    S->dev_bytes = total;
-  }
-  const uint64_t host_bytes = res_off + nres * sizeof(double);
-  if (S->host_bytes < host_bytes) {
-    if (S->host) QS_CHECK_HIP(hipHostFree(S->host));
-    S->host = nullptr, S->host_bytes = 0;
-    QS_CHECK_HIP(hipHostMalloc((void**)&S->host, host_bytes, hipHostMallocDefault));
-    S->host_bytes = host_bytes;
-  }
+  int rc = S->room(total, res_off + nres * sizeof(double));
+  if (rc) return rc;
   for (int j = 0; j < G.n; ++j) std::memcpy(S->host + base[j], im[j]->host.data(), im[j]->host.size());
   std::memcpy(S->host + col_off, cols.data(), nc * sizeof(ColSum));
   double* hx = (double*)(S->host + x_off);
@@ -401,8 +359,7 @@ static int qnn_part(qs_ctx* ctx, QnnState* S, const int32_t* order, int n, int n
   const double* dx = (const double*)(d + x_off);
   const double* dt = (const double*)(d + t_off);
   QS_CHECK_HIP(hipMemcpyAsync(d, S->host, up, hipMemcpyHostToDevice, s));
-  int rc = prof_begin(ctx, PROF_QNN, s);
-  if (rc) return rc;
+  if ((rc = prof_begin(ctx, PROF_QNN, s))) return rc;
   const dim3 block(256), all((unsigned)units);
   hipLaunchKernelGGL(k_qnn_init, all, block, 0, s, G, dx, nfeat, psi);
   QS_CHECK_HIP(hipGetLastError());
@@ -470,11 +427,11 @@ static int qnn_part(qs_ctx* ctx, QnnState* S, const int32_t* order, int n, int n
 }
 
 int qnn_planned(qs_ctx* ctx, int ncirc, const int32_t* widths, int nfeat, const double* x, const double* target, int layers,
-                int max_width, const double* theta, double* expval, double* loss, double* grad_theta, double* grad_x) try {
+                int max_width, const double* theta, double* expval, double* loss, double* grad_theta, double* grad_x) {
   QnnState* S = ctx->qnn;
   std::lock_guard<std::mutex> lock(S->mu);
-  QS_CHECK_HIP(hipSetDevice(ctx->device));
-  if (!S->stream) QS_CHECK_HIP(hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking));
+  int rc0 = S->open(ctx->device);
+  if (rc0) return rc0;
   if (S->images.size() > QNN_MAX_IMAGES - QNN_MAX_W) S->images.clear();
   // widest first; as many circuits at a time as two vectors of 4 GiB hold, fewer if
   // the device has less to give
@@ -504,9 +461,6 @@ int qnn_planned(qs_ctx* ctx, int ncirc, const int32_t* widths, int nfeat, const 
   for (int i = 0; i < ncirc; ++i) L += terms[i];
   *loss = L / ncirc;
   return QS_OK;
-} catch (const std::exception& e) {
-  set_error(std::string("batch of variational circuits: ") + e.what());
-  return QS_ERR_DEVICE;
 }
 
 }  // namespace qs

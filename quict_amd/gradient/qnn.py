@@ -1,6 +1,6 @@
 """Batched QNN: many uneven-width parameterised circuits, forward + adjoint
 backward in one call (qs_qnn_batch): complex128 as planned tile passes over all
-circuits, complex64 in one persistent, graph-captured launch.
+circuits, complex64 with a workgroup a circuit.
 
 The circuit family (angle encoding, hardware-efficient ansatz, <Z_0> readout,
 squared loss) is documented in quict_amd/csrc/qsim_qnn.hip.  ``QNNBatch``
@@ -9,8 +9,9 @@ per-circuit <Z_0>, d loss / d theta and d loss / d x.
 
 ``autotune`` times every launch shape of a small search space on the real
 batch (LDS width limit, workgroup size, workgroups per CU) and caches the
-winner per (dtype, width histogram, layers, features) in a JSON file.  The shape
-matters to complex64; complex128 batches take the library's own.
+winner per (dtype, width histogram, layers, features) in a JSON file.  (The library
+takes its launch shapes from the widths; the values are checked, and fuse_qubits
+selects the order of rounding of complex64 results.)
 """
 import ctypes
 import json
