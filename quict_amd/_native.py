@@ -18,6 +18,7 @@ import numpy as np
 from .core import exception as qerr
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libqsim_hip.so")
+RECORDS_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libgate_records.so")
 
 QS_OK = 0
 QS_ERR_ARG = -1

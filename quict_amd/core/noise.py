@@ -113,9 +113,12 @@ class QuantumNoiseError:
         """The channels this one is the tensor product of (first = first qubit), or [self]."""
         return list(self._factors) if self._factors else [self]
 
-    def apply_to_gate(self, matrix: np.ndarray) -> List[np.ndarray]:
+    def check_gate(self, matrix: np.ndarray):
         if matrix.shape != (1 << self._qubits, 1 << self._qubits):
             raise qerr.NoiseApplyError("gate size differs from the noise's qubit count")
+
+    def apply_to_gate(self, matrix: np.ndarray) -> List[np.ndarray]:
+        self.check_gate(matrix)
         return [k @ matrix for k in self.kraus]
 
     def prob_mapping_operator(self, prob: float) -> np.ndarray:
@@ -284,23 +287,29 @@ class NoiseModel:
             raise qerr.NoiseApplyError("multi-qubit readout error needs exactly that many qubits")
         self._readout_errors.append((noise, qubits))
 
-    def transpile(self, circuit, accumulated_mode: bool = False):
+    def transpile(self, circuit, accumulated_mode: bool = False, lazy: bool = False):
         """Insert channels after (Kraus, ``NoiseGate``) or before (sampled Pauli
-        ``Unitary``) every listed gate (noise_model.py:152-185)."""
+        ``Unitary``) every listed gate (noise_model.py:152-185).  ``lazy``: the channels'
+        Kraus operators are multiplied by the gate's matrix when asked for."""
         from .circuit import Circuit
         out = Circuit(circuit.width())
         if circuit.precision != out.precision:
             out.convert_precision()
         for gate in circuit.gates:
-            if isinstance(gate, BasicGate) and gate.type.name in self._basic_gates:
+            # (_name_: Enum.name is a Python-level descriptor)
+            if isinstance(gate, BasicGate) and gate.type._name_ in self._error_by_gate:
                 args = gate.cargs + gate.targs
                 keep = True
-                for noise, qubits in self._error_by_gate[gate.type.name]:
+                for noise, qubits in self._error_by_gate[gate.type._name_]:
                     if qubits == -1 or set(qubits) & set(args) == set(args):
                         if accumulated_mode or noise.type == NoiseChannel.damping:
-                            ng = NoiseGate(noise.apply_to_gate(gate.matrix.astype(np.complex128)), len(args))
-                            ng.targs = list(args)
-                            ng.source = (gate, noise)
+                            matrix = gate.matrix.astype(np.complex128)
+                            if lazy:
+                                ng = NoiseGate.after_gate(gate, matrix, noise, len(args))
+                            else:
+                                ng = NoiseGate(noise.apply_to_gate(matrix), len(args))
+                                ng.source = (gate, noise)
+                            ng.targs = args
                             out.append(ng)
                             keep = False
                         else:

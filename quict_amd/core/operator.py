@@ -56,12 +56,38 @@ class NoiseGate(Operator):
 
     def __init__(self, noise_matrix: List[np.ndarray], args_num: int):
         super().__init__(args_num)
-        self._noise_matrix = [np.asarray(m) for m in noise_matrix]
-        self._precision = self._noise_matrix[0].dtype
+        self._matrices = [np.asarray(m) for m in noise_matrix]
+        self._precision = self._matrices[0].dtype
         # (gate, QuantumNoiseError) this channel was built from, when known: the
         # density-matrix simulator then applies the gate and the channel's
         # single-qubit factors separately (the same map, fewer operations)
         self.source = None
+        # the gate's matrix, while the Kraus operators have not been asked for
+        self.source_matrix = None
+
+    @classmethod
+    def after_gate(cls, gate, matrix: np.ndarray, noise, args_num: int) -> "NoiseGate":
+        """The channel ``noise`` after a gate with this (complex128) matrix; the Kraus
+        operators are multiplied out when somebody asks for them."""
+        noise.check_gate(matrix)
+        self = cls.__new__(cls)
+        Operator.__init__(self, args_num)
+        self._matrices = None
+        self._precision = np.result_type(noise.kraus[0].dtype, matrix.dtype)
+        self.source = (gate, noise)
+        self.source_matrix = matrix
+        return self
+
+    @property
+    def _noise_matrix(self) -> List[np.ndarray]:
+        if self._matrices is None:
+            self._matrices = [np.asarray(m) for m in self.source[1].apply_to_gate(self.source_matrix)]
+        return self._matrices
+
+    @_noise_matrix.setter
+    def _noise_matrix(self, matrices):
+        self._matrices = matrices
+        self.source_matrix = None
 
     @property
     def noise_matrix(self) -> List[np.ndarray]:

@@ -1164,20 +1164,25 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
   const int G = (int)W.g.size();
   const uint64_t all_wires = n >= 64 ? ~0ull : (1ull << n) - 1;
   std::vector<WClass> cls(G);
-  // the remaining gates, in order: bits, mixed bits, bits needed in the tile, weight
-  std::vector<uint64_t> ra(G), rm(G), rn(G);
-  std::vector<int> rid(G);
-  std::vector<int> rw(G);
+  // the remaining gates, in order
+  enum { ALONE = 1, TABLE = 2, MEAS = 4 };
+  struct Rem {
+    uint64_t a, m, need;  // its wires, those it mixes, those it needs in the tile
+    int id, w, flags;     // gate, weight
+  };
+  std::vector<Rem> rem(G);
   for (int i = 0; i < G; ++i) {
     const qs_gate& g = W.g[i];
-    cls[i] = wire_class(g, W.single[i], W.sym[i]);
-    ra[i] = gate_mask(g);
-    uint64_t t = 0;
-    for (int k = 0; k < g.ntargets; ++k) t |= 1ull << g.bits[g.ncontrols + k];
-    rm[i] = cls[i] == W_SINGLE ? ra[i] : cls[i] == W_PHASE || cls[i] == W_TABLE || cls[i] == W_ZMEAS ? 0 : t;
-    rn[i] = cls[i] == W_TABLE || cls[i] == W_ZMEAS ? ra[i] : rm[i];
-    rid[i] = i;
-    rw[i] = cls[i] == W_PHASE ? 1 : cls[i] == W_FLIP ? 0 : 2;
+    const WClass t = cls[i] = wire_class(g, W.single[i], W.sym[i]);
+    Rem& r = rem[i];
+    r.a = gate_mask(g);
+    uint64_t targets = 0;
+    for (int k = 0; k < g.ntargets; ++k) targets |= 1ull << g.bits[g.ncontrols + k];
+    r.m = t == W_SINGLE ? r.a : t == W_PHASE || t == W_TABLE || t == W_ZMEAS ? 0 : targets;
+    r.need = t == W_TABLE || t == W_ZMEAS ? r.a : r.m;
+    r.id = i;
+    r.w = t == W_PHASE ? 1 : t == W_FLIP ? 0 : 2;
+    r.flags = (t == W_SINGLE ? ALONE : 0) | (t == W_TABLE ? TABLE : 0) | (W.sym[i].meas != 0.0 ? MEAS : 0);
   }
   prog.pgates = W.g;
   prog.psym = W.sym;
@@ -1195,26 +1200,38 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
   int R = G;
   const int max_tables = FMAX_PASS_COEF / (4 << c.RB);  // staged in LDS
   // Weight of the gates that run with tile wires S; cand: what further unblocked
-  // gates need besides (in order, each once); taken: the gates (positions).
-  auto scan = [&](uint64_t S, std::vector<uint64_t>* cand, std::vector<int>* taken) -> int {
+  // gates need besides (in order, each once); taken: the gates (positions).  from:
+  // where the first gate is that does not run, and what was counted before; more wires
+  // do not change that part.
+  struct From {
+    int k = 0, w = 0, tables = 0, meas = 0;
+  };
+  auto scan = [&](uint64_t S, From& from, std::vector<uint64_t>* cand, std::vector<int>* taken) -> int {
     uint64_t wa = 0, wm = 0;
-    int w = 0, tables = 0, meas = 0;
-    for (int k = 0; k < R; ++k) {
-      const uint64_t a = ra[k], m = rm[k];
-      if (!((a & wm) | (m & wa))) {
-        const uint64_t need = rn[k] & ~S;
-        bool room = cls[rid[k]] != W_TABLE || ++tables <= max_tables;
-        if (W.sym[rid[k]].meas != 0.0) room = ++meas <= FMAX_GRAD;
-        if (!need && room && cls[rid[k]] != W_SINGLE) {
-          w += rw[k];
+    int w = from.w, tables = from.tables, meas = from.meas;
+    for (int k = from.k; k < R; ++k) {
+      const Rem& r = rem[k];
+      if (!((r.a & wm) | (r.m & wa))) {
+        const uint64_t need = r.need & ~S;
+        const int t0 = tables, m0 = meas;
+        bool room = true;
+        if (r.flags) {
+          if (r.flags & TABLE) room = ++tables <= max_tables;
+          if (r.flags & MEAS) room = ++meas <= FMAX_GRAD;
+        }
+        const bool able = room && !(r.flags & ALONE);
+        if (!need && able) {
+          w += r.w;
           if (taken) taken->push_back(k);
           continue;
         }
-        if (cand && need && room && cls[rid[k]] != W_SINGLE && std::find(cand->begin(), cand->end(), need) == cand->end())
-          cand->push_back(need);
+        if (cand) {
+          if (!wa) from.k = k, from.w = w, from.tables = t0, from.meas = m0;
+          if (need && able && std::find(cand->begin(), cand->end(), need) == cand->end()) cand->push_back(need);
+        }
       }
-      wa |= a;
-      wm |= m;
+      wa |= r.a;
+      wm |= r.m;
       if (wm == all_wires) break;
     }
     return w;
@@ -1284,23 +1301,25 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
       return __builtin_popcountll(S) <= K && (!have || __builtin_popcountll(S & ~PS) <= K - L);
     };
     uint64_t S = start;
+    From from;
     for (;;) {
       cand.clear();
-      const int base = scan(S, &cand, nullptr);
+      const int base = scan(S, from, &cand, nullptr);
       uint64_t best = 0;
       double best_gain = -1;
       int nfit = 0;
       for (uint64_t m : cand) nfit += fits(S | m);
       for (uint64_t m : cand) {
         if (!fits(S | m)) continue;
-        const double gain = nfit == 1 ? 0 : (double)(scan(S | m, nullptr, nullptr) - base) / __builtin_popcountll(m);
+        const double gain = nfit == 1 ? 0 : (double)(scan(S | m, from, nullptr, nullptr) - base) / __builtin_popcountll(m);
         if (gain > best_gain) best_gain = gain, best = m;
       }
       if (!best) break;
       S |= best;
     }
     taken.clear();
-    scan(S, nullptr, &taken);
+    from = From();
+    scan(S, from, nullptr, &taken);
     // Phases that no later gate of the pass waits for stay for a pass that needs
     // them, where one of their bits is a register bit; unless no mixing gate is left.
     std::vector<char> drop(R, 0);
@@ -1308,13 +1327,13 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
       std::vector<char> in(R, 0);
       for (int k : taken) in[k] = 1;
       bool left = false;
-      for (int k = 0; k < R; ++k) left = left || (!in[k] && rn[k] != 0);
+      for (int k = 0; k < R; ++k) left = left || (!in[k] && rem[k].need != 0);
       if (left) {
         uint64_t later = 0;
         for (size_t i = taken.size(); i-- > 0;) {
           const int k = taken[i];
-          if (cls[rid[k]] == W_PHASE && !(ra[k] & later)) drop[k] = 1;
-          else later |= rm[k];
+          if (cls[rem[k].id] == W_PHASE && !(rem[k].a & later)) drop[k] = 1;
+          else later |= rem[k].m;
         }
       }
       size_t o = 0;
@@ -1333,23 +1352,20 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
       }
       PassPlan p;
       p.fused = false;
-      p.single = rid[0];
+      p.single = rem[0].id;
       translate(p.single);
       prog.plans.push_back(std::move(p));
-      for (int k = 1; k < R; ++k) ra[k - 1] = ra[k], rm[k - 1] = rm[k], rn[k - 1] = rn[k], rid[k - 1] = rid[k], rw[k - 1] = rw[k];
+      rem.erase(rem.begin());
       --R;
       continue;
     }
     std::vector<int> ids;
     {
       std::vector<char> in(R, 0);
-      for (int k : taken) in[k] = 1, ids.push_back(rid[k]);
+      for (int k : taken) in[k] = 1, ids.push_back(rem[k].id);
       int o = 0;
       for (int k = 0; k < R; ++k)
-        if (!in[k]) {
-          ra[o] = ra[k], rm[o] = rm[k], rn[o] = rn[k], rid[o] = rid[k], rw[o] = rw[k];
-          ++o;
-        }
+        if (!in[k]) rem[o++] = rem[k];
       R = o;
     }
     // fill the tile: wires of the pass before (they leave its store a choice of

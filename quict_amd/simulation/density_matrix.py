@@ -19,7 +19,6 @@ entry (r, c) at index r*2^n + c) is treated as a 2n-bit vector:
 """
 import ctypes
 import random
-from typing import List
 
 import numpy as np
 
@@ -28,52 +27,133 @@ from ..core import exception as qerr
 from ..core.noise import NoiseModel
 from .. import _native as nat
 from .device_array import DeviceArray
-from .gate_compiler import compile_gate, superop_record
+from .gate_compiler import _translate, _write, superop_record, superop_write, superoperators
+from .uniforms import uniforms
 
 
-def op_records(g, n: int, keep: list) -> list:
-    """Records of one unitary gate or noise channel on the 2n-bit image of rho
-    (row bits n..2n-1, column bits 0..n-1): a gate U is U on its row bits and
-    conj(U) on its column bits; a channel is its superoperator.  A tensor-product
-    channel applied after a gate (accumulated mode) is the gate's two records
-    followed by one superoperator per single-qubit factor."""
-    out = []
+_NO_MATRIX = (GateType.id, GateType.barrier, GateType.measure, GateType.reset, GateType.perm)
 
-    def unitary(gate):
-        row = np.zeros(1, dtype=nat.QS_GATE_DTYPE)[0]
-        col = np.zeros(1, dtype=nat.QS_GATE_DTYPE)[0]
-        if compile_gate(gate, n, row, keep, row_offset=n):
-            compile_gate(gate, n, col, keep, row_offset=0, conj=True)
-            out.extend([row, col])
 
-    if isinstance(g, NoiseGate):
-        factors = g.source[1].factors if g.source is not None else None
-        if factors and len(factors) > 1 and len(factors) == len(g.targs) and all(f.qubits == 1 for f in factors):
-            unitary(g.source[0])
-            for f, q in zip(factors, g.targs):
-                rec = np.zeros(1, dtype=nat.QS_GATE_DTYPE)[0]
-                superop_record(f.kraus, [q], n, rec, keep)
-                out.append(rec)
-        else:
-            rec = np.zeros(1, dtype=nat.QS_GATE_DTYPE)[0]
-            superop_record(g.noise_matrix, list(g.targs), n, rec, keep)
-            out.append(rec)
-    else:
-        unitary(g)
-    return out
+class _Program:
+    """Records of unitary gates and noise channels on the 2n-bit image of rho (row
+    bits n..2n-1, column bits 0..n-1): a gate U is U on its row bits and conj(U) on its
+    column bits; a channel is its superoperator.  A tensor-product channel applied
+    after a gate (accumulated mode) is the gate's two records followed by one
+    superoperator per single-qubit factor.
+
+    A record without its bits depends on a matrix (or on a channel and a matrix) only,
+    and a circuit repeats few of them: within one program each is made once, the
+    superoperators of a channel all together."""
+
+    def __init__(self, n: int):
+        self.n = n
+        self.keep: list = []
+        self._templates = np.zeros(32, dtype=nat.QS_GATE_DTYPE)  # distinct records, bits unset
+        self._count = 0
+        self._rows: list = []        # template of each record ...
+        self._bits: list = []        # ... and its bits
+        self._memo: dict = {}
+        self._channels: dict = {}    # id(channel) -> (channel, [template], [matrix])
+        self._held: list = []        # objects whose ids are keys
+
+    def _new(self) -> int:
+        if self._count == len(self._templates):
+            grown = np.zeros(2 * self._count, dtype=nat.QS_GATE_DTYPE)
+            grown[: self._count] = self._templates
+            self._templates = grown
+        self._count += 1
+        return self._count - 1
+
+    def _put(self, template: int, bits: list):
+        self._rows.append(template)
+        self._bits.append(bits + [0] * (nat.QS_MAX_GATE_BITS - len(bits)))
+
+    def add(self, g):
+        if not isinstance(g, NoiseGate):
+            self._unitary(g)
+            return
+        if g.source is not None:
+            noise = g.source[1]
+            factors = noise.factors
+            if len(factors) > 1 and len(factors) == len(g.targs) and all(f.qubits == 1 for f in factors):
+                self._unitary(g.source[0])
+                self._held.append(noise)
+                for f, q in zip(factors, g.targs):
+                    self._superop(("factor", id(f)), f.kraus, [q])
+                return
+            if g.source_matrix is not None:
+                self._after_gate(noise, g.source_matrix, list(g.targs))
+                return
+        self._superop(None, g.noise_matrix, list(g.targs))
+
+    def _unitary(self, gate):
+        n = self.n
+        key = None
+        if gate.params == 0 and gate.type not in _NO_MATRIX:
+            m = np.asarray(gate.matrix)
+            key = (id(gate.type), gate.controls, gate.targets, m.dtype.char, m.tobytes())
+        pair = self._memo.get(key) if key else None
+        if pair is None:
+            r = _translate(gate, n, self.keep, n, False, False)
+            if r is None:
+                return
+            kind, c, t, _, payload, big = r
+            pair = (self._new(), self._new())
+            _write(self._templates[pair[0]], (kind, c, t, (), payload, big))
+            if big:
+                payload, big = _translate(gate, n, self.keep, 0, True, False)[4:]
+            else:
+                payload = np.conj(payload)
+            _write(self._templates[pair[1]], (kind, c, t, (), payload, big))
+            if key:
+                self._memo[key] = pair
+        args = gate.cargs + gate.targs
+        self._put(pair[0], [2 * n - 1 - a for a in args])
+        self._put(pair[1], [n - 1 - a for a in args])
+
+    def _channel_bits(self, args):
+        return [2 * self.n - 1 - a for a in args] + [self.n - 1 - a for a in args]
+
+    def _superop(self, key, kraus, args):
+        t = self._memo.get(key) if key else None
+        if t is None:
+            t = self._new()
+            superop_record(kraus, args, self.n, self._templates[t], self.keep)
+            if key:
+                self._memo[key] = t
+        self._put(t, self._channel_bits(args))
+
+    def _after_gate(self, noise, matrix, args):
+        """A channel's Kraus operators times the gate's matrix: left to ``array``."""
+        key = (id(noise), matrix.tobytes())
+        t = self._memo.get(key)
+        if t is None:
+            t = self._memo[key] = self._new()
+            _, ts, ms = self._channels.setdefault(id(noise), (noise, [], []))
+            ts.append(t)
+            ms.append(matrix)
+        self._put(t, self._channel_bits(args))
+
+    def array(self) -> np.ndarray:
+        for noise, ts, ms in self._channels.values():
+            K = np.matmul(np.asarray(noise.kraus)[None], np.stack(ms)[:, None])
+            for t, S in zip(ts, superoperators(K)):
+                superop_write(S, self._templates[t], self.keep)
+        arr = self._templates[self._rows]
+        arr["bits"] = self._bits
+        return arr
+
+    def __len__(self):
+        return len(self._rows)
 
 
 def program_records(ops, n: int):
     """Record array of a measurement-free list of gates and channels (the program
     the density-matrix simulator hands to qs_sv_apply_gates on 2n bits)."""
-    keep: list = []
-    recs = []
+    prog = _Program(n)
     for g in ops:
-        recs.extend(op_records(g, n, keep))
-    arr = np.zeros(len(recs), dtype=nat.QS_GATE_DTYPE)
-    for i, r in enumerate(recs):
-        arr[i] = r
-    return arr, keep
+        prog.add(g)
+    return (prog.array() if len(prog) else np.zeros(0, dtype=nat.QS_GATE_DTYPE)), prog.keep
 
 
 class DensityMatrixSimulator:
@@ -112,7 +192,7 @@ class DensityMatrixSimulator:
 
     def initial_circuit(self, circuit: Circuit, noise_model: NoiseModel):
         self._origin_circuit = circuit
-        self._circuit = circuit if noise_model is None else noise_model.transpile(circuit, self._accumulated_mode)
+        self._circuit = circuit if noise_model is None else noise_model.transpile(circuit, self._accumulated_mode, lazy=True)
         self._noise_model = noise_model
         self._qubits = int(circuit.width())
 
@@ -153,22 +233,20 @@ class DensityMatrixSimulator:
 
     def _run(self, circuit: Circuit):
         n = self._qubits
-        recs: List = []
-        keep: list = []
+        prog = _Program(n)
 
         def flush():
-            if not recs:
+            nonlocal prog
+            if not len(prog):
                 return
-            arr = np.zeros(len(recs), dtype=nat.QS_GATE_DTYPE)
-            for i, r in enumerate(recs):
-                arr[i] = r
+            arr = prog.array()
             passes = ctypes.c_int(0)
             rc = self._lib.qs_sv_apply_gates(self._ctx, self._rptr(), 2 * n, self._dcode, nat.gate_array_ptr(arr),
                                              len(arr), 1 if self._fusion else 0, ctypes.byref(passes),
                                              self._stream())
             nat.check(rc, "qs_sv_apply_gates(density matrix)")
             self.last_passes += passes.value
-            recs.clear()
+            prog = _Program(n)
 
         for g in circuit.gates:
             if isinstance(g, BasicGate) and g.type == GateType.measure:
@@ -177,11 +255,10 @@ class DensityMatrixSimulator:
             elif isinstance(g, BasicGate) and g.type in (GateType.reset, GateType.perm):
                 raise qerr.GateTypeNotImplementError(f"{g.type.name} in the density-matrix simulator")
             elif isinstance(g, (BasicGate, NoiseGate)):
-                recs.extend(op_records(g, n, keep))
+                prog.add(g)
             else:
                 raise qerr.TypeError("DensityMatrixSimulator takes BasicGate / NoiseGate, got", type(g))
         flush()
-        del keep
 
     def apply_measure(self, index: int):
         """density_matrix_simulator.py:182-208 (``index`` is the qubit)."""
@@ -225,7 +302,7 @@ class DensityMatrixSimulator:
         if self._accumulated_mode or self._noise_model is None:
             if len(measured) == n and self._noise_model is None or (len(measured) == n and
                                                                      not self._noise_model._readout_errors):
-                u = np.array([random.random() for _ in range(shots * n)], dtype=np.float64)
+                u = uniforms(shots * n)
                 d = self._torch.empty(1 << n, dtype=self._torch.float64, device=f"cuda:{self._device_id}")
                 nat.check(self._lib.qs_dm_diagonal(self._ctx, self._rptr(), n, self._dcode,
                                                    ctypes.c_void_p(d.data_ptr()), self._stream()), "qs_dm_diagonal")
@@ -256,7 +333,7 @@ class DensityMatrixSimulator:
             self._noise_model.apply_readout_error(self._circuit.qubits)
             counts[int(self._circuit.qubits)] += 1
             self.initial_density_matrix(n)
-            noised = self._noise_model.transpile(self._origin_circuit, self._accumulated_mode)
+            noised = self._noise_model.transpile(self._origin_circuit, self._accumulated_mode, lazy=True)
             self._circuit = noised
             self._run(noised)
         return counts

@@ -16,6 +16,8 @@ kernel by (MatrixType, #controls, #targets) and passes reversed qubit indices
 Gate arguments are ``cargs + targs`` with argument 0 the most significant bit
 of the gate-matrix index, mapped to amplitude bit ``n-1-q``.
 """
+import ctypes
+import os
 from typing import List, Tuple
 
 import numpy as np
@@ -119,10 +121,51 @@ def compile_gate(gate: BasicGate, n: int, rec: np.ndarray, keep: list, row_offse
     r = _translate(gate, n, keep, row_offset, conj, dagger)
     if r is None:
         return False
+    _write(rec, r)
+    return True
+
+
+# Gate types that the native helper turns into records: rotations, in its order, whose
+# payloads it computes, and parameter-free types of fixed shape, whose record depends
+# only on the type and precision.
+_ROTATION_TYPES = (GateType.rx, GateType.ry, GateType.rz, GateType.crz, GateType.u1, GateType.cu1, GateType.u3)
+_STATIC_TYPES = (
+    GateType.h, GateType.hy, GateType.s, GateType.sdg, GateType.x, GateType.y, GateType.z, GateType.sx,
+    GateType.sy, GateType.sw, GateType.t, GateType.tdg, GateType.cx, GateType.cy, GateType.cz, GateType.ch,
+    GateType.swap, GateType.iswap, GateType.iswapdg, GateType.sqiswap, GateType.cswap, GateType.ccx,
+    GateType.ccz)
+_RECORDS_LIB = None  # (function, types, prototypes), set on first use
+
+
+def _static_prototypes() -> np.ndarray:
+    """Records of the fixed types, each in complex128 and complex64, bits unset."""
+    protos = np.zeros(2 * len(_STATIC_TYPES), dtype=nat.QS_GATE_DTYPE)
+    for i, gt in enumerate(_STATIC_TYPES):
+        gate = BasicGate(_type=gt)
+        gate._cargs, gate._targs = list(range(gate.controls)), list(range(gate.controls, gate.controls + gate.targets))
+        for single in (0, 1):
+            compile_gate(gate, gate.controls + gate.targets, protos[2 * i + single], [])
+            gate.convert_precision()
+    protos["bits"] = 0
+    return protos
+
+
+def _records_lib():
+    global _RECORDS_LIB
+    if _RECORDS_LIB is None:
+        if not os.path.exists(nat.RECORDS_PATH):
+            raise nat.qerr.NativeRuntimeError(f"{nat.RECORDS_PATH} is missing: build it with `make -C quict_amd/csrc`")
+        fn = ctypes.PyDLL(nat.RECORDS_PATH).gate_records
+        fn.restype = ctypes.c_int
+        O, P = ctypes.py_object, ctypes.c_void_p
+        fn.argtypes = [O, O, O, O, O, P, ctypes.c_int, P, P]
+        _RECORDS_LIB = (fn, _ROTATION_TYPES + _STATIC_TYPES, _static_prototypes())
+    return _RECORDS_LIB
+
+
+def _write(rec, r):
     kind, c, t, bits, payload, big = r
-    rec["kind"] = kind
-    rec["ncontrols"] = c
-    rec["ntargets"] = t
+    rec["kind"], rec["ncontrols"], rec["ntargets"] = kind, c, t
     rec["bits"][:] = 0
     rec["bits"][: len(bits)] = bits
     rec["m"][:] = 0
@@ -130,174 +173,64 @@ def compile_gate(gate: BasicGate, n: int, rec: np.ndarray, keep: list, row_offse
         v = np.ascontiguousarray(payload, dtype=np.complex128).view(np.float64)
         rec["m"][: len(v)] = v
     rec["big"] = big
-    return True
-
-
-# Parameter-free gate types of fixed shape: the record (kind, controls, targets,
-# payload) depends only on the type and precision, so it is translated once and
-# reused; only the bit positions differ between instances.
-_STATIC_TYPES = frozenset([
-    GateType.h, GateType.hy, GateType.s, GateType.sdg, GateType.x, GateType.y, GateType.z, GateType.sx,
-    GateType.sy, GateType.sw, GateType.t, GateType.tdg, GateType.cx, GateType.cy, GateType.cz, GateType.ch,
-    GateType.swap, GateType.iswap, GateType.iswapdg, GateType.sqiswap, GateType.cswap, GateType.ccx,
-    GateType.ccz])
-_STATIC_RECORDS = {}
-# One-angle / three-angle rotations whose payloads are computed for all gates of
-# a call at once with the closed forms of the gate module (core/gate.py).
-_ROTATION_TYPES = frozenset([GateType.rx, GateType.ry, GateType.rz, GateType.crz, GateType.u1, GateType.u3])
-
-
-def _rotation_records(gt: GateType, P: np.ndarray, dt):
-    """(kind per gate, payload rows, degenerate mask) for rotations of type gt with
-    parameter rows P, matching _translate: the matrix in the gate's precision dt,
-    the same record-kind decisions.  Degenerate gates (a dense matrix that is
-    exactly diagonal) go back to the generic path."""
-    G = P.shape[0]
-    cast = (lambda a: a.astype(dt).astype(np.complex128))
-    if gt in (GateType.rx, GateType.ry, GateType.u3):
-        th = P[:, 0]
-        c, s = np.cos(th / 2), np.sin(th / 2)
-        if gt == GateType.rx:
-            pay = np.stack([c + 0j, 1j * -s, 1j * -s, c + 0j], 1)
-        elif gt == GateType.ry:
-            pay = np.stack([c + 0j, -s + 0j, s + 0j, c + 0j], 1)
-        else:
-            pay = np.stack([np.cos(th / 2) + 0j, -np.exp(1j * P[:, 2]) * np.sin(th / 2),
-                            np.exp(1j * P[:, 1]) * np.sin(th / 2), np.exp(1j * (P[:, 1] + P[:, 2])) * np.cos(th / 2)],
-                           1)
-        pay = cast(pay)
-        degenerate = (pay[:, 1] == 0) & (pay[:, 2] == 0)
-        return np.full(G, nat.GATE_DENSE, dtype=np.int32), pay, degenerate
-    if gt == GateType.u1:
-        pay = cast(np.exp(1j * P[:, 0]))[:, None]
-        return np.full(G, nat.GATE_PHASE, dtype=np.int32), pay, np.zeros(G, dtype=bool)
-    # rz, crz: diagonal (e^{-i th/2}, e^{i th/2}); PHASE when the first entry is 1
-    d = cast(np.stack([np.exp(-P[:, 0] / 2 * 1j), np.exp(P[:, 0] / 2 * 1j)], 1))
-    phase = d[:, 0] == 1
-    kind = np.where(phase, nat.GATE_PHASE, nat.GATE_DIAG).astype(np.int32)
-    pay = np.where(phase[:, None], np.stack([d[:, 1], np.zeros(G, dtype=np.complex128)], 1), d)
-    return kind, pay, np.zeros(G, dtype=bool)
 
 
 def compile_gates(gates: List[BasicGate], n: int, row_offset: int = 0, conj: bool = False,
                   dagger: bool = False) -> Tuple[np.ndarray, list]:
     """Records for a run of unitary gates; ``keep`` holds arrays referenced by pointer.
-    The fields are gathered in plain arrays and written column-wise.  Fixed gate
-    types reuse one translated record per type; Rx / Ry / Rz / CRz / U1 / U3
-    payloads are computed for the whole run at once (plain records only: no row
-    offset, conjugation or inverse); everything else goes through _translate."""
+    The native helper fills the records of fixed gate types and of rotations (plain
+    records only: no row offset, conjugation or inverse); the rest goes through
+    _translate."""
     keep: list = []
+    gates = list(gates)
     G = len(gates)
-    kind = np.zeros(G, dtype=np.int32)
-    nc = np.zeros(G, dtype=np.int32)
-    nt = np.zeros(G, dtype=np.int32)
-    bits = np.zeros((G, nat.QS_MAX_GATE_BITS), dtype=np.int32)
-    m = np.zeros((G, 32), dtype=np.float64)
-    big = np.zeros(G, dtype=np.uint64)
-    fast = row_offset == 0 and not conj and not dagger
-    rot = {}   # (type, precision) -> ([slot], [gate])
-    static = {}  # (type, precision) -> [slot]
-    b1k, b1 = [], []              # one-argument gates: slot, argument
-    b2k, b2a, b2b = [], [], []    # two-argument gates: slot, arguments
-    k = 0
-    for g in gates:
-        gt = g.type
-        if fast and (gt in _STATIC_TYPES or gt in _ROTATION_TYPES):
-            args = g.cargs + g.targs
-            if len(args) == 1:
-                b1k.append(k)
-                b1.append(args[0])
-            elif len(args) == 2:
-                b2k.append(k)
-                b2a.append(args[0])
-                b2b.append(args[1])
-            else:
-                bits[k, : len(args)] = [n - 1 - a for a in args]
-            key = (gt, g.precision)
-            if gt in _STATIC_TYPES:
-                lst = static.get(key)
-                if lst is None:
-                    lst = static[key] = [g]  # the first entry: a gate to translate once
-                lst.append(k)
-            else:
-                lst = rot.setdefault(key, ([], []))
-                lst[0].append(k)
-                lst[1].append(g)
-            k += 1
-            continue
-        r = _translate(g, n, keep, row_offset, conj, dagger)
+    arr = np.empty(G, dtype=nat.QS_GATE_DTYPE)
+    if row_offset == 0 and not conj and not dagger:
+        fn, types, protos = _records_lib()
+        left = np.empty(G, dtype=np.int32)
+        nleft = fn(gates, BasicGate, types, np.complex128, np.complex64, protos.ctypes.data, n, arr.ctypes.data,
+                   left.ctypes.data)
+        rest = left[:nleft].tolist()
+    else:
+        rest = range(G)
+    drop = []
+    for k in rest:
+        r = _translate(gates[k], n, keep, row_offset, conj, dagger)
         if r is None:
-            continue
-        kind[k], nc[k], nt[k] = r[0], r[1], r[2]
-        bits[k, : len(r[3])] = r[3]
-        if r[4] is not None:
-            v = np.ascontiguousarray(r[4], dtype=np.complex128).view(np.float64)
-            m[k, : len(v)] = v
-        big[k] = r[5]
-        k += 1
-    if b1k:
-        bits[b1k, 0] = n - 1 - np.asarray(b1)
-    if b2k:
-        bits[b2k, 0] = n - 1 - np.asarray(b2a)
-        bits[b2k, 1] = n - 1 - np.asarray(b2b)
-    for key, lst in static.items():
-        rec = _STATIC_RECORDS.get(key)
-        if rec is None:
-            r = _translate(lst[0], n, keep, 0, False, False)
-            rec = _STATIC_RECORDS[key] = (r[0], r[1], r[2], None if r[4] is None else
-                                          np.ascontiguousarray(r[4], dtype=np.complex128).view(np.float64))
-        idx = np.asarray(lst[1:])
-        kind[idx], nc[idx], nt[idx] = rec[0], rec[1], rec[2]
-        if rec[3] is not None:
-            m[idx, : len(rec[3])] = rec[3]
-    for (gt, dt), (slots, gl) in rot.items():
-        nc[slots], nt[slots] = gl[0].controls, gl[0].targets
-    for (gt, dt), (slots, gl) in rot.items():
-        slots = np.asarray(slots)
-        P = np.array([g.pargs for g in gl], dtype=np.float64)
-        kk, pay, degenerate = _rotation_records(gt, P, dt)
-        kind[slots] = kk
-        m[slots, : 2 * pay.shape[1]] = np.ascontiguousarray(pay).view(np.float64)
-        for i in np.nonzero(degenerate)[0]:
-            r = _translate(gl[i], n, keep, 0, False, False)
-            j = slots[i]
-            kind[j], nc[j], nt[j] = r[0], r[1], r[2]
-            bits[j, :] = 0
-            bits[j, : len(r[3])] = r[3]
-            m[j, :] = 0
-            v = np.ascontiguousarray(r[4], dtype=np.complex128).view(np.float64)
-            m[j, : len(v)] = v
-    arr = np.zeros(k, dtype=nat.QS_GATE_DTYPE)
-    arr["kind"] = kind[:k]
-    arr["ncontrols"] = nc[:k]
-    arr["ntargets"] = nt[:k]
-    arr["bits"] = bits[:k]
-    arr["m"] = m[:k]
-    arr["big"] = big[:k]
+            drop.append(k)
+        else:
+            _write(arr[k], r)
+    if drop:
+        arr = np.delete(arr, drop)
     return arr, keep
 
 
-def superop_record(kraus: List[np.ndarray], args: List[int], n: int, rec, keep: list):
-    """Record for a channel sum_k K (.) K^dagger on density-matrix qubits ``args``:
-    dense superoperator sum_k K (x) conj(K) on [row bits..., column bits...]."""
-    m = len(args)
-    d = 1 << m
-    Ks = np.asarray(kraus, dtype=np.complex128).reshape(-1, d, d)
-    # sum_k kron(K_k, conj(K_k)): S[(a, c), (b, e)] = sum_k K_k[a, b] conj(K_k[c, e])
-    S = np.einsum("kab,kce->acbe", Ks, Ks.conj()).reshape(d * d, d * d)
-    row_bits = [2 * n - 1 - a for a in args]
-    col_bits = [n - 1 - a for a in args]
-    rec["kind"] = nat.GATE_DENSE
-    rec["ncontrols"] = 0
-    rec["ntargets"] = 2 * m
+def superoperators(K: np.ndarray) -> np.ndarray:
+    """sum_k K_k (x) conj(K_k) of channels with Kraus operators K[channel, k]:
+    S[(a, c), (b, e)] = sum_k K_k[a, b] conj(K_k[c, e])."""
+    d = K.shape[-1]
+    return np.einsum("nkab,nkce->nacbe", K, K.conj()).reshape(-1, d * d, d * d)
+
+
+def superop_write(S: np.ndarray, rec, keep: list):
+    """S as a dense record, bits unset."""
+    v = np.ascontiguousarray(S).view(np.float64).ravel()
+    t = S.shape[0].bit_length() - 1
+    rec["kind"], rec["ncontrols"], rec["ntargets"] = nat.GATE_DENSE, 0, t
     rec["bits"][:] = 0
-    rec["bits"][: 2 * m] = row_bits + col_bits
     rec["m"][:] = 0
     rec["big"] = 0
-    v = np.ascontiguousarray(S).view(np.float64).ravel()
-    if 2 * m <= 2:
+    if t <= 2:
         rec["m"][: len(v)] = v
     else:
         big = v.copy()
         keep.append(big)
         rec["big"] = big.ctypes.data
+
+
+def superop_record(kraus: List[np.ndarray], args: List[int], n: int, rec, keep: list):
+    """Record for a channel sum_k K (.) K^dagger on density-matrix qubits ``args``:
+    dense superoperator sum_k K (x) conj(K) on [row bits..., column bits...]."""
+    d = 1 << len(args)
+    superop_write(superoperators(np.asarray(kraus, dtype=np.complex128).reshape(1, -1, d, d))[0], rec, keep)
+    rec["bits"][: 2 * len(args)] = [2 * n - 1 - a for a in args] + [n - 1 - a for a in args]

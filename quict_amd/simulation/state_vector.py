@@ -27,6 +27,7 @@ from ..core import exception as qerr
 from .. import _native as nat
 from .device_array import DeviceArray
 from .gate_compiler import compile_gates
+from .uniforms import uniforms
 
 
 class CapturedCircuit:
@@ -155,26 +156,35 @@ class StateVectorSimulator:
         elif not use_previous or self._vector is None or self._vector.numel() != (1 << self._qubits):
             self.initial_state_vector()
         self.last_passes = 0
-        pending: List[BasicGate] = []
         idx = 0
         while idx < len(self._pipeline):
-            op = self._pipeline[idx]
-            idx += 1
-            if isinstance(op, BasicGate) and op.type not in (GateType.measure, GateType.reset, GateType.perm):
-                pending.append(op)
-                continue
-            self._flush(pending)
-            pending = []
+            end = self._run_of_gates(idx)
+            self._flush(self._pipeline[idx:end])
+            if end == len(self._pipeline):
+                break
+            op = self._pipeline[end]
+            idx = end + 1
             if isinstance(op, Trigger):
                 self.apply_trigger(op, idx)
             elif isinstance(op, BasicGate):
                 self.apply_gate(op)
             else:
                 raise qerr.TypeError("StateVectorSimulator.run takes BasicGate / Trigger, got", type(op))
-        self._flush(pending)
         if self._sync:
             self._torch.cuda.synchronize(self._device_id)
         return self.vector
+
+    def _run_of_gates(self, idx: int) -> int:
+        """End of the run of unitary gates that starts at pipeline position ``idx``."""
+        measure, reset, perm = GateType.measure, GateType.reset, GateType.perm
+        for k in range(idx, len(self._pipeline)):
+            op = self._pipeline[k]
+            if not isinstance(op, BasicGate):
+                return k
+            t = op.type
+            if t is measure or t is reset or t is perm:
+                return k
+        return len(self._pipeline)
 
     def capture(self, circuit: Circuit) -> CapturedCircuit:
         """Plan and capture a circuit of unitary gates once; ``replay()`` then runs
@@ -307,7 +317,7 @@ class StateVectorSimulator:
         if self._circuit is None or self._vector is None:
             raise qerr.SampleBeforeRunError("StateVectorSimulator sample without run any circuit.")
         n = self._qubits
-        u = np.array([random.random() for _ in range(shots * n)], dtype=np.float64)
+        u = uniforms(shots * n)
         out = np.zeros(shots, dtype=np.uint64)
         rc = self._lib.qs_sv_sample(self._ctx, self._vptr(), n, self._dcode, u.ctypes.data_as(ctypes.c_void_p),
                                     shots, out.ctypes.data_as(ctypes.c_void_p), self._stream())
