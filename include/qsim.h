@@ -117,6 +117,15 @@ int qs_sv_apply_gate(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* ga
 int qs_sv_apply_gates(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates,
                       int fuse, int* passes, void* stream);
 
+/* The same from a start that need not be in the vector: |0...0>, or on 2n bits the
+   2^n x 2^n identity (qs_sv_init or qs_mat_identity, then qs_sv_apply_gates, in one
+   call).  The fused passes neither write the start nor run tiles that are still all
+   zeros: a pass reaches the tile bits of the passes before it, 12 more bits at most. */
+#define QS_START_ZERO 0
+#define QS_START_IDENTITY 1
+int qs_run(qs_ctx* ctx, void* vec, int nbits, int dtype, int start, const qs_gate* gates, int ngates, int fuse,
+           int* passes, void* stream);
+
 /* Fusion tile shape: log2 amplitudes per tile (0 = built-in default 12; also
    11 or 13 for complex128, 13 for complex64) and the number of low bits always
    kept contiguous (0 = 4, or 2..8, at most tile_log2 - 4; checked again when

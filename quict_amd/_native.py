@@ -79,6 +79,7 @@ SIGNATURES = {
     "qs_sv_init": (_I, [_P, _P, _I, _I, _U64, _P]),
     "qs_sv_apply_gate": (_I, [_P, _P, _I, _I, _P, _P]),
     "qs_sv_apply_gates": (_I, [_P, _P, _I, _I, _P, _I, _I, ctypes.POINTER(_I), _P]),
+    "qs_run": (_I, [_P, _P, _I, _I, _I, _P, _I, _I, ctypes.POINTER(_I), _P]),
     "qs_sv_prob_zero": (_I, [_P, _P, _I, _I, _I, ctypes.POINTER(_D), _P]),
     "qs_sv_collapse": (_I, [_P, _P, _I, _I, _I, _I, _D, _P]),
     "qs_sv_reset": (_I, [_P, _P, _I, _I, _I, _D, _P]),
@@ -122,6 +123,8 @@ class QsQnnOp(ctypes.Structure):
 
 
 QS_QNN_RX, QS_QNN_RY, QS_QNN_RZ, QS_QNN_CX, QS_QNN_CZ, QS_QNN_ENC_RY = range(6)
+
+QS_START_ZERO, QS_START_IDENTITY = range(2)
 
 _lib = None
 _lib_lock = threading.Lock()

@@ -500,7 +500,7 @@ int qs_sv_apply_gates(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* g
     if (rc) return rc;
   }
   QS_REQUIRE(fuse >= 0 && fuse <= 2, "fuse must be 0, 1 or 2");
-  if (fuse) return apply_gates_fused(ctx, vec, n, dtype, gates, ngates, passes, as_stream(stream));
+  if (fuse) return apply_gates_fused(ctx, vec, n, dtype, gates, ngates, -1, passes, as_stream(stream));
   for (int i = 0; i < ngates; ++i) {
     rc = prof_begin(ctx, PROF_GATE, as_stream(stream));
     if (rc) return rc;
@@ -511,6 +511,22 @@ int qs_sv_apply_gates(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* g
   }
   if (passes) *passes = ngates;
   return QS_OK;
+}
+
+int qs_run(qs_ctx* ctx, void* vec, int nbits, int dtype, int start, const qs_gate* gates, int ngates, int fuse,
+           int* passes, void* stream) {
+  int rc = check_state_args(vec, nbits, dtype);
+  if (rc) return rc;
+  QS_REQUIRE(ctx, "null ctx");
+  QS_REQUIRE(start == QS_START_ZERO || (start == QS_START_IDENTITY && nbits % 2 == 0), "bad start");
+  QS_REQUIRE(ngates >= 0 && (ngates == 0 || gates), "bad gate list");
+  for (int i = 0; i < ngates; ++i)
+    if ((rc = validate_gate(&gates[i], nbits))) return rc;
+  QS_REQUIRE(fuse >= 0 && fuse <= 2, "fuse must be 0, 1 or 2");
+  if (fuse) return apply_gates_fused(ctx, vec, nbits, dtype, gates, ngates, start, passes, as_stream(stream));
+  rc = start == QS_START_ZERO ? qs_sv_init(ctx, vec, nbits, dtype, 0, stream)
+                              : qs_mat_identity(ctx, vec, nbits / 2, dtype, stream);
+  return rc ? rc : qs_sv_apply_gates(ctx, vec, nbits, dtype, gates, ngates, 0, passes, stream);
 }
 
 int qs_sv_permute(qs_ctx* ctx, const void* vec, void* out, int n, int dtype, const int32_t* perm, void* stream) {

@@ -95,31 +95,54 @@ template <typename R> struct ProgDev {
         C((const cx<R>*)(d + im.hb + im.ob + im.xb)) {}
 };
 
+// Writes what a vector with known zeros has not had written: its start, or the zeros.
+template <typename R>
+__global__ __launch_bounds__(256) void k_rest(cx<R>* __restrict__ v, uint64_t N, uint64_t fixed, uint32_t sh,
+                                              uint32_t fresh) {
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += stride) {
+    const bool zero = ((sh ? i ^ (i >> sh) : i) & fixed) != 0;
+    if (zero || fresh) st(v + i, mk<R>(zero ? (R)0 : (R)1, (R)0));
+  }
+}
+template <typename R> static int write_rest(cx<R>* v, int n, KnownZeros& z, hipStream_t s) {
+  if (!z.fixed) return QS_OK;
+  const uint64_t N = 1ull << n, blocks = std::min<uint64_t>((N + 255) / 256, 1ull << 20);
+  hipLaunchKernelGGL(k_rest<R>, dim3((unsigned)blocks), dim3(256), 0, s, v, N, z.fixed, (uint32_t)z.sh,
+                     (uint32_t)z.fresh);
+  QS_CHECK_HIP(hipGetLastError());
+  z = KnownZeros();
+  return QS_OK;
+}
+
 // One fused pass: host header hd, its device copy dh.  prof: bracket the
 // launch with the context's timing events (never while capturing a graph).
 template <typename R, int RB, int TB>
 static int launch_fused(qs_ctx* ctx, cx<R>* v, int n, const Config& c, const PassHdr& hd, const PassHdr* dh,
-                        const ProgDev<R>& d, hipStream_t s, bool prof) {
+                        const ProgDev<R>& d, KnownZeros& z, hipStream_t s, bool prof) {
   constexpr int K = RB + TB;
-  const uint64_t tiles = n > K ? 1ull << (n - K) : 1;
+  int rc = QS_OK;
+  // (the kernel that prefetches tiles takes a vector that is there)
+  if (!c.wires && !hd.has_dk && ctx->fused_prefetch && (rc = write_rest(v, n, z, s))) return rc;
+  const PassStart S = enter_pass(z, hd, K, std::max(n, K));
+  const uint64_t tiles = S.fixed ? 1ull << __builtin_popcountll(S.free) : n > K ? 1ull << (n - K) : 1;
   const size_t lds_bytes = (size_t)(1u << (K - 1)) * sizeof(cx<R>);  // half-tile relayout image
   const size_t lds_relayout = hd.uses_lds ? lds_bytes : 0;
   const size_t lds = hd.has_dk && !c.wires ? lds_relayout : lds_relayout + (size_t)hd.nstage * sizeof(cx<R>);
-  int rc = QS_OK;
   if (prof && (rc = prof_begin(ctx, PROF_FUSED, s))) return rc;
   if (c.wires) {
-    launch_wires<R, RB, TB>(v, tiles, hd, dh, (const WireOp<R>*)d.O, d.C, d.X, n < K ? 1u << n : 0u, lds, s);
+    launch_wires<R, RB, TB>(v, tiles, hd, dh, (const WireOp<R>*)d.O, d.C, d.X, n < K ? 1u << n : 0u, S, lds, s);
   } else if (hd.has_dk) {
     hipLaunchKernelGGL((k_fused<R, RB, TB, true, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, d.O,
-                       d.C, d.X, tiles);
+                       d.C, d.X, tiles, S);
   } else if (ctx->fused_prefetch) {
     // persistent, prefetching: resident workgroups only
     const uint64_t grid = std::min<uint64_t>(tiles, (uint64_t)ctx->num_cus * ctx->fused_wg_per_cu);
     hipLaunchKernelGGL((k_fused<R, RB, TB, false, true>), dim3((unsigned)grid), dim3(1 << TB), lds, s, v, dh, d.O,
-                       d.C, d.X, tiles);
+                       d.C, d.X, tiles, S);
   } else {
     hipLaunchKernelGGL((k_fused<R, RB, TB, false, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, d.O,
-                       d.C, d.X, tiles);
+                       d.C, d.X, tiles, S);
   }
   QS_CHECK_HIP(hipGetLastError());
   if (prof && (rc = prof_end(ctx, s))) return rc;
@@ -128,8 +151,9 @@ static int launch_fused(qs_ctx* ctx, cx<R>* v, int n, const Config& c, const Pas
 
 // A pass the tile kernel cannot take: the gate's own kernel.
 template <typename R>
-static int launch_single(qs_ctx* ctx, cx<R>* v, int n, const qs_gate& g, hipStream_t s, bool prof) {
-  int rc = QS_OK;
+static int launch_single(qs_ctx* ctx, cx<R>* v, int n, const qs_gate& g, KnownZeros& z, hipStream_t s, bool prof) {
+  int rc = write_rest(v, n, z, s);
+  if (rc) return rc;
   if (prof && (rc = prof_begin(ctx, PROF_GATE, s))) return rc;
   rc = apply_gate(ctx, v, n, sizeof(R) == 8 ? QS_C128 : QS_C64, &g, s);
   if (rc) return rc;
@@ -140,21 +164,21 @@ static int launch_single(qs_ctx* ctx, cx<R>* v, int n, const qs_gate& g, hipStre
 // Launch every pass of `prog` (image at dprog) on stream s.
 template <typename R, int RB, int TB>
 static int launch_passes(qs_ctx* ctx, cx<R>* v, int n, const Config& c, const FusedProgram& prog, const char* dprog,
-                         const ProgImage& im, hipStream_t s, bool prof, int* npass_out) {
+                         const ProgImage& im, KnownZeros z, hipStream_t s, bool prof, int* npass_out) {
   const ProgDev<R> d(dprog, im);
   int npass = 0, rc = QS_OK;
   for (size_t i = 0; i < prog.plans.size(); ++i) {
     if (!prog.plans[i].fused) {
-      rc = launch_single<R>(ctx, v, n, prog.pgates[prog.plans[i].single], s, prof);
+      rc = launch_single<R>(ctx, v, n, prog.pgates[prog.plans[i].single], z, s, prof);
     } else {
       const int h = prog.hdr_of[i];
-      rc = launch_fused<R, RB, TB>(ctx, v, n, c, prog.hdrs[h], d.H + h, d, s, prof);
+      rc = launch_fused<R, RB, TB>(ctx, v, n, c, prog.hdrs[h], d.H + h, d, z, s, prof);
     }
     if (rc) return rc;
     ++npass;
   }
   if (npass_out) *npass_out = npass;
-  return QS_OK;
+  return write_rest(v, n, z, s);
 }
 
 // A gate that does not keep the norm: a noise channel's superoperator.
@@ -197,7 +221,7 @@ static Config fused_config(int RB, int TB, int L, const qs_gate* gates, int ngat
 // always schedules).
 template <typename R, int RB, int TB>
 static int run_fused_streamed(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int ngates, const Config& c,
-                              int* passes, hipStream_t s) {
+                              KnownZeros z, int* passes, hipStream_t s) {
   FusedProgram prog;
   int npass = 0;
   auto chunk = [&](const FusedProgram& sub, int) -> int {
@@ -210,30 +234,30 @@ static int run_fused_streamed(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates
     QS_CHECK_HIP(hipMemcpyAsync(slot->dev, slot->host, im.host.size(), hipMemcpyHostToDevice, s));
     const ProgDev<R> d((const char*)slot->dev, im);
     for (size_t h = 0; h < sub.hdrs.size() && !rc; ++h, ++npass)
-      rc = launch_fused<R, RB, TB>(ctx, v, n, c, sub.hdrs[h], d.H + h, d, s, true);
+      rc = launch_fused<R, RB, TB>(ctx, v, n, c, sub.hdrs[h], d.H + h, d, z, s, true);
     QS_CHECK_HIP(hipEventRecord(slot->done, s));
     slot->pending = true;
     return rc;
   };
   auto single = [&](const qs_gate& g) -> int {
     ++npass;
-    return launch_single<R>(ctx, v, n, g, s, true);
+    return launch_single<R>(ctx, v, n, g, z, s, true);
   };
   int rc = build_streamed(gates, ngates, n, c, (uint32_t)sizeof(cx<R>), prog, chunk, single);
   if (!rc)
     if (const char* dbg = getenv("QS_FUSION_DEBUG"))
       if (dbg[0] == '1') print_program_stats(prog, n, RB + TB, c.L, ngates);
   if (passes) *passes = npass;
-  return rc;
+  return rc ? rc : write_rest(v, n, z, s);
 }
 
 template <typename R, int RB, int TB>
-static int run_fused_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int ngates, int L, int* passes,
+static int run_fused_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int ngates, int L, KnownZeros z, int* passes,
                        hipStream_t s) {
   const Config c = fused_config(RB, TB, L, gates, ngates);
   if (c.remap == 0) {  // passes are final as they form: streamed
     const char* st = getenv("QS_FUSION_STREAM");
-    if (!(st && st[0] == '0')) return run_fused_streamed<R, RB, TB>(ctx, v, n, gates, ngates, c, passes, s);
+    if (!(st && st[0] == '0')) return run_fused_streamed<R, RB, TB>(ctx, v, n, gates, ngates, c, z, passes, s);
   }
   FusedProgram prog;
   int rc = build_program(gates, ngates, n, c, (uint32_t)sizeof(cx<R>), prog);
@@ -252,7 +276,7 @@ static int run_fused_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int n
     std::memcpy(slot->host, im.host.data(), im.host.size());
     QS_CHECK_HIP(hipMemcpyAsync(dprog, slot->host, im.host.size(), hipMemcpyHostToDevice, s));
   }
-  rc = launch_passes<R, RB, TB>(ctx, v, n, c, prog, dprog, im, s, true, passes);
+  rc = launch_passes<R, RB, TB>(ctx, v, n, c, prog, dprog, im, z, s, true, passes);
   QS_CHECK_HIP(hipEventRecord(slot->done, s));
   slot->pending = true;
   return rc;
@@ -270,12 +294,6 @@ struct qs_graph {
 };
 
 namespace qs {
-
-template <typename R> __global__ __launch_bounds__(256) void k_basis0(cx<R>* __restrict__ v, uint64_t N) {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += stride)
-    st(v + i, mk<R>(i == 0 ? (R)1 : (R)0, (R)0));
-}
 
 template <typename R, int RB, int TB>
 static int capture_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int ngates, int L, int init_zero,
@@ -310,13 +328,9 @@ static int capture_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int nga
     set_error(std::string("hipStreamBeginCapture: ") + hipGetErrorString(e));
     return QS_ERR_DEVICE;
   }
-  if (init_zero) {
-    const uint64_t N = 1ull << n;
-    const uint64_t blocks = std::min<uint64_t>((N + 255) / 256, 1ull << 20);
-    hipLaunchKernelGGL(k_basis0<R>, dim3((unsigned)blocks), dim3(256), 0, s, v, N);
-  }
   int npass = 0;
-  rc = launch_passes<R, RB, TB>(ctx, v, n, c, prog, (const char*)G->dprog, im, s, false, &npass);
+  rc = launch_passes<R, RB, TB>(ctx, v, n, c, prog, (const char*)G->dprog, im, init_zero ? known_start(n, 0) : KnownZeros(), s, false,
+                                &npass);
   hipGraph_t graph = nullptr;
   e = hipStreamEndCapture(s, &graph);
   (void)hipStreamDestroy(s);
@@ -349,13 +363,13 @@ template <typename R, int RB, int TB> static void set_lds_attr() {
 }
 
 static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates,
-                                  int* passes, hipStream_t s);
+                                  int start, int* passes, hipStream_t s);
 
 // The planner is host C++: no exception may cross the C ABI.
-int apply_gates_fused(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates, int* passes,
+int apply_gates_fused(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates, int start, int* passes,
                       hipStream_t s) {
   try {
-    return apply_gates_fused_impl(ctx, vec, n, dtype, gates, ngates, passes, s);
+    return apply_gates_fused_impl(ctx, vec, n, dtype, gates, ngates, start, passes, s);
   } catch (const std::exception& e) {
     set_error(std::string("fusion planner: ") + e.what());
     return QS_ERR_DEVICE;
@@ -363,7 +377,7 @@ int apply_gates_fused(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* g
 }
 
 static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates,
-                                  int* passes, hipStream_t s) {
+                                  int start, int* passes, hipStream_t s) {
   // Tile shapes (4 register bits per thread, 2^(K-4) threads, a half-tile LDS
   // image for relayouts): K = 12 by default for both precisions (256 threads;
   // 32 KiB of LDS for complex128, 16 KiB for complex64); complex128 also takes
@@ -378,7 +392,11 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
   // (5 qubits, 100 gates: 508 us a run with a kernel per gate, 247 us so); two gates or
   // fewer are no slower as kernels of their own.  Programs that keep whole gates in
   // the tile (fused_config) need more than one tile's bits.
-  if (ngates == 0 || (n < K + 1 && (ngates < 3 || !fused_config(4, K - 4, L, gates, ngates).wires))) {
+  KnownZeros z = start < 0 ? KnownZeros() : known_start(n, start == QS_START_IDENTITY);
+  const bool per_gate = ngates == 0 || (n < K + 1 && (ngates < 3 || !fused_config(4, K - 4, L, gates, ngates).wires));
+  if (per_gate) {
+    const int rc = dtype == QS_C128 ? write_rest((cx<double>*)vec, n, z, s) : write_rest((cx<float>*)vec, n, z, s);
+    if (rc) return rc;
     for (int i = 0; i < ngates; ++i) {
       int rc = apply_gate(ctx, vec, n, dtype, &gates[i], s);
       if (rc) return rc;
@@ -391,13 +409,13 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
     switch (K) {
       case 11:
         set_lds_attr<double, 4, 7>();
-        return run_fused_t<double, 4, 7>(ctx, v, n, gates, ngates, L, passes, s);
+        return run_fused_t<double, 4, 7>(ctx, v, n, gates, ngates, L, z, passes, s);
       case 12:
         set_lds_attr<double, 4, 8>();
-        return run_fused_t<double, 4, 8>(ctx, v, n, gates, ngates, L, passes, s);
+        return run_fused_t<double, 4, 8>(ctx, v, n, gates, ngates, L, z, passes, s);
       case 13:
         set_lds_attr<double, 4, 9>();
-        return run_fused_t<double, 4, 9>(ctx, v, n, gates, ngates, L, passes, s);
+        return run_fused_t<double, 4, 9>(ctx, v, n, gates, ngates, L, z, passes, s);
       default:
         set_error("complex128 fusion tiles: tile_log2 must be 11, 12 or 13");
         return QS_ERR_UNSUPPORTED;
@@ -407,10 +425,10 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
   switch (K) {
     case 12:
       set_lds_attr<float, 4, 8>();
-      return run_fused_t<float, 4, 8>(ctx, v, n, gates, ngates, L, passes, s);
+      return run_fused_t<float, 4, 8>(ctx, v, n, gates, ngates, L, z, passes, s);
     case 13:
       set_lds_attr<float, 4, 9>();
-      return run_fused_t<float, 4, 9>(ctx, v, n, gates, ngates, L, passes, s);
+      return run_fused_t<float, 4, 9>(ctx, v, n, gates, ngates, L, z, passes, s);
     default:
       set_error("complex64 fusion tiles: tile_log2 must be 12 or 13");
       return QS_ERR_UNSUPPORTED;

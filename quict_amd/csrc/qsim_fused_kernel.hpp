@@ -470,13 +470,21 @@ __device__ __forceinline__ void run_ops(cx<R> (&a)[1 << RB], char* lds, const Pa
   }
 }
 
-// One pass over all 2^(n-K) tiles.  PF: persistent workgroups that prefetch
+// Its amplitude a, 0 or 1 where that is known.
+template <typename R>
+__device__ __forceinline__ cx<R> start_load(const PassStart& S, const cx<R>* __restrict__ v, uint64_t a) {
+  const uint64_t t = S.sh ? a ^ (a >> S.sh) : a;
+  if (t & S.fixed) return mk<R>((R)0, (R)0);
+  return S.fresh ? mk<R>((R)1, (R)0) : ld_nt(v + a);
+}
+
+// One pass over all 2^(n-K) tiles, or those that hold anything (S).  PF: persistent workgroups that prefetch
 // the next tile into a second register set while the current one is computed
 // (grid = resident workgroups); otherwise one tile per workgroup.
 template <typename R, int RB, int TB, bool DK, bool PF>
 __global__ __launch_bounds__(1 << TB) void k_fused(cx<R>* __restrict__ v, const PassHdr* __restrict__ H,
                                                    const FOpW* __restrict__ ops, const cx<R>* __restrict__ coef,
-                                                   const uint32_t* __restrict__ aux, uint64_t ntiles) {
+                                                   const uint32_t* __restrict__ aux, uint64_t ntiles, const PassStart S) {
   constexpr int NR = 1 << RB;
   constexpr int K = RB + TB;
   extern __shared__ __align__(16) char lds_raw[];
@@ -500,7 +508,9 @@ __global__ __launch_bounds__(1 << TB) void k_fused(cx<R>* __restrict__ v, const 
     // One tile per workgroup, straight-line: the store address is derived from
     // the header after the ops, so only the tile base stays live across them
     // (the op interpreter needs every scalar register it can get).
-    const uint64_t tb = insert_zeros((uint64_t)blockIdx.x, H->sorted, K);
+    uint32_t number;
+    const uint64_t tb =
+        S.fixed ? start_tile(S, blockIdx.x, H->sorted, K, number) : insert_zeros((uint64_t)blockIdx.x, H->sorted, K);
     {
       uint64_t gin = 0;
 #pragma unroll
@@ -515,7 +525,7 @@ __global__ __launch_bounds__(1 << TB) void k_fused(cx<R>* __restrict__ v, const 
 #pragma unroll
         for (int b = 0; b < RB; ++b)
           if ((r >> b) & 1) g |= min_[b];
-        a[r] = ld_nt(v + (base | g));
+        a[r] = S.fixed ? start_load(S, v, base | g) : ld_nt(v + (base | g));
       }
     }
     run_ops<R, RB, TB, DK, !DK>(a, lds_raw, H, P, C, coef + H->coef0, aux, tid);

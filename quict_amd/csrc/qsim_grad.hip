@@ -633,7 +633,7 @@ static int adjoint_t(qs_ctx* ctx, cx<R>* psi, cx<R>* lam, int n, const qs_gate* 
     // the forward state by the fused passes, before this call takes a program
     // slot (their uploads cycle through the slots)
     rc = qs_sv_init(ctx, psi, n, dt, 0, s);
-    if (!rc) rc = apply_gates_fused(ctx, psi, n, dt, fwd, ngates, nullptr, s);
+    if (!rc) rc = apply_gates_fused(ctx, psi, n, dt, fwd, ngates, -1, nullptr, s);
     if (rc) return rc;
   }
   // Every device buffer of the call lives in one pinned program slot, sized

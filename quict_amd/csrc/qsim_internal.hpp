@@ -23,7 +23,8 @@ int validate_gate(const qs_gate* g, int n);
 int apply_gate(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* g, hipStream_t s);
 
 // Fused multi-gate passes (qsim_fused.hip).
-int apply_gates_fused(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates, int* passes,
+// start: QS_START_*, or -1: what the vector holds.
+int apply_gates_fused(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates, int start, int* passes,
                       hipStream_t s);
 
 // Double-precision reductions (qsim_measure.hip).

@@ -342,6 +342,23 @@ __device__ __forceinline__ void wire_load(cx<R> (&a)[NV][1 << RB], const cx<R>* 
     }
 }
 
+// The same for a vector with known zeros.
+template <typename R, int RB, int TB>
+__device__ __forceinline__ void wire_load_start(cx<R> (&a)[1 << RB], const cx<R>* v, const PassHdr* __restrict__ H,
+                                                const PassStart& S, uint64_t tb, uint32_t tid) {
+  uint64_t base = tb;
+#pragma unroll
+  for (int b = 0; b < TB; ++b) base |= (uint64_t)((tid >> b) & 1u) << H->tbits[H->ts0[b]];
+#pragma unroll
+  for (int r = 0; r < 1 << RB; ++r) {
+    uint64_t g = 0;
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      if ((r >> b) & 1) g |= 1ull << H->tbits[H->rs0[b]];
+    a[r] = start_load(S, v, base | g);
+  }
+}
+
 // Store: per-lane and per-register address bits, flips that depend on the tile.
 template <typename R, int RB, int TB, int NV>
 __device__ __forceinline__ void wire_store(const cx<R> (&a)[NV][1 << RB], cx<R>* const (&v)[NV],
@@ -416,14 +433,17 @@ __device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, 
 template <typename R, int RB, int TB, bool HEAVY>
 __global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k_wires(
     cx<R>* __restrict__ v, const PassHdr* __restrict__ H, const WireOp<R>* __restrict__ ops, const cx<R>* __restrict__ coef,
-    const uint32_t* __restrict__ aux, uint32_t nsmall) {
+    const uint32_t* __restrict__ aux, uint32_t nsmall, const PassStart S) {
   extern __shared__ __align__(16) char lds_raw[];
-  const uint32_t tid = threadIdx.x, blk = blockIdx.x;
+  const uint32_t tid = threadIdx.x;
+  uint32_t blk = blockIdx.x;
   cx<R> a[1][1 << RB];
-  const uint64_t tb = insert_zeros((uint64_t)blk, H->sorted, RB + TB);
+  const uint64_t tb =
+      S.fixed ? start_tile(S, blockIdx.x, H->sorted, RB + TB, blk) : insert_zeros((uint64_t)blk, H->sorted, RB + TB);
   uint32_t seen = 0;
   touch_pass<R, TB>(H, ops, aux, tid, seen);
-  wire_load<R, RB, TB, 1>(a, {v}, H, tb, tid, nsmall);
+  if (S.fixed) wire_load_start<R, RB, TB>(a[0], v, H, S, tb, tid);
+  else wire_load<R, RB, TB, 1>(a, {v}, H, tb, tid, nsmall);
   asm volatile("" ::"v"(seen));
   wire_ops<R, RB, TB, 1, HEAVY>(a, lds_raw, H, ops, coef, aux, tid, blk);
   if (H->sync_store) __syncthreads();

@@ -10,13 +10,13 @@ namespace qs {
 
 template <typename R, int RB, int TB>
 void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const WireOp<R>* ops, const cx<R>* coef,
-                  const uint32_t* aux, uint32_t nsmall, size_t lds, hipStream_t s) {
+                  const uint32_t* aux, uint32_t nsmall, const PassStart& S, size_t lds, hipStream_t s) {
   if (hd.has_dk)
     hipLaunchKernelGGL((k_wires<R, RB, TB, true>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef, aux,
-                       nsmall);
+                       nsmall, S);
   else
     hipLaunchKernelGGL((k_wires<R, RB, TB, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, ops, coef,
-                       aux, nsmall);
+                       aux, nsmall, S);
 }
 
 template <typename R, int RB, int TB> void wires_lds_attr() {
@@ -51,7 +51,7 @@ template void launch_jobs<float>(cx<float>*, cx<float>*, const char*, const Wire
 
 #define QS_WIRES(R, TB)                                                                                          \
   template void launch_wires<R, 4, TB>(cx<R>*, uint64_t, const PassHdr&, const PassHdr*, const WireOp<R>*,       \
-                                       const cx<R>*, const uint32_t*, uint32_t, size_t, hipStream_t);            \
+                                       const cx<R>*, const uint32_t*, uint32_t, const PassStart&, size_t, hipStream_t); \
   template void wires_lds_attr<R, 4, TB>();
 QS_WIRES(double, 7)
 QS_WIRES(double, 8)

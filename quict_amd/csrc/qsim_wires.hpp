@@ -136,7 +136,7 @@ void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs
 // program's device arrays; nsmall: amplitudes of a register below a tile, else 0.  The caller checks hipGetLastError().
 template <typename R, int RB, int TB>
 void launch_wires(cx<R>* v, uint64_t tiles, const PassHdr& hd, const PassHdr* dh, const WireOp<R>* ops, const cx<R>* coef,
-                  const uint32_t* aux, uint32_t nsmall, size_t lds, hipStream_t s);
+                  const uint32_t* aux, uint32_t nsmall, const PassStart& S, size_t lds, hipStream_t s);
 // Lets the kernels take their largest LDS allocation (once per process).
 template <typename R, int RB, int TB> void wires_lds_attr();
 

@@ -173,6 +173,7 @@ class DensityMatrixSimulator:
         self._accumulated_mode = accumulated_mode
         self._fusion = fusion
         self._density_matrix = None
+        self._start = False   # rho stands for |0...0><0...0|, which is not written yet
         self._circuit = None
         self._noise_model = None
         self.last_passes = 0
@@ -197,9 +198,16 @@ class DensityMatrixSimulator:
         self._qubits = int(circuit.width())
 
     def initial_density_matrix(self, qubits: int):
-        D = 1 << qubits
-        self._density_matrix = self._torch.zeros(D * D, dtype=self._tdtype, device=f"cuda:{self._device_id}")
-        self._density_matrix[0] = 1
+        self._density_matrix = self._torch.empty(1 << (2 * qubits), dtype=self._tdtype,
+                                                 device=f"cuda:{self._device_id}")
+        self._start = True
+        self._write_start(qubits)
+
+    def _write_start(self, qubits: int):
+        if self._start:
+            self._start = False
+            nat.check(self._lib.qs_sv_init(self._ctx, self._rptr(), 2 * qubits, self._dcode, 0, self._stream()),
+                      "qs_sv_init")
 
     def check_matrix(self, matrix) -> bool:
         """density_matrix_simulator.py:70-86: Hermitian, PSD, unit trace."""
@@ -223,9 +231,14 @@ class DensityMatrixSimulator:
                                                          device=f"cuda:{self._device_id}")
         elif self._density_matrix is None or not use_previous or \
                 self._density_matrix.numel() != (1 << (2 * self._qubits)):
-            self.initial_density_matrix(self._qubits)
+            self._density_matrix = self._torch.empty(1 << (2 * self._qubits), dtype=self._tdtype,
+                                                     device=f"cuda:{self._device_id}")
+            self._start = True
         self.last_passes = 0
-        self._run(self._circuit)
+        try:
+            self._run(self._circuit)
+        finally:
+            self._write_start(self._qubits)
         if noise_model is not None:
             noise_model.apply_readout_error(circuit.qubits)
         self._torch.cuda.synchronize(self._device_id)
@@ -241,9 +254,12 @@ class DensityMatrixSimulator:
                 return
             arr = prog.array()
             passes = ctypes.c_int(0)
-            rc = self._lib.qs_sv_apply_gates(self._ctx, self._rptr(), 2 * n, self._dcode, nat.gate_array_ptr(arr),
-                                             len(arr), 1 if self._fusion else 0, ctypes.byref(passes),
-                                             self._stream())
+            args = (nat.gate_array_ptr(arr), len(arr), 1 if self._fusion else 0, ctypes.byref(passes), self._stream())
+            if self._start:
+                rc = self._lib.qs_run(self._ctx, self._rptr(), 2 * n, self._dcode, nat.QS_START_ZERO, *args)
+                self._start = rc != nat.QS_OK
+            else:
+                rc = self._lib.qs_sv_apply_gates(self._ctx, self._rptr(), 2 * n, self._dcode, *args)
             nat.check(rc, "qs_sv_apply_gates(density matrix)")
             self.last_passes += passes.value
             prog = _Program(n)
@@ -251,6 +267,7 @@ class DensityMatrixSimulator:
         for g in circuit.gates:
             if isinstance(g, BasicGate) and g.type == GateType.measure:
                 flush()
+                self._write_start(n)
                 self.apply_measure(g.targ)
             elif isinstance(g, BasicGate) and g.type in (GateType.reset, GateType.perm):
                 raise qerr.GateTypeNotImplementError(f"{g.type.name} in the density-matrix simulator")

@@ -88,6 +88,7 @@ class StateVectorSimulator:
         self._using_matrix_aggregation = matrix_aggregation  # accepted; matrices travel inline in gate records
         self._circuit: Optional[Circuit] = None
         self._vector = None
+        self._start = False   # the vector stands for |0...0>, which is not written yet
         self._qubits = 0
         self.last_passes = 0
         self._ctx = nat.context(gpu_device_id)
@@ -154,14 +155,31 @@ class StateVectorSimulator:
                 raise qerr.StateVectorUnmatchedError("the state vector must have 2^width amplitudes")
             self.vector = sv
         elif not use_previous or self._vector is None or self._vector.numel() != (1 << self._qubits):
-            self.initial_state_vector()
+            self._vector = self._torch.empty(1 << self._qubits, dtype=self._tdtype, device=f"cuda:{self._device_id}")
+            self._start = True
         self.last_passes = 0
+        try:
+            self._run_pipeline()
+        finally:
+            self._write_start()
+        if self._sync:
+            self._torch.cuda.synchronize(self._device_id)
+        return self.vector
+
+    def _write_start(self):
+        if self._start:
+            self._start = False
+            nat.check(self._lib.qs_sv_init(self._ctx, self._vptr(), self._qubits, self._dcode, 0, self._stream()),
+                      "qs_sv_init")
+
+    def _run_pipeline(self):
         idx = 0
         while idx < len(self._pipeline):
             end = self._run_of_gates(idx)
             self._flush(self._pipeline[idx:end])
             if end == len(self._pipeline):
                 break
+            self._write_start()
             op = self._pipeline[end]
             idx = end + 1
             if isinstance(op, Trigger):
@@ -170,9 +188,6 @@ class StateVectorSimulator:
                 self.apply_gate(op)
             else:
                 raise qerr.TypeError("StateVectorSimulator.run takes BasicGate / Trigger, got", type(op))
-        if self._sync:
-            self._torch.cuda.synchronize(self._device_id)
-        return self.vector
 
     def _run_of_gates(self, idx: int) -> int:
         """End of the run of unitary gates that starts at pipeline position ``idx``."""
@@ -212,9 +227,12 @@ class StateVectorSimulator:
         if len(recs) == 0:
             return
         passes = ctypes.c_int(0)
-        rc = self._lib.qs_sv_apply_gates(self._ctx, self._vptr(), self._qubits, self._dcode,
-                                         nat.gate_array_ptr(recs), len(recs), 2 if self._fusion else 0,
-                                         ctypes.byref(passes), self._stream())
+        args = (nat.gate_array_ptr(recs), len(recs), 2 if self._fusion else 0, ctypes.byref(passes), self._stream())
+        if self._start:
+            rc = self._lib.qs_run(self._ctx, self._vptr(), self._qubits, self._dcode, nat.QS_START_ZERO, *args)
+            self._start = rc != nat.QS_OK
+        else:
+            rc = self._lib.qs_sv_apply_gates(self._ctx, self._vptr(), self._qubits, self._dcode, *args)
         del keep
         nat.check(rc, "qs_sv_apply_gates")
         self.last_passes += passes.value

@@ -59,13 +59,11 @@ def build_columns(gates, n: int, dtype_code: int, device_id: int = 0, fusion: bo
         raise qerr.ValueError("circuit matrix width must be in [1, 20], got", n)
     tdt = torch.complex128 if dtype_code == nat.QS_C128 else torch.complex64
     W = torch.empty(1 << (2 * n), dtype=tdt, device=f"cuda:{device_id}")
-    nat.check(lib.qs_mat_identity(ctx, ctypes.c_void_p(W.data_ptr()), n, dtype_code, stream), "qs_mat_identity")
     recs, keep = compile_gates(_unitary_gates(gates), n)
     passes = ctypes.c_int(0)
-    if len(recs):
-        rc = lib.qs_sv_apply_gates(ctx, ctypes.c_void_p(W.data_ptr()), 2 * n, dtype_code, nat.gate_array_ptr(recs),
-                                   len(recs), 1 if fusion else 0, ctypes.byref(passes), stream)
-        nat.check(rc, "qs_sv_apply_gates(circuit matrix)")
+    nat.check(lib.qs_run(ctx, ctypes.c_void_p(W.data_ptr()), 2 * n, dtype_code, nat.QS_START_IDENTITY,
+                         nat.gate_array_ptr(recs), len(recs), 1 if fusion else 0, ctypes.byref(passes), stream),
+              "qs_run(circuit matrix)")
     del keep
     return W, passes.value
 

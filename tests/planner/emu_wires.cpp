@@ -41,21 +41,25 @@ static void dense(zc* A, int NR, const int* pos, int k, const zc* M, const FOp& 
 }
 
 static void wire_pass(zc* v, int n, int RB, int TB, uint32_t S, const PassHdr& H, const FOp* P, const double* Cd,
-                      const uint32_t* X) {
+                      const uint32_t* X, const PassStart& known = PassStart{}) {
   const int NR = 1 << RB, NT = 1 << TB, K = RB + TB;
   std::vector<zc> a((size_t)NT * NR), lds((size_t)NT * NR), out((size_t)NT * NR);
   std::vector<int> written((size_t)NT * NR);
   auto cz = [&](int i) { return zc(Cd[2 * i], Cd[2 * i + 1]); };
   // a register below a tile: the amplitudes it lacks are zeros and not stored
   const uint64_t N = 1ull << n;
-  for (uint64_t t = 0; t < (n > K ? 1ull << (n - K) : 1); ++t) {
-    const uint64_t tb = insert_zeros(t, H.sorted, K);
+  const uint64_t tiles = known.fixed ? 1ull << __builtin_popcountll(known.free) : n > K ? 1ull << (n - K) : 1;
+  for (uint64_t i = 0; i < tiles; ++i) {
+    uint32_t number = (uint32_t)i;
+    const uint64_t tb = known.fixed ? start_tile(known, i, H.sorted, K, number) : insert_zeros(i, H.sorted, K);
+    const uint64_t t = number;
     for (int tid = 0; tid < NT; ++tid)
       for (int r = 0; r < NR; ++r) {
         uint64_t g = tb;
         for (int b = 0; b < TB; ++b) g |= (uint64_t)((tid >> b) & 1) << H.tbits[H.ts0[b]];
         for (int b = 0; b < RB; ++b) g |= (uint64_t)((r >> b) & 1) << H.tbits[H.rs0[b]];
-        a[(size_t)tid * NR + r] = g < N ? v[g] : zc(0);
+        const bool zero = ((known.sh ? g ^ (g >> known.sh) : g) & known.fixed) != 0;
+        a[(size_t)tid * NR + r] = zero || g >= N ? zc(0) : known.fixed && known.fresh ? zc(1) : v[g];
       }
     for (int o = 0; o < H.nops; ++o) {
       const FOp& op = P[o];
@@ -245,6 +249,51 @@ extern "C" int wires_apply(double* vec, int n, const qs_gate* gates, int ngates,
     for (const PassHdr& h : prog.hdrs) stats[7] = std::max(stats[7], h.nstage);
     if (getenv("QS_FUSION_DEBUG")) print_program_stats(prog, n, RB + TB, L, ngates);
     return 0;
+  } catch (const std::exception& e) {
+    g_err = e.what();
+    return -99;
+  }
+}
+
+// The program from |0...0> (identity: from the identity matrix on n = 2m bits), vec
+// holding anything before: as the launches do, with what is known to be zero neither
+// read nor computed.  stats: passes, tiles run, tiles there are.
+extern "C" int wires_run(double* vec, int n, int identity, const qs_gate* gates, int ngates, int RB, int TB, int L,
+                         int amp_bytes, int64_t* stats) {
+  using namespace qs;
+  try {
+    Config c{RB, TB, L};
+    c.wires = true;
+    FusedProgram prog;
+    const int K = RB + TB;
+    KnownZeros z = known_start(n, identity);
+    std::fill(stats, stats + 3, 0);
+    zc* v = reinterpret_cast<zc*>(vec);
+    auto rest = [&]() {
+      for (uint64_t i = 0; z.fixed && i < 1ull << n; ++i) {
+        const bool zero = ((z.sh ? i ^ (i >> z.sh) : i) & z.fixed) != 0;
+        if (zero || z.fresh) v[i] = zero ? 0.0 : 1.0;
+      }
+      z = KnownZeros();
+    };
+    auto chunk = [&](const FusedProgram& sub, int) -> int {
+      for (const PassHdr& H : sub.hdrs) {
+        const PassStart S = enter_pass(z, H, K, std::max(n, K));
+        ++stats[0];
+        stats[1] += S.fixed ? 1ll << __builtin_popcountll(S.free) : n > K ? 1ll << (n - K) : 1;
+        stats[2] += n > K ? 1ll << (n - K) : 1;
+        wire_pass(v, n, RB, TB, (uint32_t)amp_bytes, H, sub.ops.data() + H.op0, sub.coef.data() + 2 * (size_t)H.coef0,
+                  sub.aux.data(), S);
+      }
+      return 0;
+    };
+    auto single = [&](const qs_gate& g) -> int {
+      rest();
+      return cpu_apply_gates(vec, n, &g, 1, 1);
+    };
+    const int rc = build_streamed(gates, ngates, n, c, (uint32_t)amp_bytes, prog, chunk, single);
+    rest();
+    return rc;
   } catch (const std::exception& e) {
     g_err = e.what();
     return -99;
