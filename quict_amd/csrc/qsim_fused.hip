@@ -64,15 +64,15 @@ template <typename R> static void pack_program(const FusedProgram& prog, const C
   im.cb = al(ncoef * sizeof(cx<R>));
   im.host.assign(im.hb + im.ob + im.xb + im.cb, 0);
   char* h = im.host.data();
-  if (!prog.hdrs.empty()) std::memcpy(h, prog.hdrs.data(), prog.hdrs.size() * sizeof(PassHdr));
+  PassHdr* hd = reinterpret_cast<PassHdr*>(h);
+  for (size_t i = 0; i < prog.hdrs.size(); ++i) std::memcpy(hd + i, &prog.hdrs[i], sizeof(PassHdr));
   if (c.wires) {
     WireOp<R>* w = reinterpret_cast<WireOp<R>*>(h + im.hb);
-    for (const PassHdr& H : prog.hdrs)
-      for (int i = H.op0; i < H.op0 + H.nops; ++i) {
-        const bool payload = prog.ops[i].kind == F_ROT || prog.ops[i].kind == F_PHASE;
-        w[i] = encode_wire_op<R>(prog.ops[i],
-                                 payload ? prog.coef.data() + 2 * ((size_t)H.coef0 + prog.ops[i].coef) : nullptr);
-      }
+    for (size_t i = 0; i < prog.hdrs.size(); ++i) {
+      const PassHdr& H = prog.hdrs[i];
+      hd[i].nops = encode_wire_pass<R>(prog.ops.data() + H.op0, H.nops, prog.coef.data() + 2 * (size_t)H.coef0, w + H.op0,
+                                       nullptr);
+    }
   } else {
     for (size_t i = 0; i < prog.ops.size(); ++i) {
       const FOpW e = encode_op(prog.ops[i]);

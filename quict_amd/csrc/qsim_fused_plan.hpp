@@ -99,6 +99,8 @@ static bool wire_heavy(const FOp& o) {
       return true;
     case F_DENSE1:
       return o.creg != 0 || o.cthr != 0;
+    case F_PHASE:
+      return o.pure == 0;
     case F_PERM1:
       return !o.pure || (o.creg != 0 && (o.cthr != 0 || __builtin_popcount(o.creg) != 1 || o.cregv != o.creg));
     default:

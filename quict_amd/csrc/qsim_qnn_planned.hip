@@ -13,7 +13,7 @@
 // product state.
 //
 // What bounds it: f64 vector work of the two-vector passes.  1024 circuits of 8..18
-// qubits, 6 layers: 78.3 -> 8.1 ms against one persistent workgroup a circuit at a
+// qubits, 6 layers: 78.3 -> 7.0 ms against one persistent workgroup a circuit at a
 // time (k_qnn), which swept the state w / 2 times a layer forward and w / 2 back, in LDS
 // up to 11 qubits and in memory above; here 18 qubits take 4 passes forward and 3 back.
 #include "qsim_internal.hpp"

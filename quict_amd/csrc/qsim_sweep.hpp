@@ -61,13 +61,14 @@ class VarImage {
       const FusedProgram& p = prog[d];
       for (size_t h = 0; h < p.hdrs.size(); ++h) {
         PassHdr H = p.hdrs[h];
-        for (int i = 0; i < H.nops; ++i) {
-          FOp o = p.ops[H.op0 + i];
-          if (o.sym) refs.push_back({o0 + (uint32_t)(H.op0 + i), o.sym - 1, o.sgn, o.kind == F_ROT, o.creg});
+        std::vector<FOp> ops(p.ops.begin() + H.op0, p.ops.begin() + H.op0 + H.nops);
+        for (FOp& o : ops)
           if (o.kind == F_RELAYOUT) o.coef += (int)x0;
-          const bool payload = o.kind == F_ROT || o.kind == F_PHASE;
-          op<R>(o0 + (uint64_t)H.op0 + i) =
-              encode_wire_op<R>(o, payload ? p.coef.data() + 2 * ((size_t)H.coef0 + o.coef) : nullptr);
+        std::vector<WirePlace> at;
+        H.nops = encode_wire_pass<R>(ops.data(), H.nops, p.coef.data() + 2 * (size_t)H.coef0, &op<R>(o0 + (uint64_t)H.op0), &at);
+        for (const WirePlace& w : at) {
+          const FOp& o = ops[w.fop];
+          if (o.sym) refs.push_back({o0 + (uint32_t)(H.op0 + w.op), w.which, o.sym - 1, o.sgn, o.kind == F_ROT, w.code, w.minus});
         }
         const int nv = d + 1;
         const size_t image = (size_t)nv * 2048 * sizeof(cx<R>);
@@ -98,19 +99,19 @@ class VarImage {
       } else {
         const int pure = phase_payload_sym(v[2], v[3], r.sgn, p);
         uint32_t& w0 = op<R>(r.op).w[0];
-        w0 = (w0 & ~0xffu) | ((pure == 3 ? WC_PHS : WC_PHR) + r.mask);
+        w0 = (w0 & ~0xffu) | (pure == 3 ? r.minus : r.code);
       }
-      op<R>(r.op).f = mk<R>((R)p[0], (R)p[1]);
+      op<R>(r.op).f[r.which] = mk<R>((R)p[0], (R)p[1]);
     }
   }
 
  private:
   struct Ref {
     uint32_t op;
-    int slot;
+    int which, slot;
     double sgn;
     bool rot;
-    uint32_t mask;
+    uint32_t code, minus;
   };
   std::vector<Ref> refs;
   template <typename R> WireOp<R>& op(uint64_t i) { return reinterpret_cast<WireOp<R>*>(host.data() + ob)[i]; }

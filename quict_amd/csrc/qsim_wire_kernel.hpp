@@ -181,10 +181,10 @@ __device__ __forceinline__ double wave_total(double v) {
   return v;
 }
 
-// This wave's part of Im <lam|P|psi>, P = Z (Y false) or Y on register bit PB, in
-// double for both precisions; lane 63 writes it to its place in the gradient row.
+// This lane's part of Im <lam|P|psi>, P = Z (Y false) or Y on register bit PB, in
+// double for both precisions.
 template <typename R, int NR, int PB, bool Y>
-__device__ __forceinline__ void wo_measure(const cx<R> (&psi)[NR], const cx<R> (&lam)[NR], double* slot, uint32_t tid) {
+__device__ __forceinline__ double measure(const cx<R> (&psi)[NR], const cx<R> (&lam)[NR]) {
   double s0 = 0, s1 = 0;  // two chains
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
@@ -202,8 +202,35 @@ __device__ __forceinline__ void wo_measure(const cx<R> (&psi)[NR], const cx<R> (
       s1 = rfma(-(double)b1.im, (double)a1.re, s1);
     }
   }
-  const double s = wave_total(s0 - s1);
+  return s0 - s1;
+}
+// The wave's part, in lane 63, which writes it to its place in the gradient row.
+template <typename R, int NR, int PB, bool Y>
+__device__ __forceinline__ void wo_measure(const cx<R> (&psi)[NR], const cx<R> (&lam)[NR], double* slot, uint32_t tid) {
+  const double s = wave_total(measure<R, NR, PB, Y>(psi, lam));
   if ((tid & 63) == 63) *slot = s;
+}
+// Column Z, a phase, column Y, a rotation: a parameter pair of a gradient sweep.  The two
+// columns share the steps of their sums: halves of the wave are exchanged first, then
+// lanes 0..31 add up one and 32..63 the other.
+template <typename R, int NR, int P, int MODE>
+__device__ __forceinline__ void wo_back(cx<R> (&psi)[NR], cx<R> (&lam)[NR], cx<R> ph, cx<R> ts, double* slot_z,
+                                        double* slot_y, uint32_t tid) {
+  const double z = measure<R, NR, P, false>(psi, lam);
+  wo_phase<R, NR, 1u << P, MODE>(psi, ph);
+  wo_phase<R, NR, 1u << P, MODE>(lam, ph);
+  const double y = measure<R, NR, P, true>(psi, lam);
+  wo_rot<R, NR, P>(psi, ts);
+  wo_rot<R, NR, P>(lam, ts);
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)__double2loint(z), (uint32_t)__double2loint(y), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)__double2hiint(z), (uint32_t)__double2hiint(y), false, false);
+  double s = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+  s += wave_move<0x111, 0xf>(s);
+  s += wave_move<0x112, 0xf>(s);
+  s += wave_move<0x114, 0xf>(s);
+  s += wave_move<0x118, 0xf>(s);
+  s += wave_move<0x142, 0xa>(s);
+  if ((tid & 31) == 31) *(tid & 32 ? slot_y : slot_z) = s;
 }
 
 // One op on NV vectors (2: psi and lam of a gradient sweep); grad: this wave's column
@@ -218,6 +245,38 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, cons
   const uint32_t cthr = e.w[3] & 0xffff;
   const bool tok = (tid & cthr) == e.w[3] >> 16;
   const cx<R>* g = G + e.w[2];  // uniform payloads, through scalar loads
+#define QS_V(...)                                  \
+  _Pragma("unroll") for (int v = 0; v < NV; ++v) { \
+    __VA_ARGS__;                                   \
+  }
+#define QS_4(X) X(0) X(1) X(2) X(3)
+  if (code < WC_HOT) {
+    switch (code) {
+#define QS_ROT(P) case WC_ROT + P: QS_V(wo_rot<R, NR, P>(a[v], e.f[0])) break;
+      QS_4(QS_ROT)
+#define QS_RP(BASE, MODE, P)                            \
+  case BASE + P:                                        \
+    QS_V(wo_rot<R, NR, P>(a[v], e.f[0]))                \
+    QS_V(wo_phase<R, NR, 1u << P, MODE>(a[v], e.f[1]))  \
+    break;
+#define QS_PR(BASE, MODE, P)                            \
+  case BASE + P:                                        \
+    QS_V(wo_phase<R, NR, 1u << P, MODE>(a[v], e.f[0]))  \
+    QS_V(wo_rot<R, NR, P>(a[v], e.f[1]))                \
+    break;
+#define QS_BW(BASE, MODE, P)                                                                                     \
+  case BASE + P:                                                                                                 \
+    if constexpr (NV == 2)                                                                                       \
+      wo_back<R, NR, P, MODE>(a[0], a[1], e.f[0], e.f[1], grad + (e.w[2] << (TB - 6)), grad + (e.w[5] << (TB - 6)), tid); \
+    else __builtin_unreachable();                                                                                \
+    break;
+#define QS_HOT(P) \
+  QS_RP(WC_RP, 2, P) QS_RP(WC_RPS, 3, P) QS_PR(WC_PR, 2, P) QS_PR(WC_PRS, 3, P) QS_BW(WC_BW, 2, P) QS_BW(WC_BWS, 3, P)
+      QS_4(QS_HOT)
+      default: __builtin_unreachable();
+    }
+    return;
+  }
   switch (code) {
     case WC_RELAYOUT: {
       const uint32_t* x = X + e.w[2];
@@ -231,14 +290,7 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, cons
       }
       break;
     }
-#define QS_V(...)                                  \
-  _Pragma("unroll") for (int v = 0; v < NV; ++v) { \
-    __VA_ARGS__;                                   \
-  }
-#define QS_4(X) X(0) X(1) X(2) X(3)
 #define QS_16(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15)
-#define QS_ROT(P) case WC_ROT + P: QS_V(wo_rot<R, NR, P>(a[v], e.f))  break;
-    QS_4(QS_ROT)
 #define QS_EX(P) case WC_EX + P: QS_V(wo_ex<R, NR, P, -1>(a[v])) break;
     QS_4(QS_EX)
 #define QS_EXT(P) case WC_EXT + P: if (tok) QS_V(wo_ex<R, NR, P, -1>(a[v])) break;
@@ -250,13 +302,11 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, cons
     break;
     QS_16(QS_EXC)
 // lanes whose thread bits fail sit these out: a wave all of whose lanes do skips the op
-#define QS_PH(BASE, MODE, M) case BASE + M: if (tok) QS_V(wo_phase<R, NR, M, MODE>(a[v], e.f)) break;
+#define QS_PH(BASE, MODE, M) case BASE + M: if (tok) QS_V(wo_phase<R, NR, M, MODE>(a[v], e.f[0])) break;
 #define QS_PHR(M) QS_PH(WC_PHR, 2, M)
     QS_16(QS_PHR)
 #define QS_PHS(M) QS_PH(WC_PHS, 3, M)
     QS_16(QS_PHS)
-#define QS_PHC(M) QS_PH(WC_PHC, 0, M)
-    QS_16(QS_PHC)
 #define QS_PHN(M) QS_PH(WC_PHN, 1, M)
     QS_16(QS_PHN)
     case WC_TABLE:
@@ -290,6 +340,8 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, cons
         const uint32_t creg = (e.w[0] >> 8) & 0xff, cregv = (e.w[0] >> 16) & 0xff;
         const bool pure = e.w[5] != 0;
         switch (code) {
+#define QS_PHC(M) QS_PH(WC_PHC, 0, M)
+          QS_16(QS_PHC)
 #define QS_U2G(P) case WC_U2G + P: QS_V(do_dense1<R, NR, P, 3>(a[v], g, creg, cregv, tok)) break;
           QS_4(QS_U2G)
 #define QS_EXG(P)                                                          \
