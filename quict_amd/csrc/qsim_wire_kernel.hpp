@@ -122,8 +122,10 @@ __device__ __forceinline__ void wo_u2(cx<R> (&a)[NR], const cx<R>* m) {
 }
 
 // Relayout in two rounds (see relayout_half) of NV tiles, each through a half-tile
-// image of its own, so that they share the barriers.
-template <typename R, int RB, int TB, int NV, int P>
+// image of its own, so that they share the barriers; or (IMAGES = 1) one after another
+// through the same image: half the LDS, so that a CU holds three workgroups of two
+// complex128 tiles instead of two.
+template <typename R, int RB, int TB, int NV, int IMAGES, int P>
 __device__ __forceinline__ void wire_relayout(cx<R> (&a)[NV][1 << RB], char* lds, const uint32_t* __restrict__ x,
                                               bool tile_flips, uint32_t tid, uint32_t blk) {
   constexpr int NR = 1 << RB;
@@ -144,22 +146,23 @@ __device__ __forceinline__ void wire_relayout(cx<R> (&a)[NV][1 << RB], char* lds
   for (int b = 0; b < RB; ++b) lq[b] = y[b];
   const uint32_t rd = thr_off<TB>(y + RB, tid);
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
+  for (int k = 0; k < 2 * (NV / IMAGES); ++k) {
+    const int v0 = IMAGES == NV ? 0 : k >> 1, v1 = IMAGES == NV ? NV : v0 + 1;
     lds_barrier();
 #pragma unroll
     for (int r = 0; r < NR; ++r)
-      if (((r >> P) & 1) == k) {
+      if (((r >> P) & 1) == (k & 1)) {
         const uint32_t o = w ^ reg_off<RB>(r, lw);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) st_lds<R>(lds + v * image, o, a[v][r]);
+        for (int v = v0; v < v1; ++v) st_lds<R>(lds + (v - v0) * image, o, a[v][r]);
       }
     lds_barrier();
 #pragma unroll
     for (int r = 0; r < NR; ++r)
-      if (((r >> P) & 1) == k) {
+      if (((r >> P) & 1) == (k & 1)) {
         const uint32_t o = rd ^ reg_off<RB>(r, lq);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) a[v][r] = ld_lds<R>(lds + v * image, o);
+        for (int v = v0; v < v1; ++v) a[v][r] = ld_lds<R>(lds + (v - v0) * image, o);
       }
   }
 }
@@ -235,7 +238,7 @@ __device__ __forceinline__ void wo_back(cx<R> (&psi)[NR], cx<R> (&lam)[NR], cx<R
 
 // One op on NV vectors (2: psi and lam of a gradient sweep); grad: this wave's column
 // 0 of the tile's gradient row.
-template <typename R, int RB, int TB, int NV, bool HEAVY>
+template <typename R, int RB, int TB, int NV, int IMAGES, bool HEAVY>
 __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, const WireOp<R>& e, const cx<R>* __restrict__ C,
                                         const cx<R>* __restrict__ G, const uint32_t* __restrict__ X, uint32_t tid,
                                         uint32_t blk, double* grad) {
@@ -282,10 +285,10 @@ __device__ __forceinline__ void wire_op(cx<R> (&a)[NV][1 << RB], char* lds, cons
       const uint32_t* x = X + e.w[2];
       const bool tf = e.w[4] != 0;
       switch (x[0]) {
-        case 0: wire_relayout<R, RB, TB, NV, 0>(a, lds, x, tf, tid, blk); break;
-        case 1: wire_relayout<R, RB, TB, NV, 1>(a, lds, x, tf, tid, blk); break;
-        case 2: wire_relayout<R, RB, TB, NV, 2>(a, lds, x, tf, tid, blk); break;
-        case 3: wire_relayout<R, RB, TB, NV, 3>(a, lds, x, tf, tid, blk); break;
+        case 0: wire_relayout<R, RB, TB, NV, IMAGES, 0>(a, lds, x, tf, tid, blk); break;
+        case 1: wire_relayout<R, RB, TB, NV, IMAGES, 1>(a, lds, x, tf, tid, blk); break;
+        case 2: wire_relayout<R, RB, TB, NV, IMAGES, 2>(a, lds, x, tf, tid, blk); break;
+        case 3: wire_relayout<R, RB, TB, NV, IMAGES, 3>(a, lds, x, tf, tid, blk); break;
         default: __builtin_unreachable();
       }
       break;
@@ -455,7 +458,7 @@ __device__ __forceinline__ void touch_pass(const PassHdr* __restrict__ H, const 
 
 // The ops of a pass on the wave's tiles.  Returns the workgroup's gradient row in LDS
 // (NV = 2): per column one entry a wave.
-template <typename R, int RB, int TB, int NV, bool HEAVY>
+template <typename R, int RB, int TB, int NV, int IMAGES, bool HEAVY>
 __device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, const PassHdr* __restrict__ H,
                                             const WireOp<R>* __restrict__ ops, const cx<R>* __restrict__ coef,
                                             const uint32_t* __restrict__ aux, uint32_t tid, uint32_t blk) {
@@ -463,7 +466,7 @@ __device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, 
   const WireOp<R>* P = ops + H->op0;
   const cx<R>* G = coef + H->coef0;
   // behind the relayout images: diagonal tables (read per lane), the gradient row
-  cx<R>* C = reinterpret_cast<cx<R>*>(lds) + (H->uses_lds ? NV << (K - 1) : 0);
+  cx<R>* C = reinterpret_cast<cx<R>*>(lds) + (H->uses_lds ? IMAGES << (K - 1) : 0);
   if (H->nstage) {
     for (int i = (int)tid; i < H->nstage; i += (int)blockDim.x) C[i] = G[i];
     __syncthreads();
@@ -474,7 +477,7 @@ __device__ __forceinline__ double* wire_ops(cx<R> (&a)[NV][1 << RB], char* lds, 
   WireOp<R> e = P[0];
   for (int o = 0; o < nops; ++o) {
     const WireOp<R> nx = P[o + 1];  // (past the last op: what follows in the program's memory)
-    if ((blk & e.w[6]) == e.w[7]) wire_op<R, RB, TB, NV, HEAVY>(a, lds, e, C, G, aux, tid, blk, grad);
+    if ((blk & e.w[6]) == e.w[7]) wire_op<R, RB, TB, NV, IMAGES, HEAVY>(a, lds, e, C, G, aux, tid, blk, grad);
     e = nx;
   }
   return row;
@@ -497,15 +500,15 @@ __global__ __launch_bounds__(1 << TB, HEAVY ? 2 : sizeof(R) == 8 ? 4 : 7) void k
   if (S.fixed) wire_load_start<R, RB, TB>(a[0], v, H, S, tb, tid);
   else wire_load<R, RB, TB, 1>(a, {v}, H, tb, tid, nsmall);
   asm volatile("" ::"v"(seen));
-  wire_ops<R, RB, TB, 1, HEAVY>(a, lds_raw, H, ops, coef, aux, tid, blk);
+  wire_ops<R, RB, TB, 1, 1, HEAVY>(a, lds_raw, H, ops, coef, aux, tid, blk);
   if (H->sync_store) __syncthreads();
   wire_store<R, RB, TB, 1>(a, {v}, H, tb, tid, blk, nsmall);
 }
 
 // The same for one pass of several programs (jobs), each on its own part of psi (NV
 // = 1) or of psi and lam (NV = 2, with the tile's gradient row).
-template <typename R, int NV, bool HEAVY>
-__global__ __launch_bounds__(256, HEAVY || (NV == 2 && sizeof(R) == 8) ? 2 : NV == 2 ? 3 : sizeof(R) == 8 ? 4 : 7) void k_jobs(
+template <typename R, int NV, int IMAGES, bool HEAVY>
+__global__ __launch_bounds__(256, HEAVY || (IMAGES == 2 && sizeof(R) == 8) ? 2 : NV == 2 ? 3 : sizeof(R) == 8 ? 4 : 7) void k_jobs(
     cx<R>* __restrict__ psi, cx<R>* __restrict__ lam, const char* __restrict__ image, const WireJobs J,
     double* __restrict__ partial) {
   extern __shared__ __align__(16) char lds_raw[];
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(256, HEAVY || (NV == 2 && sizeof(R) == 8) ? 2 : NV 
     wire_load<R, 4, 8, 2>(a, {psi + job.off, lam + job.off}, H, tb, tid, 0);
   }
   asm volatile("" ::"v"(seen));
-  double* row = wire_ops<R, 4, 8, NV, HEAVY>(a, lds_raw, H, ops, reinterpret_cast<const cx<R>*>(image + job.coef), aux,
+  double* row = wire_ops<R, 4, 8, NV, IMAGES, HEAVY>(a, lds_raw, H, ops, reinterpret_cast<const cx<R>*>(image + job.coef), aux,
                                              tid, blk);
   if (H->sync_store || NV == 2) __syncthreads();
   if constexpr (NV == 1) {
