@@ -123,6 +123,8 @@ int qs_sv_apply_gates(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* g
    zeros: a pass reaches the tile bits of the passes before it, 12 more bits at most. */
 #define QS_START_ZERO 0
 #define QS_START_IDENTITY 1
+#define QS_START_ZERO_WHOLE 3 /* |0...0>, planned with whole gates in the tile and no moves: the order of
+                                 rounding that complex64 gradients have had */
 int qs_run(qs_ctx* ctx, void* vec, int nbits, int dtype, int start, const qs_gate* gates, int ngates, int fuse,
            int* passes, void* stream);
 

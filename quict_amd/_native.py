@@ -124,7 +124,7 @@ class QsQnnOp(ctypes.Structure):
 
 QS_QNN_RX, QS_QNN_RY, QS_QNN_RZ, QS_QNN_CX, QS_QNN_CZ, QS_QNN_ENC_RY = range(6)
 
-QS_START_ZERO, QS_START_IDENTITY = range(2)
+QS_START_ZERO, QS_START_IDENTITY, QS_START_ZERO_WHOLE = 0, 1, 3
 
 _lib = None
 _lib_lock = threading.Lock()

@@ -518,13 +518,13 @@ int qs_run(qs_ctx* ctx, void* vec, int nbits, int dtype, int start, const qs_gat
   int rc = check_state_args(vec, nbits, dtype);
   if (rc) return rc;
   QS_REQUIRE(ctx, "null ctx");
-  QS_REQUIRE(start == QS_START_ZERO || (start == QS_START_IDENTITY && nbits % 2 == 0), "bad start");
+  QS_REQUIRE(start == QS_START_ZERO || start == QS_START_ZERO_WHOLE || (start == QS_START_IDENTITY && nbits % 2 == 0), "bad start");
   QS_REQUIRE(ngates >= 0 && (ngates == 0 || gates), "bad gate list");
   for (int i = 0; i < ngates; ++i)
     if ((rc = validate_gate(&gates[i], nbits))) return rc;
   QS_REQUIRE(fuse >= 0 && fuse <= 2, "fuse must be 0, 1 or 2");
   if (fuse) return apply_gates_fused(ctx, vec, nbits, dtype, gates, ngates, start, passes, as_stream(stream));
-  rc = start == QS_START_ZERO ? qs_sv_init(ctx, vec, nbits, dtype, 0, stream)
+  rc = start != QS_START_IDENTITY ? qs_sv_init(ctx, vec, nbits, dtype, 0, stream)
                               : qs_mat_identity(ctx, vec, nbits / 2, dtype, stream);
   return rc ? rc : qs_sv_apply_gates(ctx, vec, nbits, dtype, gates, ngates, 0, passes, stream);
 }

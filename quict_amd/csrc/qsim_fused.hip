@@ -254,7 +254,8 @@ static int run_fused_streamed(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates
 template <typename R, int RB, int TB>
 static int run_fused_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int ngates, int L, KnownZeros z, int* passes,
                        hipStream_t s) {
-  const Config c = fused_config(RB, TB, L, gates, ngates);
+  Config c = fused_config(RB, TB, L, gates, ngates);
+  if (z.whole) c.wires = false, c.remap = 0;
   if (c.remap == 0) {  // passes are final as they form: streamed
     const char* st = getenv("QS_FUSION_STREAM");
     if (!(st && st[0] == '0')) return run_fused_streamed<R, RB, TB>(ctx, v, n, gates, ngates, c, z, passes, s);
@@ -393,7 +394,8 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
   // fewer are no slower as kernels of their own.  Programs that keep whole gates in
   // the tile (fused_config) need more than one tile's bits.
   KnownZeros z = start < 0 ? KnownZeros() : known_start(n, start == QS_START_IDENTITY);
-  const bool per_gate = ngates == 0 || (n < K + 1 && (ngates < 3 || !fused_config(4, K - 4, L, gates, ngates).wires));
+  z.whole = start == QS_START_ZERO_WHOLE;
+  const bool per_gate = ngates == 0 || (n < K + 1 && (ngates < 3 || z.whole || !fused_config(4, K - 4, L, gates, ngates).wires));
   if (per_gate) {
     const int rc = dtype == QS_C128 ? write_rest((cx<double>*)vec, n, z, s) : write_rest((cx<float>*)vec, n, z, s);
     if (rc) return rc;

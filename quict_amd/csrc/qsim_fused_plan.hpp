@@ -1002,6 +1002,7 @@ struct KnownZeros {
   uint64_t fixed = 0;
   int sh = 0;
   bool fresh = false;
+  bool whole = false;  // the program is planned with whole gates in the tile (QS_START_ZERO_WHOLE)
 };
 static KnownZeros known_start(int n, bool identity) {
   KnownZeros z;
