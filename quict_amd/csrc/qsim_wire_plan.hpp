@@ -397,7 +397,10 @@ struct WireReducer {
     }
   }
 
-  // m = f diag(1, pa) [[c, -s], [s, c]] diag(1, pb); false if m is not unitary to tol.
+  // m = f diag(1, pa) [[c, -s], [s, c]] diag(1, pb); false if no such product gives m to
+  // tol.  Three of the four entries' phases fix f, pa and pb: the larger two are among
+  // them.  (Where gates on a wire cancel, the smaller two are rounding, and the phase of
+  // a rounding error would go into a large entry.)
   static bool factor(const double* m, double tol, cplx& f, cplx& pa, cplx& pb, double& c_, double& s_) {
     auto e = [&](int i) { return cplx{m[2 * i], m[2 * i + 1]}; };
     auto mag = [](cplx z) { return std::hypot(z.first, z.second); };
@@ -405,33 +408,29 @@ struct WireReducer {
       const double r = mag(z);
       return cplx{z.first / r, z.second / r};
     };
+    auto neg = [](cplx z) { return cplx{-z.first, -z.second}; };
     c_ = mag(e(0)), s_ = mag(e(2));
     const double h = std::hypot(c_, s_);
-    if (!(std::fabs(h - 1.0) <= tol) || std::fabs(mag(e(3)) - c_) > tol || std::fabs(mag(e(1)) - s_) > tol) return false;
-    // orthogonal columns: conj(m00) m01 + conj(m10) m11 = 0
-    const cplx d0 = cm_({m[0], -m[1]}, e(1)), d1 = cm_({m[4], -m[5]}, e(3));
-    if (std::hypot(d0.first + d1.first, d0.second + d1.second) > tol) return false;
+    if (!(std::fabs(h - 1.0) <= tol)) return false;
     c_ /= h, s_ /= h;
-    if (s_ == 0.0) {
-      f = unit(e(0)), pb = {1.0, 0.0}, pa = unit(cdiv_(e(3), e(0)));
-      return true;
-    }
-    if (c_ == 0.0) {
-      f = unit(e(2)), pa = {1.0, 0.0}, pb = unit(cdiv_(e(1), e(2)));
-      pb = {-pb.first, -pb.second};
-      return true;
-    }
-    f = unit(e(0));
-    pa = unit(cdiv_(e(2), f));
-    pb = unit(cdiv_(e(1), f));
-    pb = {-pb.first, -pb.second};
+    f = c_ == 0.0 ? unit(e(2)) : unit(e(0));
+    pa = s_ == 0.0 || c_ == 0.0 ? cplx{1.0, 0.0} : unit(cdiv_(e(2), f));
+    if (s_ == 0.0) pa = unit(cdiv_(e(3), f)), pb = {1.0, 0.0};
+    else if (c_ >= s_) pb = unit(cdiv_(e(3), cm_(f, pa)));
+    else pb = neg(unit(cdiv_(e(1), f)));
+    // (written so that a phase of a zero, which is not a number, fails)
+    auto gives = [&](int i, cplx z, double r) {
+      return mag({m[2 * i] - z.first * r, m[2 * i + 1] - z.second * r}) <= tol;
+    };
+    const cplx fa = cm_(f, pa);
+    if (!(gives(0, f, c_) && gives(1, cm_(f, pb), -s_) && gives(2, fa, s_) && gives(3, cm_(fa, pb), c_))) return false;
     // s may have either sign: the one that leaves a factor at 1, else any
     const double d = 1e-15;
     auto neg_one = [&](cplx z) { return std::fabs(z.first + 1.0) <= d && std::fabs(z.second) <= d; };
-    if (neg_one(pa) || neg_one(pb)) {
+    if (s_ != 0.0 && c_ != 0.0 && (neg_one(pa) || neg_one(pb))) {
       s_ = -s_;
-      pa = {-pa.first, -pa.second};
-      pb = {-pb.first, -pb.second};
+      pa = neg(pa);
+      pb = neg(pb);
     }
     return true;
   }
