@@ -330,7 +330,7 @@ static int capture_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int nga
     return QS_ERR_DEVICE;
   }
   int npass = 0;
-  rc = launch_passes<R, RB, TB>(ctx, v, n, c, prog, (const char*)G->dprog, im, init_zero ? known_start(n, 0) : KnownZeros(), s, false,
+  rc = launch_passes<R, RB, TB>(ctx, v, n, c, prog, (const char*)G->dprog, im, init_zero ? known_start(n, false, RB + TB) : KnownZeros(), s, false,
                                 &npass);
   hipGraph_t graph = nullptr;
   e = hipStreamEndCapture(s, &graph);
@@ -393,7 +393,7 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
   // (5 qubits, 100 gates: 508 us a run with a kernel per gate, 247 us so); two gates or
   // fewer are no slower as kernels of their own.  Programs that keep whole gates in
   // the tile (fused_config) need more than one tile's bits.
-  KnownZeros z = start < 0 ? KnownZeros() : known_start(n, start == QS_START_IDENTITY);
+  KnownZeros z = start < 0 ? KnownZeros() : known_start(n, start == QS_START_IDENTITY, K);
   z.whole = start == QS_START_ZERO_WHOLE;
   const bool per_gate = ngates == 0 || (n < K + 1 && (ngates < 3 || z.whole || !fused_config(4, K - 4, L, gates, ngates).wires));
   if (per_gate) {

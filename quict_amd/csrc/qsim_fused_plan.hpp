@@ -1004,11 +1004,14 @@ struct KnownZeros {
   bool fresh = false;
   bool whole = false;  // the program is planned with whole gates in the tile (QS_START_ZERO_WHOLE)
 };
-static KnownZeros known_start(int n, bool identity) {
+// A register of fewer bits than a tile (n < K): the idle ones are 0 as well.  All of a
+// single tile's bits are in its first pass, which leaves nothing known: the passes after
+// it load what the register has, no more.
+static KnownZeros known_start(int n, bool identity, int K) {
   KnownZeros z;
   z.sh = identity ? n / 2 : 0;
-  // (|0...0> on fewer bits than a tile has: the idle ones are 0 as well)
-  z.fixed = identity ? (1ull << (n / 2)) - 1 : (1ull << std::max(n, 13)) - 1;
+  z.fixed = (1ull << (identity ? n / 2 : n)) - 1;
+  for (int b = n; b < K; ++b) z.fixed |= 1ull << b;
   z.fresh = true;
   return z;
 }

@@ -59,7 +59,10 @@ static void wire_pass(zc* v, int n, int RB, int TB, uint32_t S, const PassHdr& H
         for (int b = 0; b < TB; ++b) g |= (uint64_t)((tid >> b) & 1) << H.tbits[H.ts0[b]];
         for (int b = 0; b < RB; ++b) g |= (uint64_t)((r >> b) & 1) << H.tbits[H.rs0[b]];
         const bool zero = ((known.sh ? g ^ (g >> known.sh) : g) & known.fixed) != 0;
-        a[(size_t)tid * NR + r] = zero || g >= N ? zc(0) : known.fixed && known.fresh ? zc(1) : v[g];
+        if (!known.fixed) a[(size_t)tid * NR + r] = g >= N ? zc(0) : v[g];  // (wire_load: with nsmall)
+        else if (zero || known.fresh) a[(size_t)tid * NR + r] = zero ? 0.0 : 1.0;
+        else if (g >= N) throw std::runtime_error("load outside the vector");
+        else a[(size_t)tid * NR + r] = v[g];
       }
     for (int o = 0; o < H.nops; ++o) {
       const FOp& op = P[o];
@@ -266,7 +269,7 @@ extern "C" int wires_run(double* vec, int n, int identity, const qs_gate* gates,
     c.wires = true;
     FusedProgram prog;
     const int K = RB + TB;
-    KnownZeros z = known_start(n, identity);
+    KnownZeros z = known_start(n, identity, K);
     std::fill(stats, stats + 3, 0);
     zc* v = reinterpret_cast<zc*>(vec);
     auto rest = [&]() {
