@@ -1212,20 +1212,16 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
       const Rem& r = rem[k];
       if (!((r.a & wm) | (r.m & wa))) {
         const uint64_t need = r.need & ~S;
-        const int t0 = tables, m0 = meas;
-        bool room = true;
-        if (r.flags) {
-          if (r.flags & TABLE) room = ++tables <= max_tables;
-          if (r.flags & MEAS) room = ++meas <= FMAX_GRAD;
-        }
+        const bool room = !((r.flags & TABLE) && tables >= max_tables) && !((r.flags & MEAS) && meas >= FMAX_GRAD);
         const bool able = room && !(r.flags & ALONE);
         if (!need && able) {
           w += r.w;
+          tables += (r.flags & TABLE) != 0, meas += (r.flags & MEAS) != 0;
           if (taken) taken->push_back(k);
           continue;
         }
         if (cand) {
-          if (!wa) from.k = k, from.w = w, from.tables = t0, from.meas = m0;
+          if (!wa) from.k = k, from.w = w, from.tables = tables, from.meas = meas;
           if (need && able && std::find(cand->begin(), cand->end(), need) == cand->end()) cand->push_back(need);
         }
       }
