@@ -377,6 +377,21 @@ int apply_gates_fused(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* g
   }
 }
 
+// Whether a list on a register of at most a tile is faster planned and run in one launch
+// than as a kernel a gate.  us a call on MI355X, 10 qubits, kernels / one launch: 6 gates
+// on one or two qubits 27 / 26 to 35, 8 of them 40 to 60 / 30 to 40, 40 of them 160 / 39 to
+// 114.  The workgroup's dense op on three targets (four in complex128) takes longer than
+// the gate's own kernel: 20 such gates 123 / 185 (462 / 539), and pays for it only among
+// enough others; on four targets in complex64 it is the faster by far, 3 gates 74 / 45.
+static bool one_launch_pays(const qs_gate* gates, int ngates, int dtype) {
+  int gain = 0;
+  for (int i = 0; i < ngates; ++i) {
+    const bool wide = gates[i].kind == QS_GATE_DENSE && (gates[i].ntargets == 3 || gates[i].ntargets == 4);
+    gain += !wide ? 1 : gates[i].ntargets == 4 && dtype == QS_C64 ? 3 : -1;
+  }
+  return gain >= 7;
+}
+
 static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates,
                                   int start, int* passes, hipStream_t s) {
   // Tile shapes (4 register bits per thread, 2^(K-4) threads, a half-tile LDS
@@ -389,13 +404,12 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
     set_error("low_bits must not exceed tile_log2 - 4");
     return QS_ERR_ARG;
   }
-  // Registers of at most a tile run whole programs planned in wires in one launch
-  // (5 qubits, 100 gates: 508 us a run with a kernel per gate, 247 us so); two gates or
-  // fewer are no slower as kernels of their own.  Programs that keep whole gates in
-  // the tile (fused_config) need more than one tile's bits.
+  // Registers of at most a tile run programs planned in wires in one launch where that
+  // pays (one_launch_pays).  Programs that keep whole gates in the tile (fused_config)
+  // need more than one tile's bits.
   KnownZeros z = start < 0 ? KnownZeros() : known_start(n, start == QS_START_IDENTITY, K);
   z.whole = start == QS_START_ZERO_WHOLE;
-  const bool per_gate = ngates == 0 || (n < K + 1 && (ngates < 3 || z.whole || !fused_config(4, K - 4, L, gates, ngates).wires));
+  const bool per_gate = ngates == 0 || (n < K + 1 && (!one_launch_pays(gates, ngates, dtype) || z.whole || !fused_config(4, K - 4, L, gates, ngates).wires));
   if (per_gate) {
     const int rc = dtype == QS_C128 ? write_rest((cx<double>*)vec, n, z, s) : write_rest((cx<float>*)vec, n, z, s);
     if (rc) return rc;
