@@ -1205,6 +1205,10 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
   struct From {
     int k = 0, w = 0, tables = 0, meas = 0;
   };
+  // Candidates beyond the first 48 (more than there are wires; gates on several wires
+  // have more sets than that) cost a scan each and do not make plans shorter: 200
+  // three-qubit diagonal gates on 20 qubits 10 passes in 1.9 ms of planning, now 1.5 ms.
+  constexpr size_t MAX_CAND = 48;
   auto scan = [&](uint64_t S, From& from, std::vector<uint64_t>* cand, std::vector<int>* taken) -> int {
     uint64_t wa = 0, wm = 0;
     int w = from.w, tables = from.tables, meas = from.meas;
@@ -1222,7 +1226,8 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
         }
         if (cand) {
           if (!wa) from.k = k, from.w = w, from.tables = tables, from.meas = meas;
-          if (need && able && std::find(cand->begin(), cand->end(), need) == cand->end()) cand->push_back(need);
+          if (need && able && cand->size() < MAX_CAND && std::find(cand->begin(), cand->end(), need) == cand->end())
+            cand->push_back(need);
         }
       }
       wa |= r.a;
