@@ -155,9 +155,14 @@ struct WireReducer {
       gphase = cm_(gphase, f);
       return;
     }
+    int flipped = 0;
+    for (int i = 0; i < k; ++i) flipped += (F >> ws[i]) & 1;
+    // Every flipped bit splits the phase in two (below): from two of them on, on more
+    // than two bits (whose parts join what is on their wires), the flips become gates.
+    const bool split = (flipped == 1 || k <= 2) && (f.first != 0.0 || f.second != 0.0);
     for (int i = 0; i < k; ++i) {
       if (!((F >> ws[i]) & 1)) continue;
-      if (f.first == 0.0 && f.second == 0.0) {
+      if (!split) {
         materialize(ws[i]);
         continue;
       }

@@ -4,9 +4,10 @@ import ctypes
 import random
 
 import numpy as np
+import pytest
 
 from quict_amd import _native as nat
-from quict_amd.core import Circuit, Unitary
+from quict_amd.core import Circuit, H, Unitary, X
 from quict_amd.simulation.gate_compiler import compile_gates
 from test_wire_planner import check, emu  # noqa: F401  (the fixture)
 
@@ -34,3 +35,31 @@ def test_a_pass_takes_as_many_tables_as_it_stages(emu):  # noqa: F811
     assert plan(emu, recs, 20)[0] <= 12
     recs, keep = tables(15, 200)
     check(emu, recs, 15)
+
+
+def all_ones_phase(n, k, hadamards):
+    """X on k qubits, a phase on all of them, X again; with Hadamard gates around: a
+    Grover diffusion."""
+    c = Circuit(n)
+    args = list(range(n - k, n))
+    m = np.eye(1 << k, dtype=complex)
+    m[-1, -1] = np.exp(0.7j)
+    for g in [H, X] if hadamards else [X]:
+        for q in args:
+            g | c(q)
+    Unitary(m) | c(args)
+    for g in [X, H] if hadamards else [X]:
+        for q in args:
+            g | c(q)
+    return c
+
+
+@pytest.mark.parametrize("hadamards", [False, True])
+@pytest.mark.parametrize("k", [3, 4, 6, 8, 10])
+def test_a_phase_under_flips_stays_one_phase(emu, k, hadamards):  # noqa: F811
+    n = 14
+    recs, keep = compile_gates(all_ones_phase(n, k, hadamards).gates, n)
+    # a phase, at most a flip or a rotation with two phases on either side of it per
+    # qubit, relayouts between them
+    assert plan(emu, recs, n)[2] <= 8 * k
+    check(emu, recs, n)
