@@ -12,7 +12,7 @@
 //     conjugated (a CX with a flipped control also flips the target's frame), and
 //     what is left is one X at the end, which joins the wire's last gate or is a
 //     flip of a store address;
-//   * every diagonal gate on one or two targets becomes phases "all these bits
+//   * every diagonal gate on one or two targets (of modulus 1) becomes phases "all these bits
 //     are 1: times f" (Rz, S, T, CZ, CRz, Rzz, ...), their common factors one
 //     number for the whole program;
 //   * one-qubit gates on a wire are multiplied together, past phases that
@@ -67,6 +67,11 @@ static cplx cdiv_(cplx a, cplx b) {
   const double d = b.first * b.first + b.second * b.second;
   return {(a.first * b.first + a.second * b.second) / d, (a.second * b.first - a.first * b.second) / d};
 }
+
+// Whether f may be taken out of a gate as a common factor and divided by.  Entries far
+// from modulus 1 stay in their gate: a program's common factor, or the reciprocal of
+// one, would leave the range of its precision where no amplitude does.
+static bool near_unit(cplx f) { return std::fabs(std::hypot(f.first, f.second) - 1.0) <= 1e-5; }
 
 struct WireReducer {
   const Config& c;
@@ -159,7 +164,7 @@ struct WireReducer {
     for (int i = 0; i < k; ++i) flipped += (F >> ws[i]) & 1;
     // Every flipped bit splits the phase in two (below): from two of them on, on more
     // than two bits (whose parts join what is on their wires), the flips become gates.
-    const bool split = (flipped == 1 || k <= 2) && (f.first != 0.0 || f.second != 0.0);
+    const bool split = (flipped == 1 || k <= 2) && near_unit(f);
     for (int i = 0; i < k; ++i) {
       if (!((F >> ws[i]) & 1)) continue;
       if (!split) {
@@ -262,7 +267,8 @@ struct WireReducer {
     const int* w = g.bits;
     auto entry = [&](int i) { return cplx{g.m[2 * i], g.m[2 * i + 1]}; };
     auto zero = [&](int i) { return g.m[2 * i] == 0.0 && g.m[2 * i + 1] == 0.0; };
-    if (g.kind == QS_GATE_XPERM && nc <= 1 && (pure_exchange(g) || (!zero(0) && !zero(1)))) {
+    auto unit = [&](int i) { return near_unit(entry(i)); };
+    if (g.kind == QS_GATE_XPERM && nc <= 1 && (pure_exchange(g) || (unit(0) && !zero(1)))) {
       const int t = w[nc];
       if (nc == 0) {
         F ^= 1ull << t;
@@ -283,12 +289,12 @@ struct WireReducer {
       phase(w, nc + nt, entry(0));
       return;
     }
-    if (g.kind == QS_GATE_DIAG && nt == 1 && !zero(0)) {
+    if (g.kind == QS_GATE_DIAG && nt == 1 && unit(0)) {
       phase(w, nc, entry(0));
       phase(w, nc + 1, cdiv_(entry(1), entry(0)));
       return;
     }
-    if (g.kind == QS_GATE_DIAG && nt == 2 && !zero(0) && !zero(1) && !zero(2)) {
+    if (g.kind == QS_GATE_DIAG && nt == 2 && unit(0) && unit(1) && unit(2)) {
       int a[QS_MAX_GATE_BITS];
       for (int i = 0; i < nc; ++i) a[i] = w[i];
       phase(a, nc, entry(0));
