@@ -392,6 +392,17 @@ static bool one_launch_pays(const qs_gate* gates, int ngates, int dtype) {
   return gain >= 7;
 }
 
+// A program's upload reads a staging slot that later calls use again, and waits for the
+// slot's event: neither belongs into a caller's graph.
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();  // (the null stream while another stream captures)
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, const qs_gate* gates, int ngates,
                                   int start, int* passes, hipStream_t s) {
   // Tile shapes (4 register bits per thread, 2^(K-4) threads, a half-tile LDS
@@ -405,11 +416,12 @@ static int apply_gates_fused_impl(qs_ctx* ctx, void* vec, int n, int dtype, cons
     return QS_ERR_ARG;
   }
   // Registers of at most a tile run programs planned in wires in one launch where that
-  // pays (one_launch_pays).  Programs that keep whole gates in the tile (fused_config)
-  // need more than one tile's bits.
+  // pays (one_launch_pays); into a graph of the caller's they go as a kernel a gate.
+  // Programs that keep whole gates in the tile (fused_config) need more than one tile's
+  // bits.
   KnownZeros z = start < 0 ? KnownZeros() : known_start(n, start == QS_START_IDENTITY, K);
   z.whole = start == QS_START_ZERO_WHOLE;
-  const bool per_gate = ngates == 0 || (n < K + 1 && (!one_launch_pays(gates, ngates, dtype) || z.whole || !fused_config(4, K - 4, L, gates, ngates).wires));
+  const bool per_gate = ngates == 0 || (n < K + 1 && (!one_launch_pays(gates, ngates, dtype) || z.whole || capturing(s) || !fused_config(4, K - 4, L, gates, ngates).wires));
   if (per_gate) {
     const int rc = dtype == QS_C128 ? write_rest((cx<double>*)vec, n, z, s) : write_rest((cx<float>*)vec, n, z, s);
     if (rc) return rc;
