@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -128,6 +129,7 @@ struct qs_ctx {
   };
   ProgSlot prog_slot[2];
   int prog_next = 0;
+  std::mutex slot_mu;  // held from acquire_prog_slot until the slot's event is recorded
   qs::QnnState* qnn = nullptr;  // batches of variational circuits (qsim_qnn_planned.hip)
   // kernel timing (HIP events recorded on the launch stream around each launch)
   int profile = 0;
@@ -141,7 +143,8 @@ namespace qs {
 // Grow-only scratch buffers owned by the context.
 int ensure_scratch(qs_ctx* ctx, uint64_t bytes);
 // A free program slot of at least `bytes` (host and device), waiting for its
-// previous use to finish.
+// previous use to finish.  The caller holds ctx->slot_mu, and until it has recorded
+// the slot's event: threads that run circuits on one device share its context.
 int acquire_prog_slot(qs_ctx* ctx, uint64_t bytes, qs_ctx::ProgSlot** out);
 // The same with separate pinned-host and device sizes.
 int acquire_prog_slot(qs_ctx* ctx, uint64_t host_bytes, uint64_t dev_bytes, qs_ctx::ProgSlot** out);

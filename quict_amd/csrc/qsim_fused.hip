@@ -227,6 +227,7 @@ static int run_fused_streamed(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates
   auto chunk = [&](const FusedProgram& sub, int) -> int {
     ProgImage im;
     pack_program<R>(sub, c, im);
+    std::lock_guard<std::mutex> lock(ctx->slot_mu);
     qs_ctx::ProgSlot* slot = nullptr;
     int rc = acquire_prog_slot(ctx, im.host.size() + 256, &slot);
     if (rc) return rc;
@@ -269,6 +270,7 @@ static int run_fused_t(qs_ctx* ctx, cx<R>* v, int n, const qs_gate* gates, int n
   pack_program<R>(prog, c, im);
   // upload from a pinned slot that stays untouched until this call's passes
   // have run (its event), so the call returns without waiting for the device
+  std::lock_guard<std::mutex> lock(ctx->slot_mu);
   qs_ctx::ProgSlot* slot = nullptr;
   rc = acquire_prog_slot(ctx, im.host.size() + 256, &slot);
   if (rc) return rc;

@@ -654,6 +654,7 @@ static int adjoint_t(qs_ctx* ctx, cx<R>* psi, cx<R>* lam, int n, const qs_gate* 
   const uint64_t part_off = al(up), sums_off = al(part_off + rows * ADJ_MAX_BLOCKS * sizeof(double));
   const uint64_t ip_off = al(sums_off + rows * sizeof(double));
   const uint64_t dev_end = ip_off + (2 * (uint64_t)inner_partial_blocks() + 64) * sizeof(double);
+  std::lock_guard<std::mutex> lock(ctx->slot_mu);
   qs_ctx::ProgSlot* pslot = nullptr;
   rc = acquire_prog_slot(ctx, res_off + (rows + 2) * sizeof(double), dev_end, &pslot);
   if (rc) return rc;
