@@ -291,7 +291,8 @@ int qs_adjoint_gradient_pauli(qs_ctx* ctx, void* psi, void* lam, int n, int dtyp
    rotation exp(-i theta[param_slot[i]] P / 2) on bit gates[i].bits[0], P = X, Y, Z for
    axis[i] = 0, 1, 2 (nothing else of the record is read; a phase diag(1, e^{i theta})
    is a Z rotation up to a common phase).  The plan does not depend on the angles.
-   QS_ERR_UNSUPPORTED: a gate needs a pass of its own (see qs_graph_capture).
+   QS_ERR_UNSUPPORTED: a gate needs a pass of its own (see qs_graph_capture), or device
+   memory for the gradient rows (at most 64 MiB, or one pass's) is missing.
    qs_var_gradient: energy <psi|H|psi> of psi = circuit |0...0> and its derivatives,
    added to grads[0..nslots); psi and lam are caller buffers of max(2^n, 4096)
    amplitudes whose contents are ignored and overwritten.  It waits for the stream.

@@ -53,6 +53,10 @@ struct qs_var {
   qs::VarImage im;
   qs::AngleTable angles;
   std::vector<qs::ColSum> colsums;
+  // per backward pass: first entry of its gradient rows, and the columns summed so far
+  // once they have been written (0: not after this pass)
+  std::vector<uint64_t> row0;
+  std::vector<int> sum_to;
   // device: image, column descriptors, column sums, gradient rows, inner-product partials
   char* dev = nullptr;
   uint64_t col_off = 0, sum_off = 0, part_off = 0, ip_off = 0, dev_bytes = 0;
@@ -68,20 +72,38 @@ template <typename R> static int var_build(qs_var* v, const std::vector<VarOp>& 
   const int n = std::max(v->n, 12);
   int rc = v->im.build<R>(ops, n);
   if (rc) return rc;
+  // Rows of as many passes as fit, then their sums, then the next ones in their place:
+  // 33 qubits and 480 parameters would be 8 GB of rows beside 275 GB of state.
+  constexpr uint64_t MAX_ROWS = (64ull << 20) / sizeof(double);
   const uint64_t tiles = 1ull << (n - 12);
-  uint64_t part = 0;
+  uint64_t part = 0, most = 0;
   for (const VarImage::Pass& p : v->im.bwd) {
+    const uint64_t rows = tiles * p.ngrad;
+    if (part > 0 && part + rows > MAX_ROWS) {
+      v->sum_to.back() = (int)v->colsums.size();
+      part = 0;
+    }
+    v->row0.push_back(part);
+    v->sum_to.push_back(0);
     for (int i = 0; i < p.ngrad; ++i) v->colsums.push_back({part + i, (uint32_t)tiles, (uint32_t)p.ngrad});
-    part += tiles * p.ngrad;
+    part += rows;
+    most = std::max(most, part);
   }
+  if (!v->sum_to.empty()) v->sum_to.back() = (int)v->colsums.size();
   const uint64_t nc = v->colsums.size();
   v->col_off = al256(v->im.host.size());
   v->sum_off = al256(v->col_off + nc * sizeof(ColSum));
   v->part_off = al256(v->sum_off + nc * sizeof(double));
-  v->ip_off = al256(v->part_off + part * sizeof(double));
+  v->ip_off = al256(v->part_off + most * sizeof(double));
   v->dev_bytes = v->ip_off + (2 * (uint64_t)inner_partial_blocks() + 64) * sizeof(double);
   v->res_off = al256(v->im.host.size());
-  QS_CHECK_HIP(hipMalloc((void**)&v->dev, v->dev_bytes));
+  const hipError_t err = hipMalloc((void**)&v->dev, v->dev_bytes);
+  if (err != hipSuccess) {  // (the call that takes gate records needs less)
+    (void)hipGetLastError();
+    v->dev = nullptr;
+    set_error(std::string("planned gradient: ") + hipGetErrorString(err));
+    return QS_ERR_UNSUPPORTED;
+  }
   QS_CHECK_HIP(hipHostMalloc((void**)&v->host, v->res_off + (nc + 2) * sizeof(double), hipHostMallocDefault));
   if (nc) QS_CHECK_HIP(hipMemcpy(v->dev + v->col_off, v->colsums.data(), nc * sizeof(ColSum), hipMemcpyHostToDevice));
   return QS_OK;
@@ -121,18 +143,22 @@ static int var_gradient(qs_var* v, cx<R>* psi, cx<R>* lam, const double* theta, 
   if (!rc) rc = inner_async(psi, lam, v->n, v->dtype, ipart, ires, s);
   if (rc) return rc;
   if ((rc = prof_begin(ctx, PROF_GRAD, s))) return rc;
+  const int nc = (int)v->colsums.size();
+  double* sums = (double*)(v->dev + v->sum_off);
+  int summed = 0;
   for (size_t i = 0; i < v->im.bwd.size(); ++i) {
     const VarImage::Pass& p = v->im.bwd[i];
     j.hdr = h++ * (uint32_t)sizeof(PassHdr);
     j.keep = i + 1 < v->im.bwd.size() ? 3 : 0;  // nothing reads the vectors after the sweep
+    j.part = v->row0[i];
     launch_jobs<R>(psi, lam, v->dev, J, (uint32_t)tiles, p.heavy, partial, p.lds, s);
     QS_CHECK_HIP(hipGetLastError());
-    j.part += tiles * p.ngrad;
+    if (v->sum_to[i] > summed) {
+      column_sums(partial, (const ColSum*)(v->dev + v->col_off) + summed, v->sum_to[i] - summed, sums + summed, s);
+      QS_CHECK_HIP(hipGetLastError());
+      summed = v->sum_to[i];
+    }
   }
-  const int nc = (int)v->colsums.size();
-  double* sums = (double*)(v->dev + v->sum_off);
-  column_sums(partial, (const ColSum*)(v->dev + v->col_off), nc, sums, s);
-  QS_CHECK_HIP(hipGetLastError());
   if ((rc = prof_end(ctx, s))) return rc;
   double* res = (double*)(v->host + v->res_off);
   if (nc) QS_CHECK_HIP(hipMemcpyAsync(res, sums, nc * sizeof(double), hipMemcpyDeviceToHost, s));
