@@ -53,6 +53,17 @@ int qnn_planned(qs_ctx* ctx, int ncirc, const int32_t* widths, int nfeat, const 
 QnnState* qnn_state_create();
 void qnn_state_destroy(QnnState* S);
 
+// Waits for what a call has queued if the call returns before it has waited itself: the
+// next one writes the same staging memory.
+struct WaitOnError {
+  hipStream_t s;
+  bool waited = false;
+  explicit WaitOnError(hipStream_t st) : s(st) {}
+  ~WaitOnError() {
+    if (!waited) (void)hipStreamSynchronize(s);
+  }
+};
+
 inline size_t amp_bytes(int dtype) { return dtype == QS_C128 ? 16 : 8; }
 
 }  // namespace qs

@@ -582,6 +582,7 @@ static int qnn_c64(qs_ctx* ctx, int fuse, int ncirc, const int32_t* widths, int 
   }
   hipStream_t s = S->stream;
   char* d = S->dev;
+  WaitOnError wait(s);
   QS_CHECK_HIP(hipMemcpyAsync(d, S->host, up, hipMemcpyHostToDevice, s));
   QnnArgs A;
   A.nfeat = nfeat, A.layers = layers, A.max_width = max_width;
@@ -624,6 +625,7 @@ static int qnn_c64(qs_ctx* ctx, int fuse, int ncirc, const int32_t* widths, int 
   const double* r = (const double*)(S->host + res_off);
   QS_CHECK_HIP(hipMemcpyAsync((void*)r, res, (grad_x ? nres : nres - nx) * sizeof(double), hipMemcpyDeviceToHost, s));
   QS_CHECK_HIP(hipStreamSynchronize(s));
+  wait.waited = true;
   std::vector<double> terms(ncirc);
   for (int i = 0; i < ncirc; ++i) {
     expval[order[i]] = r[i];

@@ -358,6 +358,7 @@ static int qnn_part(qs_ctx* ctx, QnnState* S, const int32_t* order, int n, int n
   double* epart = (double*)(d + e_off);
   const double* dx = (const double*)(d + x_off);
   const double* dt = (const double*)(d + t_off);
+  WaitOnError wait(s);
   QS_CHECK_HIP(hipMemcpyAsync(d, S->host, up, hipMemcpyHostToDevice, s));
   if ((rc = prof_begin(ctx, PROF_QNN, s))) return rc;
   const dim3 block(256), all((unsigned)units);
@@ -412,6 +413,7 @@ static int qnn_part(qs_ctx* ctx, QnnState* S, const int32_t* order, int n, int n
   double* res = (double*)(S->host + res_off);
   QS_CHECK_HIP(hipMemcpyAsync(res, sums, nres * sizeof(double), hipMemcpyDeviceToHost, s));
   QS_CHECK_HIP(hipStreamSynchronize(s));
+  wait.waited = true;
   const double* r = res;
   for (int j = 0; j < G.n; ++j) {
     const int w = G.g[j].w;

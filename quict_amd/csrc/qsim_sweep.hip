@@ -118,6 +118,7 @@ static int var_gradient(qs_var* v, cx<R>* psi, cx<R>* lam, const double* theta, 
   v->angles.fill(theta, v->nslots);
   v->im.bind<R>(v->angles, [](int slot) { return slot; });
   std::memcpy(v->host, v->im.host.data(), v->im.host.size());
+  WaitOnError wait(s);
   QS_CHECK_HIP(hipMemcpyAsync(v->dev, v->host, v->im.host.size(), hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_basis<R>, dim3((unsigned)std::min<uint64_t>(N / 256, 1u << 16)), dim3(256), 0, s, psi,
                      v->n < 12 ? lam : nullptr, N);
@@ -164,6 +165,7 @@ static int var_gradient(qs_var* v, cx<R>* psi, cx<R>* lam, const double* theta, 
   if (nc) QS_CHECK_HIP(hipMemcpyAsync(res, sums, nc * sizeof(double), hipMemcpyDeviceToHost, s));
   QS_CHECK_HIP(hipMemcpyAsync(res + nc, ires, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
   QS_CHECK_HIP(hipStreamSynchronize(s));
+  wait.waited = true;
   *energy = res[nc];
   for (int i = 0; i < nc; ++i) grads[v->im.cols[i].slot] += v->im.cols[i].sgn * res[i];
   return QS_OK;
