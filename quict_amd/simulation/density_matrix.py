@@ -193,9 +193,15 @@ class DensityMatrixSimulator:
 
     def initial_circuit(self, circuit: Circuit, noise_model: NoiseModel):
         self._origin_circuit = circuit
-        self._circuit = circuit if noise_model is None else noise_model.transpile(circuit, self._accumulated_mode, lazy=True)
+        self._circuit = circuit if noise_model is None else self._noisy(noise_model, circuit)
         self._noise_model = noise_model
         self._qubits = int(circuit.width())
+
+    def _noisy(self, noise_model, circuit: Circuit) -> Circuit:
+        """The circuit with its channels; Kraus products on demand where ``transpile`` is
+        the library's own (others take the two documented arguments)."""
+        own = getattr(noise_model.transpile, "__func__", None) is NoiseModel.transpile
+        return noise_model.transpile(circuit, self._accumulated_mode, **({"lazy": True} if own else {}))
 
     def initial_density_matrix(self, qubits: int):
         self._density_matrix = self._torch.empty(1 << (2 * qubits), dtype=self._tdtype,
@@ -350,7 +356,7 @@ class DensityMatrixSimulator:
             self._noise_model.apply_readout_error(self._circuit.qubits)
             counts[int(self._circuit.qubits)] += 1
             self.initial_density_matrix(n)
-            noised = self._noise_model.transpile(self._origin_circuit, self._accumulated_mode, lazy=True)
+            noised = self._noisy(self._noise_model, self._origin_circuit)
             self._circuit = noised
             self._run(noised)
         return counts
