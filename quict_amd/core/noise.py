@@ -304,7 +304,7 @@ class NoiseModel:
                     if qubits == -1 or set(qubits) & set(args) == set(args):
                         if accumulated_mode or noise.type == NoiseChannel.damping:
                             matrix = gate.matrix.astype(np.complex128)
-                            if lazy:
+                            if lazy and type(noise).apply_to_gate is QuantumNoiseError.apply_to_gate:
                                 ng = NoiseGate.after_gate(gate, matrix, noise, len(args))
                             else:
                                 ng = NoiseGate(noise.apply_to_gate(matrix), len(args))
