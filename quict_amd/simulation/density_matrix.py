@@ -237,9 +237,13 @@ class DensityMatrixSimulator:
                                                          device=f"cuda:{self._device_id}")
         elif self._density_matrix is None or not use_previous or \
                 self._density_matrix.numel() != (1 << (2 * self._qubits)):
-            self._density_matrix = self._torch.empty(1 << (2 * self._qubits), dtype=self._tdtype,
-                                                     device=f"cuda:{self._device_id}")
-            self._start = True
+            own = DensityMatrixSimulator.initial_density_matrix
+            if getattr(self.initial_density_matrix, "__func__", None) is own:
+                self._density_matrix = self._torch.empty(1 << (2 * self._qubits), dtype=self._tdtype,
+                                                         device=f"cuda:{self._device_id}")
+                self._start = True
+            else:  # a subclass's own start
+                self.initial_density_matrix(self._qubits)
         self.last_passes = 0
         try:
             self._run(self._circuit)

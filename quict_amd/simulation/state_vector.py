@@ -155,8 +155,12 @@ class StateVectorSimulator:
                 raise qerr.StateVectorUnmatchedError("the state vector must have 2^width amplitudes")
             self.vector = sv
         elif not use_previous or self._vector is None or self._vector.numel() != (1 << self._qubits):
-            self._vector = self._torch.empty(1 << self._qubits, dtype=self._tdtype, device=f"cuda:{self._device_id}")
-            self._start = True
+            if getattr(self.initial_state_vector, "__func__", None) is StateVectorSimulator.initial_state_vector:
+                self._vector = self._torch.empty(1 << self._qubits, dtype=self._tdtype,
+                                                 device=f"cuda:{self._device_id}")
+                self._start = True
+            else:  # a subclass's own start
+                self.initial_state_vector()
         self.last_passes = 0
         try:
             self._run_pipeline()
