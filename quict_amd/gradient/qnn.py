@@ -7,11 +7,11 @@ squared loss) is documented in quict_amd/csrc/qsim_qnn.hip.  ``QNNBatch``
 mirrors a torch loss module: ``forward_backward(theta)`` returns the mean loss,
 per-circuit <Z_0>, d loss / d theta and d loss / d x.
 
-``autotune`` times every launch shape of a small search space on the real
-batch (LDS width limit, workgroup size, workgroups per CU) and caches the
-winner per (dtype, width histogram, layers, features) in a JSON file.  (The library
-takes its launch shapes from the widths; the values are checked, and fuse_qubits
-selects the order of rounding of complex64 results.)
+``autotune`` times the configurations of ``search_space`` on the real batch and caches
+the winner per (dtype, width histogram, layers, features) in a JSON file.  The library
+takes its launch shapes from the widths (a configuration's values are checked; its
+fuse_qubits selects the order of rounding of complex64 results), so the space is the
+batch's own configuration; caches of earlier versions are read.
 """
 import ctypes
 import json
@@ -116,18 +116,10 @@ class QNNBatch:
         return json.dumps({"dtype": self.precision, "hist": hist, "layers": self.layers, "nfeat": self.nfeat})
 
     def search_space(self):
-        """LDS width limit (tile size) x fusion depth (qubits per pass) x workgroup size x
-        workgroups per CU."""
-        lds_cap = 12 if self.precision == "double" else 13
-        for lds in sorted({min(10, lds_cap), min(11, lds_cap), lds_cap}):
-            for fuse in (1, 2, 3):
-                for threads in (256, 512):
-                    for per_cu in (1, 2):
-                        amp = 16 if self.precision == "double" else 8
-                        if per_cu * 2 * (1 << lds) * amp > 160 * 1024:
-                            continue
-                        yield {"lds_max_width": lds, "block_threads": threads, "blocks_per_cu": per_cu,
-                               "use_graph": 1, "fuse_qubits": fuse}
+        """Configurations that may differ in time.  The library takes its launch shapes from
+        the widths, which leaves the batch's own; its fuse_qubits, on which the order of
+        rounding of complex64 results depends, is not chosen by time."""
+        yield dict(self.config)
 
     def autotune(self, theta: np.ndarray, reps: int = 2, use_cache: bool = True) -> Dict:
         key = self._key()
