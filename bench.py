@@ -5,10 +5,12 @@ Headline workload (one "step" = simulate the whole circuit from |0...0>):
   gates from {H,X,Y,Z,S,T,Rx,Ry,Rz,U3,CX,CZ,CRz,Swap} (60% one-qubit / 40%
   two-qubit, seed 2), gates fused into register/LDS-resident tile passes.
 
-value = achieved HBM GB/s over the timed steps = passes * 2 * 2^n * 16 B / time.
-roofline = the dominant kernel (the fused tile pass): algorithmic bytes per
-launch (2 * 2^n * 16 B, one read and one write of the state) / its average
-launch time, measured with HIP events on the launch stream.
+value = achieved HBM GB/s over the timed steps = bytes of state that the passes read
+and wrote / time.  A pass reads and writes the state once (2 * 2^n * 16 B); the first
+ones of a run from |0...0> take only the tiles that hold anything, and only those are
+counted (qs_profile_bytes).
+roofline = the dominant kernel (the fused tile pass): those bytes / the summed launch
+times, measured with HIP events on the launch stream.
 cpu_baseline = the C restatement of the reference CPU simulator (one pass per
 gate, gather / mat-vec / scatter) on a bounded sample of the same workload.
 
@@ -41,6 +43,14 @@ def profile_read(lib, ctx, reset=True):
     return list(ms), list(cnt)
 
 
+def profile_bytes(lib, ctx):
+    """State bytes that the fused passes read and wrote since the last call."""
+    from quict_amd import _native as nat
+    b = ctypes.c_double(0)
+    nat.check(lib.qs_profile_bytes(ctx, ctypes.byref(b), 1), "qs_profile_bytes")
+    return b.value
+
+
 def run_sv(n, circuit, precision, fusion, steps, warmup, lib, ctx):
     import torch
     from quict_amd.simulation import StateVectorSimulator
@@ -49,6 +59,7 @@ def run_sv(n, circuit, precision, fusion, steps, warmup, lib, ctx):
         sim.run(circuit)
     torch.cuda.synchronize()
     profile_read(lib, ctx, reset=True)
+    profile_bytes(lib, ctx)
     lib.qs_profile_enable(ctx, 1)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
@@ -58,10 +69,11 @@ def run_sv(n, circuit, precision, fusion, steps, warmup, lib, ctx):
     dt = time.perf_counter() - t0
     lib.qs_profile_enable(ctx, 0)
     ms, cnt = profile_read(lib, ctx, reset=True)
+    moved = profile_bytes(lib, ctx)
     passes = sim.last_passes
     del sim
     torch.cuda.empty_cache()
-    return dt, passes, ms, cnt
+    return dt, passes, ms, cnt, moved
 
 
 def run_stream_copy(n, lib, ctx, reps=5):
@@ -140,7 +152,7 @@ def run_adjoint_20q(reps=20, cpu=False):
 
 def run_qnn_batch(precision, reps=3, sample_circuits=3, sample_params=6):
     """1024 circuits, widths 8..18, 16 Ry-encoded features, 6 layers, loss mean((<Z0>-t)^2):
-    one autotuned persistent launch for forward + backward, against per-circuit parameter
+    one call for forward + backward, against per-circuit parameter
     shift on this GPU (a sample of circuits and parameters, scaled to a rate)."""
     import numpy as np
     from quict_amd.gradient.qnn import QNNBatch, synthetic_batch, circuit_for
@@ -197,6 +209,7 @@ def run_dm14(lib, ctx, reps=3, cpu=False):
     sim.run(c, noise_model=nm)
     torch.cuda.synchronize()
     profile_read(lib, ctx, reset=True)
+    profile_bytes(lib, ctx)
     lib.qs_profile_enable(ctx, 1)
     t0 = time.perf_counter()
     for _ in range(reps):
@@ -206,11 +219,11 @@ def run_dm14(lib, ctx, reps=3, cpu=False):
     dt = (time.perf_counter() - t0) / reps
     lib.qs_profile_enable(ctx, 0)
     ms, cnt = profile_read(lib, ctx, reset=True)
-    pass_bytes = 2 * (1 << 28) * 16
+    moved = profile_bytes(lib, ctx) / reps
     passes = sim.last_passes
     kern_ms = (ms[0] + ms[1]) / reps
     out = {"qubits": 14, "gates": 300, "passes": passes, "ms_per_run": dt * 1e3, "kernel_ms_per_run": kern_ms,
-           "gbs_wall": passes * pass_bytes / dt / 1e9, "gbs_kernels": passes * pass_bytes / (kern_ms * 1e-3) / 1e9,
+           "gbs_wall": moved / dt / 1e9, "gbs_kernels": moved / (kern_ms * 1e-3) / 1e9,
            "trace": [tr.real, tr.imag], "diag_sum": float(d.sum())}
     del sim
     torch.cuda.empty_cache()
@@ -292,6 +305,7 @@ def run_unitary14(lib, ctx, reps=3, cpu=True):
         t_id.append(timed(lambda: nat.check(lib.qs_mat_identity(ctx, ctypes.c_void_p(W.data_ptr()), n, nat.QS_C128,
                                                                 stream))))
         profile_read(lib, ctx, reset=True)
+        profile_bytes(lib, ctx)
         lib.qs_profile_enable(ctx, 1)
         t0 = time.perf_counter()
         W2, _ = build_columns(c.gates, n, nat.QS_C128)
@@ -299,6 +313,7 @@ def run_unitary14(lib, ctx, reps=3, cpu=True):
         t_all.append((time.perf_counter() - t0) * 1e3)
         lib.qs_profile_enable(ctx, 0)
         ms, cnt = profile_read(lib, ctx, reset=True)
+        moved = profile_bytes(lib, ctx)
         t_gates.append(ms[0] + ms[1])
         t_mv.append(timed(lambda: nat.check(lib.qs_mat_vec(ctx, ctypes.c_void_p(W2.data_ptr()), n, nat.QS_C128, 1,
                                                            ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()),
@@ -310,7 +325,7 @@ def run_unitary14(lib, ctx, reps=3, cpu=True):
     med = lambda v: float(np.median(v))
     out = {"qubits": n, "gates": 300, "passes": passes, "matrix_GiB": mat_bytes / 2**30,
            "identity_ms": med(t_id), "identity_gbs": mat_bytes / (med(t_id) * 1e-3) / 1e9,
-           "gate_passes_ms": med(t_gates), "gbs_per_pass": passes * 2 * mat_bytes / (med(t_gates) * 1e-3) / 1e9,
+           "gate_passes_ms": med(t_gates), "gbs_per_pass": moved / (med(t_gates) * 1e-3) / 1e9,
            "matvec_ms": med(t_mv), "matvec_gbs": mat_bytes / (med(t_mv) * 1e-3) / 1e9,
            "transpose_ms": med(t_tr), "transpose_gbs": 2 * mat_bytes / (med(t_tr) * 1e-3) / 1e9,
            "columns_wall_ms": med(t_all)}
@@ -416,7 +431,7 @@ def host_cpu():
 def measured_traffic(n, ngates):
     """HBM bytes per tile-pass launch from the committed PMC summary (FETCH_SIZE +
     WRITE_SIZE, copy-calibrated) when this run is the workload it was measured on."""
-    path = os.path.join(ROOT, "profiles", "k_fused_sv30_c128_traffic.txt")
+    path = os.path.join(ROOT, "profiles", "k_wires_sv30_c128_traffic.txt")
     if (n, ngates) != (30, 2000) or not os.path.exists(path):
         return None
     vals = {}
@@ -515,27 +530,29 @@ def main():
     pass_bytes = 2 * state_bytes
 
     log("timed: complex128 fused")
-    dt, passes, ms, cnt = run_sv(n, circuit, "double", True, args.steps, args.warmup, lib, ctx)
+    dt, passes, ms, cnt, moved = run_sv(n, circuit, "double", True, args.steps, args.warmup, lib, ctx)
     step_ms = dt / args.steps * 1e3
-    value = passes * pass_bytes / (dt / args.steps) / 1e9
+    value = moved / dt / 1e9
     gates_per_s = args.gates / (dt / args.steps)
     fused_launches = cnt[0] // max(args.steps, 1)
     avg_fused_ms = ms[0] / max(cnt[0], 1)
-    roof_achieved = pass_bytes / (avg_fused_ms * 1e-3) / 1e9 if cnt[0] else None
-    log(f"c128 fused: {step_ms:.1f} ms/step, {passes} passes, {value:.0f} GB/s, avg tile-pass {avg_fused_ms:.3f} ms")
+    roof_achieved = moved / (ms[0] * 1e-3) / 1e9 if cnt[0] else None
+    full_passes = moved / args.steps / pass_bytes
+    log(f"c128 fused: {step_ms:.1f} ms/step, {passes} passes moving {full_passes:.2f} times the state, {value:.0f} GB/s, "
+        f"avg tile-pass {avg_fused_ms:.3f} ms")
 
     secondary = {}
     log("streaming copy of one state (bandwidth reference; its profile calibrates the counters)")
     secondary["stream_copy"] = run_stream_copy(n, lib, ctx)
     if not args.no_secondary:
         log("secondary: complex64 fused")
-        dt64, p64, ms64, cnt64 = run_sv(n, circuit, "single", True, 1, 1, lib, ctx)
+        dt64, p64, ms64, cnt64, moved64 = run_sv(n, circuit, "single", True, 1, 1, lib, ctx)
         secondary["c64_fused"] = {
-            "ms_per_step": dt64 * 1e3, "passes": p64, "gbs": p64 * 2 * (1 << n) * 8 / dt64 / 1e9,
+            "ms_per_step": dt64 * 1e3, "passes": p64, "gbs": moved64 / dt64 / 1e9,
             "gates_per_s": args.gates / dt64,
-            "tile_pass_gbs": (2 * (1 << n) * 8) / (ms64[0] / max(cnt64[0], 1) * 1e-3) / 1e9 if cnt64[0] else None}
+            "tile_pass_gbs": moved64 / (ms64[0] * 1e-3) / 1e9 if cnt64[0] else None}
         log("secondary: complex128 unfused (one pass per gate)")
-        dtu, pu, msu, cntu = run_sv(n, circuit, "double", False, 1, 0, lib, ctx)
+        dtu, pu, msu, cntu, _ = run_sv(n, circuit, "double", False, 1, 0, lib, ctx)
         touched = touched_bytes(circuit, n, 16)
         secondary["c128_unfused"] = {
             "ms_per_step": dtu * 1e3, "passes": pu, "gates_per_s": args.gates / dtu,
@@ -546,7 +563,7 @@ def main():
                     "phase gate touches 1/2^(controls+targets) of the state, a swap 1/2)"}
         log("secondary: 20-qubit 400-gate circuit + 1024 shots")
         c20 = workloads.sv20_circuit()
-        dt20, p20, _, _ = run_sv(20, c20, "double", True, 5, 2, lib, ctx)
+        dt20, p20, _, _, _ = run_sv(20, c20, "double", True, 5, 2, lib, ctx)
         from quict_amd.simulation import StateVectorSimulator
         import random
         s20 = StateVectorSimulator("GPU", precision="double")
@@ -617,15 +634,16 @@ def main():
                    "tile_low_bits": args.low_bits or 4},
         "gates_per_s": gates_per_s,
         "passes_per_step": passes,
+        "state_passes_per_step": full_passes,
         "roofline": {"bound": "hbm", "achieved": roof_achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": (roof_achieved / HBM_PEAK_GBS) if roof_achieved else None,
                      "traffic": measured_traffic(n, args.gates),
-                     "traffic_source": ("profiles/k_fused_sv30_c128_traffic.txt: rocprofv3 --pmc FETCH_SIZE and "
+                     "traffic_source": ("profiles/k_wires_sv30_c128_traffic.txt: rocprofv3 --pmc FETCH_SIZE and "
                                         "WRITE_SIZE runs of this workload, copy-calibrated; not measured in this run")
                      if measured_traffic(n, args.gates) else None,
-                     "kernel": "k_fused<double,4,8>", "launches_per_step": fused_launches,
+                     "kernel": "k_wires<double,4,8>", "launches_per_step": fused_launches,
                      "avg_launch_ms": avg_fused_ms,
-                     "bytes_per_launch": pass_bytes,
+                     "bytes_per_launch": moved / max(cnt[0], 1),
                      "frac_of_stream_copy": (roof_achieved / secondary["stream_copy"]["nontemporal"]["gbs"])
                      if roof_achieved and "stream_copy" in secondary else None},
         "cpu_baseline": cpu,

@@ -86,6 +86,10 @@ uint64_t qs_ctx_scratch_bytes(const qs_ctx* ctx);
    adjoint, qnn batch], the summed kernel milliseconds and launch counts. */
 int qs_profile_enable(qs_ctx* ctx, int on);
 int qs_profile_read(qs_ctx* ctx, double* ms /*[4]*/, int64_t* launches /*[4]*/, int reset);
+/* Bytes of state that the bracketed fused passes read and wrote since the last reset:
+   2 * 2^n amplitudes a pass, less what a pass over a vector with known zeros leaves
+   out (see qs_run). */
+int qs_profile_bytes(qs_ctx* ctx, double* fused, int reset);
 
 /* Streaming copy of `bytes` (a multiple of 16) from src to dst, 16 B per lane,
    optionally with non-temporal loads/stores: the achievable-bandwidth

@@ -75,6 +75,7 @@ SIGNATURES = {
     "qs_set_fusion_launch": (_I, [_P, _I, _I]),
     "qs_profile_enable": (_I, [_P, _I]),
     "qs_profile_read": (_I, [_P, _P, _P, _I]),
+    "qs_profile_bytes": (_I, [_P, ctypes.POINTER(_D), _I]),
     "qs_stream_copy": (_I, [_P, _P, _P, _U64, _I, _P]),
     "qs_sv_init": (_I, [_P, _P, _I, _I, _U64, _P]),
     "qs_sv_apply_gate": (_I, [_P, _P, _I, _I, _P, _P]),

@@ -425,6 +425,13 @@ int qs_profile_read(qs_ctx* ctx, double* ms, int64_t* launches, int reset) {
   return QS_OK;
 }
 
+int qs_profile_bytes(qs_ctx* ctx, double* fused, int reset) {
+  QS_REQUIRE(ctx && fused, "null argument");
+  *fused = ctx->prof_bytes;
+  if (reset) ctx->prof_bytes = 0;
+  return QS_OK;
+}
+
 uint64_t qs_ctx_scratch_bytes(const qs_ctx* ctx) {
   return ctx ? ctx->scratch_bytes + ctx->prog_slot[0].dev_bytes + ctx->prog_slot[1].dev_bytes : 0;
 }

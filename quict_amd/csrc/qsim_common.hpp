@@ -135,6 +135,7 @@ struct qs_ctx {
   int profile = 0;
   double prof_ms[4] = {0, 0, 0, 0};       // per kernel class, see qs_profile_read
   int64_t prof_count[4] = {0, 0, 0, 0};
+  double prof_bytes = 0;                  // read and written by the fused passes
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pool;
   std::vector<std::pair<int, int>> ev_pending;  // (pool index, class)
 };

@@ -124,11 +124,15 @@ static int launch_fused(qs_ctx* ctx, cx<R>* v, int n, const Config& c, const Pas
   int rc = QS_OK;
   // (the kernel that prefetches tiles takes a vector that is there)
   if (!c.wires && !hd.has_dk && ctx->fused_prefetch && (rc = write_rest(v, n, z, s))) return rc;
+  // (of a vector with known zeros the amplitudes that can differ from 0 are read, none
+  // of them before the first pass)
+  const double reads = z.fresh ? 0.0 : std::ldexp(1.0, n - __builtin_popcountll(z.fixed & ((1ull << n) - 1)));
   const PassStart S = enter_pass(z, hd, K, std::max(n, K));
   const uint64_t tiles = S.fixed ? 1ull << __builtin_popcountll(S.free) : n > K ? 1ull << (n - K) : 1;
   const size_t lds_bytes = (size_t)(1u << (K - 1)) * sizeof(cx<R>);  // half-tile relayout image
   const size_t lds_relayout = hd.uses_lds ? lds_bytes : 0;
   const size_t lds = hd.has_dk && !c.wires ? lds_relayout : lds_relayout + (size_t)hd.nstage * sizeof(cx<R>);
+  if (prof && ctx->profile) ctx->prof_bytes += (reads + std::ldexp((double)tiles, std::min(n, K))) * sizeof(cx<R>);
   if (prof && (rc = prof_begin(ctx, PROF_FUSED, s))) return rc;
   if (c.wires) {
     launch_wires<R, RB, TB>(v, tiles, hd, dh, (const WireOp<R>*)d.O, d.C, d.X, n < K ? 1u << n : 0u, S, lds, s);
