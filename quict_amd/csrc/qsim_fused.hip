@@ -136,17 +136,16 @@ static int launch_fused(qs_ctx* ctx, cx<R>* v, int n, const Config& c, const Pas
   if (prof && (rc = prof_begin(ctx, PROF_FUSED, s))) return rc;
   if (c.wires) {
     launch_wires<R, RB, TB>(v, tiles, hd, dh, (const WireOp<R>*)d.O, d.C, d.X, n < K ? 1u << n : 0u, S, lds, s);
-  } else if (hd.has_dk) {
-    hipLaunchKernelGGL((k_fused<R, RB, TB, true, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, d.O,
-                       d.C, d.X, tiles, S);
-  } else if (ctx->fused_prefetch) {
-    // persistent, prefetching: resident workgroups only
-    const uint64_t grid = std::min<uint64_t>(tiles, (uint64_t)ctx->num_cus * ctx->fused_wg_per_cu);
-    hipLaunchKernelGGL((k_fused<R, RB, TB, false, true>), dim3((unsigned)grid), dim3(1 << TB), lds, s, v, dh, d.O,
-                       d.C, d.X, tiles, S);
   } else {
-    hipLaunchKernelGGL((k_fused<R, RB, TB, false, false>), dim3((unsigned)tiles), dim3(1 << TB), lds, s, v, dh, d.O,
-                       d.C, d.X, tiles, S);
+    auto pass = [&](auto kernel, uint64_t grid) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(1 << TB), lds, s, v, dh, d.O, d.C, d.X, tiles, S);
+    };
+    if (hd.has_dk && S.fixed) pass(k_fused<R, RB, TB, true, false, true>, tiles);
+    else if (hd.has_dk) pass(k_fused<R, RB, TB, true, false, false>, tiles);
+    else if (S.fixed) pass(k_fused<R, RB, TB, false, false, true>, tiles);
+    else if (ctx->fused_prefetch)  // persistent, prefetching: resident workgroups only
+      pass(k_fused<R, RB, TB, false, true, false>, std::min<uint64_t>(tiles, (uint64_t)ctx->num_cus * ctx->fused_wg_per_cu));
+    else pass(k_fused<R, RB, TB, false, false, false>, tiles);
   }
   QS_CHECK_HIP(hipGetLastError());
   if (prof && (rc = prof_end(ctx, s))) return rc;
@@ -360,12 +359,10 @@ template <typename R, int RB, int TB> static void set_lds_attr() {
   if (done) return;
   wires_lds_attr<R, RB, TB>();
   const int bytes = (int)((1u << (RB + TB - 1)) * sizeof(cx<R>) + FMAX_PASS_COEF * sizeof(cx<R>));
-  (void)hipFuncSetAttribute((const void*)k_fused<R, RB, TB, true, false>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  (void)hipFuncSetAttribute((const void*)k_fused<R, RB, TB, false, true>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  (void)hipFuncSetAttribute((const void*)k_fused<R, RB, TB, false, false>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  for (const void* k : {(const void*)k_fused<R, RB, TB, true, false, true>, (const void*)k_fused<R, RB, TB, true, false, false>,
+                        (const void*)k_fused<R, RB, TB, false, false, true>, (const void*)k_fused<R, RB, TB, false, true, false>,
+                        (const void*)k_fused<R, RB, TB, false, false, false>})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   done = true;
 }
 
