@@ -71,7 +71,7 @@ static cplx cdiv_(cplx a, cplx b) {
 // Whether f may be taken out of a gate as a common factor and divided by.  Entries far
 // from modulus 1 stay in their gate: a program's common factor, or the reciprocal of
 // one, would leave the range of its precision where no amplitude does.
-static bool near_unit(cplx f) { return std::fabs(std::hypot(f.first, f.second) - 1.0) <= 1e-5; }
+static bool near_unit(cplx f) { return std::fabs(f.first * f.first + f.second * f.second - 1.0) <= 2e-5; }
 
 struct WireReducer {
   const Config& c;
@@ -164,7 +164,7 @@ struct WireReducer {
     for (int i = 0; i < k; ++i) flipped += (F >> ws[i]) & 1;
     // Every flipped bit splits the phase in two (below): from two of them on, on more
     // than two bits (whose parts join what is on their wires), the flips become gates.
-    const bool split = (flipped == 1 || k <= 2) && near_unit(f);
+    const bool split = flipped && (flipped == 1 || k <= 2) && near_unit(f);
     for (int i = 0; i < k; ++i) {
       if (!((F >> ws[i]) & 1)) continue;
       if (!split) {
@@ -431,7 +431,8 @@ struct WireReducer {
     else pb = neg(unit(cdiv_(e(1), f)));
     // (written so that a phase of a zero, which is not a number, fails)
     auto gives = [&](int i, cplx z, double r) {
-      return mag({m[2 * i] - z.first * r, m[2 * i + 1] - z.second * r}) <= tol;
+      const double x = m[2 * i] - z.first * r, y = m[2 * i + 1] - z.second * r;
+      return x * x + y * y <= tol * tol;
     };
     const cplx fa = cm_(f, pa);
     if (!(gives(0, f, c_) && gives(1, cm_(f, pb), -s_) && gives(2, fa, s_) && gives(3, cm_(fa, pb), c_))) return false;
@@ -1227,11 +1228,13 @@ static int plan_wires(const Fill& fill, int ngates, int nbits, const Config& c, 
       const Rem& r = rem[k];
       if (!((r.a & wm) | (r.m & wa))) {
         const uint64_t need = r.need & ~S;
-        const bool room = !((r.flags & TABLE) && tables >= max_tables) && !((r.flags & MEAS) && meas >= FMAX_GRAD);
-        const bool able = room && !(r.flags & ALONE);
+        bool able = true;
+        if (r.flags)
+          able = !(r.flags & ALONE) && !((r.flags & TABLE) && tables >= max_tables) &&
+                 !((r.flags & MEAS) && meas >= FMAX_GRAD);
         if (!need && able) {
           w += r.w;
-          tables += (r.flags & TABLE) != 0, meas += (r.flags & MEAS) != 0;
+          if (r.flags) tables += (r.flags & TABLE) != 0, meas += (r.flags & MEAS) != 0;
           if (taken) taken->push_back(k);
           continue;
         }
