@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void k_qnn_gradx_sum(const QnnGroups G, const 
   }
 }
 
-constexpr size_t QNN_MAX_IMAGES = 64;  // planned programs kept, 0.1..0.6 MB each; a batch has at most 19 widths
+constexpr size_t QNN_MAX_IMAGES = 64;  // planned programs kept, 0.1..0.6 MB each; a batch has at most 19 widths (2..20)
 
 static int qnn_image(QnnState* S, int w, int layers, VarImage** out) {
   const auto key = std::make_pair(w, layers);
@@ -396,7 +396,7 @@ static int qnn_part(qs_ctx* ctx, QnnState* S, const int32_t* order, int n, int n
         heavy = heavy || P[p].heavy;
       }
       if (!J.n) break;
-      launch_jobs<double>(psi, back ? lam : nullptr, d, J, (uint32_t)blocks, heavy, (double*)(d + part_off), lds, s);
+      launch_jobs<double>(psi, back ? lam : nullptr, d, J, (uint32_t)blocks, heavy, (double*)(d + part_off), lds, ctx->num_cus, s);
       QS_CHECK_HIP(hipGetLastError());
     }
   }

@@ -136,7 +136,7 @@ static int var_gradient(qs_var* v, cx<R>* psi, cx<R>* lam, const double* theta, 
   for (const VarImage::Pass& p : v->im.fwd) {
     if ((rc = prof_begin(ctx, PROF_FUSED, s))) return rc;
     j.hdr = h++ * (uint32_t)sizeof(PassHdr);
-    launch_jobs<R>(psi, nullptr, v->dev, J, (uint32_t)tiles, p.heavy, nullptr, p.lds, s);
+    launch_jobs<R>(psi, nullptr, v->dev, J, (uint32_t)tiles, p.heavy, nullptr, p.lds, ctx->num_cus, s);
     QS_CHECK_HIP(hipGetLastError());
     if ((rc = prof_end(ctx, s))) return rc;
   }
@@ -152,7 +152,7 @@ static int var_gradient(qs_var* v, cx<R>* psi, cx<R>* lam, const double* theta, 
     j.hdr = h++ * (uint32_t)sizeof(PassHdr);
     j.keep = i + 1 < v->im.bwd.size() ? 3 : 0;  // nothing reads the vectors after the sweep
     j.part = v->row0[i];
-    launch_jobs<R>(psi, lam, v->dev, J, (uint32_t)tiles, p.heavy, partial, p.lds, s);
+    launch_jobs<R>(psi, lam, v->dev, J, (uint32_t)tiles, p.heavy, partial, p.lds, ctx->num_cus, s);
     QS_CHECK_HIP(hipGetLastError());
     if (v->sum_to[i] > summed) {
       column_sums(partial, (const ColSum*)(v->dev + v->col_off) + summed, v->sum_to[i] - summed, sums + summed, s);

@@ -27,7 +27,7 @@ template <typename R, int RB, int TB> void wires_lds_attr() {
 
 template <typename R>
 void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs, uint32_t blocks, bool heavy, double* partial,
-                 size_t lds, hipStream_t s) {
+                 size_t lds, int cus, hipStream_t s) {
   static bool attr = false;  // two images, tables and gradient rows can pass 64 KiB
   if (!attr) {
     const int bytes = 150 * 1024;
@@ -42,7 +42,7 @@ void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs
   // One image for both vectors where a CU gets more than the two workgroups that fit
   // with one each.  1024 variational circuits 6.5 -> 6.1 ms; with a workgroup a CU (20
   // qubits) two images cost nothing and save barriers.
-  const bool shared = lam && !heavy && sizeof(R) == 8 && blocks > 512 && lds >= 2 * (sizeof(cx<R>) << 11);
+  const bool shared = lam && !heavy && sizeof(R) == 8 && blocks > 2u * (uint32_t)cus && lds >= 2 * (sizeof(cx<R>) << 11);
   if (!lam && heavy) hipLaunchKernelGGL((k_jobs<R, 1, 1, true>), g, t, lds, s, psi, lam, image, jobs, partial);
   else if (!lam) hipLaunchKernelGGL((k_jobs<R, 1, 1, false>), g, t, lds, s, psi, lam, image, jobs, partial);
   else if (heavy) hipLaunchKernelGGL((k_jobs<R, 2, 2, true>), g, t, lds, s, psi, lam, image, jobs, partial);
@@ -52,8 +52,8 @@ void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs
 }
 
 template void launch_jobs<double>(cx<double>*, cx<double>*, const char*, const WireJobs&, uint32_t, bool, double*,
-                                  size_t, hipStream_t);
-template void launch_jobs<float>(cx<float>*, cx<float>*, const char*, const WireJobs&, uint32_t, bool, double*, size_t,
+                                  size_t, int, hipStream_t);
+template void launch_jobs<float>(cx<float>*, cx<float>*, const char*, const WireJobs&, uint32_t, bool, double*, size_t, int,
                                  hipStream_t);
 
 #define QS_WIRES(R, TB)                                                                                          \

@@ -197,12 +197,12 @@ struct WireJobs {
   int n;
   WireJob j[WIRE_MAX_JOBS];
 };
-// lam == nullptr: one vector.  The kernel reads the programs through one pointer
+// lam == nullptr: one vector.  cus: the device's compute units.  The kernel reads the programs through one pointer
 // argument, which it never writes: pointers inside the jobs would make every
 // descriptor a vector load.
 template <typename R>
 void launch_jobs(cx<R>* psi, cx<R>* lam, const char* image, const WireJobs& jobs, uint32_t blocks, bool heavy, double* partial,
-                 size_t lds, hipStream_t s);
+                 size_t lds, int cus, hipStream_t s);
 
 // One pass over the 2^(n-K) tiles of v: header hd, its device copy dh and the
 // program's device arrays; nsmall: amplitudes of a register below a tile, else 0.  The caller checks hipGetLastError().
