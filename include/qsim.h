@@ -140,7 +140,8 @@ int qs_set_fusion(qs_ctx* ctx, int tile_log2, int low_bits);
 
 /* Launch shape of the fused tile pass: prefetch != 0 selects persistent
    workgroups (wg_per_cu per CU) that load the next tile while computing the
-   current one; prefetch == 0 launches one workgroup per tile. */
+   current one; prefetch == 0 launches one workgroup per tile.  For programs that keep
+   whole gates in the tile (noise superoperators, QS_START_ZERO_WHOLE); others ignore it. */
 int qs_set_fusion_launch(qs_ctx* ctx, int prefetch, int wg_per_cu);
 
 /* Captured gate sequences (HIP graphs).  qs_graph_capture plans the sequence

@@ -28,8 +28,8 @@
 //    next LDS relayout address or the store address (one XOR per tile).
 //
 // Two planners fill this scheme.  plan_wires (qsim_wire_plan.hpp, kernels in
-// qsim_wires.hip) runs every program but noisy density matrices: it wants only the
-// bits a gate mixes in the tile.  plan_groups (qsim_fused_plan.hpp, k_fused) wants
+// qsim_wires.hip) runs every program but noisy density matrices and complex64
+// gradients: it wants only the bits a gate mixes in the tile.  plan_groups (qsim_fused_plan.hpp, k_fused) wants
 // all of them; it is greedy with commutation: scanning the remaining gates in
 // order, a gate joins the current pass if its bits fit in the tile and it commutes
 // with every gate already deferred.

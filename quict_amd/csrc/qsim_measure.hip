@@ -216,7 +216,8 @@ template <typename R> static int reset_t(cx<R>* v, int n, int bit, double p0, hi
 }
 
 // Scratch layout of one sampling call: pyramid levels 1..n (sizes 2^(n-1) .. 1,
-// back to back), 2 KiB unused, the uniforms and the outcomes.
+// back to back), 2 KiB that the documented limit of the fixed array counts (nothing is
+// in them), the uniforms and the outcomes.
 struct SampleLayout {
   Levels levels;
   uint64_t pyr_bytes, off_bytes, u_bytes, o_bytes;

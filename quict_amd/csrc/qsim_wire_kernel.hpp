@@ -2,10 +2,10 @@
 // interpreter and kernel.
 //
 // What bounds it: with 3 to 4 times fewer passes than k_fused each pass carries
-// 30 to 60 ops, and the vector ALU is what a pass waits for (measured with
-// k_fused as the interpreter: 70% of the cycles of a 25-qubit complex64 pass were
-// VALU issue, 6900 instructions a wave for 46 ops).  So the ops are written to
-// need few instructions and no copies of the tile:
+// 30 to 60 ops, and a wave's instructions are what a pass waits for.  So the ops are
+// written to need few of them and no copies of the tile: 2171 vector and 1839 scalar
+// instructions a wave in a 30-qubit pass of about 63 ops, the vector ALU busy 60% of
+// the time with four waves a SIMD:
 //   * every op changes its registers in place.  A rotation is three shears,
 //     x0 += t x1, x1 += s x0, x0 += t x1 (t = -tan(theta / 2), s = sin(theta),
 //     |theta| <= pi / 2, so |t| <= 1): 3 fused multiply-adds per component pair

@@ -23,12 +23,14 @@
 // home lies in the tile.
 //
 // Measured on MI355X against plan_groups and k_fused: the 30-qubit complex128
-// 2000-gate 60/40 circuit 556 ms in 73 passes, 191 ms in 23; 8 layers of the
-// hardware-efficient ansatz on 25 qubits, complex64, 4.98 ms in 23 passes, 2.70 ms
-// in 8; the matrix of a 300-gate 13-qubit circuit 3.84 against 2.09 ms; 400 gates on
-// 20 qubits as a captured graph 295 against 193 us.  Against 80-bit arithmetic the
-// state is closer than the per-gate kernels' (838 gates on 13 qubits: 2e-15 against
-// 1.2e-14): a factored gate is unitary to the last bit, a rounded matrix is not.
+// 2000-gate 60/40 circuit 556 ms in 73 passes, 191 ms in 23 (157 with known zeros and
+// joined ops); 8 layers of the hardware-efficient ansatz on 25 qubits, complex64, 4.98
+// ms in 23 passes, 2.70 ms in 8 (1.71); the matrix of a 300-gate 13-qubit circuit 3.84
+// against 2.09 ms (1.5); 400 gates on 20 qubits as a captured graph 295 against 193 us
+// (118).  Against 80-bit arithmetic the state is closer than the per-gate kernels' (838
+// gates on 13 qubits: 2e-15 against 1.2e-14): a factored gate is unitary to the last
+// bit, a rounded matrix is not, and a split that does not give the matrix back to that
+// rounding is not taken.
 //
 // schedule_wires turns one pass into ops.  A CX is a GF(2)-linear map of the
 // index, so it needs no arithmetic at all when it is left to the addresses of
