@@ -17,9 +17,11 @@ def uniforms(count: int) -> np.ndarray:
     # (a replaced random.random, or another generator behind it, is asked draw by draw)
     if count <= 0 or type(owner) is not random.Random or getattr(random.getrandbits, "__self__", None) is not owner:
         return np.array([random.random() for _ in range(count)], dtype=np.float64)
-    out = np.empty(count, dtype=np.float64)
-    for i in range(0, count, BLOCK):
-        k = min(BLOCK, count - i)
-        w = np.frombuffer(random.getrandbits(64 * k).to_bytes(8 * k, "little"), dtype="<u8")
-        np.multiply(((w & 0xFFFFFFE0) << 21) | (w >> 38), 2.0 ** -53, out=out[i: i + k])
-    return out
+    if count <= BLOCK:
+        return _draw(count)
+    return np.concatenate([_draw(min(BLOCK, count - i)) for i in range(0, count, BLOCK)])
+
+
+def _draw(k: int) -> np.ndarray:
+    w = np.frombuffer(random.getrandbits(64 * k).to_bytes(8 * k, "little"), dtype="<u8")
+    return (((w & 0xFFFFFFE0) << 21) | (w >> 38)).astype(np.float64) * 2.0 ** -53
